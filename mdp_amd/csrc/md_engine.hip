@@ -11,9 +11,10 @@
 //   4. SNAP: Utot (k_ui), Y + energy partials (k_yi), dE/dr per pair (k_dedr)
 //   5. tally per atom without atomics: f_i = sum over own pairs - sum over incoming pairs,
 //      W_i = -sum_j r_ij (x) dE/dr_ij, E_i from the energy partials; then v += dt/2 f/m.
-// Neighbour entries are (owner j, image shift) pairs stored slot-major (slot k of atom i at k*N + i,
-// so that per-atom loops read coalesced across the lanes of a wave); positions stay unwrapped between rebuilds and
-// the displacement of a neighbour is always (x_j + shift*L) - x_i, evaluated without contraction.
+// Neighbour entries are (owner j, image shift) pairs stored atom-major (slot k of atom i at i*NBMAX + k): the
+// 16 lanes that share an atom in the per-step kernels read one contiguous run.  Positions stay unwrapped
+// between rebuilds and the displacement of a neighbour is always (x_j + shift*L) - x_i, evaluated without
+// contraction.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -221,13 +222,13 @@ __global__ void k_wrap_bin(double* __restrict__ x, double* __restrict__ xref, in
                            double Ly, double Lz, int ncx, int ncy, int ncz, int N, int check,
                            int* __restrict__ flags) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
     const double L[3] = {Lx, Ly, Lz};
     const int nc[3] = {ncx, ncy, ncz};
     double d2 = 0.0;
     int c[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
+        if (i >= N) break;
         double xi = x[3 * i + d];
         if (!isfinite(xi)) {   // keep the cell index in range; the host reports the error
             atomicOr(flags, 8);
@@ -248,7 +249,13 @@ __global__ void k_wrap_bin(double* __restrict__ x, double* __restrict__ xref, in
         xref[3 * i + d] = xi;
         c[d] = min(static_cast<int>(xi * nc[d] / L[d]), nc[d] - 1);
     }
-    if (check) atomicMax(maxd2_bits, static_cast<unsigned long long>(__double_as_longlong(d2)));
+    if (check) {   // the wave's maximum first: one atomic on the shared word instead of 64
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) d2 = fmax(d2, __shfl_xor(d2, o));
+        if ((threadIdx.x & 63) == 0)
+            atomicMax(maxd2_bits, static_cast<unsigned long long>(__double_as_longlong(d2)));
+    }
+    if (i >= N) return;
     const int cid = c[0] + ncx * (c[1] + ncy * c[2]);
     cell_of[i] = cid;
     atomicAdd(&cell_cnt[cid], 1);
@@ -263,22 +270,23 @@ __global__ void k_cell_fill(const int* __restrict__ cell_of, const int* __restri
     cell_atoms[cell_start[c] + pos] = i;
 }
 
-// ascending atom order inside each cell (deterministic list order)
-__global__ void k_cell_sort(const int* __restrict__ cell_start, int* __restrict__ cell_atoms, int ncell,
-                            int* __restrict__ overflow) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    const int b = cell_start[c], e = cell_start[c + 1];
-    if (e - b > CELLCAP) atomicOr(overflow, 2);
-    for (int k = b + 1; k < e; ++k) {
-        const int v = cell_atoms[k];
-        int m = k - 1;
-        while (m >= b && cell_atoms[m] > v) {
-            cell_atoms[m + 1] = cell_atoms[m];
-            --m;
-        }
-        cell_atoms[m + 1] = v;
+// Ascending atom order inside each cell (deterministic list order): one wave per cell, each lane ranks its atom
+// against the others of the cell.  (One lane per cell sorting by insertion took 14-19 us on any system.)
+static_assert(CELLCAP <= 64, "a cell's atoms fit the lanes of one wave");
+
+__global__ __launch_bounds__(256) void k_cell_sort(const int* __restrict__ cell_start, int* __restrict__ cell_atoms,
+                                                   int ncell, int* __restrict__ overflow) {
+    const int c = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (c >= ncell) return;   // uniform over the wave
+    const int b = cell_start[c], n = cell_start[c + 1] - b;
+    if (n > CELLCAP) {   // reported by the host; the list is not used
+        if (lane == 0) atomicOr(overflow, 2);
+        return;
     }
+    const int v = lane < n ? cell_atoms[b + lane] : 0;
+    int rank = 0;
+    for (int k = 0; k < n; ++k) rank += __shfl(v, k) < v;
+    if (lane < n) cell_atoms[b + rank] = v;
 }
 
 // Eight lanes per centre atom, atoms taken in cell order (so the atoms of a wave share their 27
@@ -290,9 +298,9 @@ constexpr int NSUB = 8;
 __global__ __launch_bounds__(256) void k_neighbors_cell(const double* __restrict__ x, const int* __restrict__ cell_of,
                                                         const int* __restrict__ cell_start,
                                                         const int* __restrict__ cell_atoms, int* __restrict__ nb_cnt,
-                                                        int* __restrict__ nb_j, int* __restrict__ nb_s, double Lx,
-                                                        double Ly, double Lz, int ncx, int ncy, int ncz, double rcs2,
-                                                        int N, int* __restrict__ overflow) {
+                                                        int2* __restrict__ nbr, double Lx, double Ly, double Lz,
+                                                        int ncx, int ncy, int ncz, double rcs2, int N,
+                                                        int* __restrict__ overflow) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int g = t / NSUB, sub = t % NSUB, lane = threadIdx.x & 63;
     const unsigned long long group = 0xFFull << (lane & ~(NSUB - 1));
@@ -325,10 +333,7 @@ __global__ __launch_bounds__(256) void k_neighbors_cell(const double* __restrict
             const unsigned long long mk = __ballot(acc) & group;
             if (acc) {
                 const int q = cnt + __popcll(mk & below);
-                if (q < NBMAX) {
-                    nb_j[static_cast<size_t>(q) * N + i] = j;
-                    nb_s[static_cast<size_t>(q) * N + i] = code;
-                }
+                if (q < NBMAX) nbr[static_cast<size_t>(i) * NBMAX + q] = make_int2(j, code);
             }
             cnt += __popcll(mk);
         }
@@ -339,78 +344,88 @@ __global__ __launch_bounds__(256) void k_neighbors_cell(const double* __restrict
     }
 }
 
-// The same lists from a per-wavefront neighbour tile in LDS.  One wave owns one centre cell: it lists the
-// 27 surrounding cells (periodic images applied) in the fixed order above, stages their atoms -- index,
-// image shift and the imaged position x_j + s L -- in LDS, NTILE candidates at a time, and its centre atoms
-// (eight lanes each, eight atoms per pass, ascending) scan the tile from LDS.  Candidates, their order and
-// the distance arithmetic are those of k_neighbors_cell, so the lists are identical.
+// The same lists from a neighbour tile in LDS.  One workgroup of TH lanes owns one centre cell: it lists the 27
+// surrounding cells (periodic images applied) in the fixed order above, stages their atoms -- index, image
+// shift and the imaged position x_j + s L -- in LDS, NTILE candidates at a time, and its centre atoms (SUB
+// lanes each, TH / SUB atoms per pass, ascending) scan the tile from LDS.  Candidates, their order and the
+// distance arithmetic are those of k_neighbors_cell, so the lists are identical.
+// A tile that holds every candidate is staged once for all passes.  TH = 128, SUB = 8 covers the 9 or so atoms of
+// a cell in one pass; TH = 256, SUB = 16 halves the serial scan where there are too few cells to fill the chip.
 constexpr int NTILE = 256;
 
-__global__ __launch_bounds__(64) void k_neighbors_tile(const double* __restrict__ x,
+template <int TH, int SUB>
+__global__ __launch_bounds__(TH) void k_neighbors_tile(const double* __restrict__ x,
                                                        const int* __restrict__ cell_start,
                                                        const int* __restrict__ cell_atoms, int* __restrict__ nb_cnt,
-                                                       int* __restrict__ nb_j, int* __restrict__ nb_s, double Lx,
-                                                       double Ly, double Lz, int ncx, int ncy, int ncz, double rcs2,
-                                                       int N, int* __restrict__ overflow) {
+                                                       int2* __restrict__ nbr, double Lx, double Ly, double Lz,
+                                                       int ncx, int ncy, int ncz, double rcs2, int N,
+                                                       int* __restrict__ overflow) {
     __shared__ double tx[NTILE], ty[NTILE], tz[NTILE];
     __shared__ int tj[NTILE], ts[NTILE];
     __shared__ int k_off[28], k_base[27], k_code[27];
     __shared__ double k_dx[27], k_dy[27], k_dz[27];
-    const int c = blockIdx.x, lane = threadIdx.x;
+    const int c = blockIdx.x, tid = threadIdx.x;
     const int cb = cell_start[c], cn = cell_start[c + 1] - cb;
     if (cn == 0) return;   // uniform over the workgroup
     const int cx = c % ncx, cy = (c / ncx) % ncy, cz = c / (ncx * ncy);
-    if (lane < 27) {
-        const int k = lane;
-        const int ux = cx + k % 3 - 1, uy = cy + (k / 3) % 3 - 1, uz = cz + k / 9 - 1;
-        const int sx = (ux < 0) ? -1 : (ux >= ncx ? 1 : 0);
-        const int sy = (uy < 0) ? -1 : (uy >= ncy ? 1 : 0);
-        const int sz = (uz < 0) ? -1 : (uz >= ncz ? 1 : 0);
-        const int nc = (ux - sx * ncx) + ncx * ((uy - sy * ncy) + ncy * (uz - sz * ncz));
-        k_base[k] = cell_start[nc];
-        k_off[k + 1] = cell_start[nc + 1] - cell_start[nc];   // count, summed below
-        k_code[k] = shift_code(sx, sy, sz);
-        k_dx[k] = sx * Lx;
-        k_dy[k] = sy * Ly;
-        k_dz[k] = sz * Lz;
-    }
-    __syncthreads();
-    if (lane == 0) {
-        k_off[0] = 0;
-        for (int k = 0; k < 27; ++k) k_off[k + 1] += k_off[k];
+    if (tid < 64) {   // the first wave
+        int cnt = 0;
+        if (tid < 27) {
+            const int k = tid;
+            const int ux = cx + k % 3 - 1, uy = cy + (k / 3) % 3 - 1, uz = cz + k / 9 - 1;
+            const int sx = (ux < 0) ? -1 : (ux >= ncx ? 1 : 0);
+            const int sy = (uy < 0) ? -1 : (uy >= ncy ? 1 : 0);
+            const int sz = (uz < 0) ? -1 : (uz >= ncz ? 1 : 0);
+            const int nc = (ux - sx * ncx) + ncx * ((uy - sy * ncy) + ncy * (uz - sz * ncz));
+            k_base[k] = cell_start[nc];
+            cnt = cell_start[nc + 1] - cell_start[nc];
+            k_code[k] = shift_code(sx, sy, sz);
+            k_dx[k] = sx * Lx;
+            k_dy[k] = sy * Ly;
+            k_dz[k] = sz * Lz;
+        }
+        int incl = cnt;   // prefix sum over the 27 cells
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+            const int v = __shfl_up(incl, o);
+            if (tid >= o) incl += v;
+        }
+        if (tid < 28) k_off[tid] = incl - cnt;
     }
     __syncthreads();
     const int total = k_off[27];
-    const int g = lane / NSUB, sub = lane % NSUB;
-    const unsigned long long group = 0xFFull << (lane & ~(NSUB - 1));
+    const int lane = tid & 63, g = tid / SUB, sub = tid % SUB;
+    const unsigned long long group = ((1ull << SUB) - 1) << (lane & ~(SUB - 1));
     const unsigned long long below = (1ull << lane) - 1;
     const int self_code = shift_code(0, 0, 0);
-    for (int a0 = 0; a0 < cn; a0 += 64 / NSUB) {
+    for (int a0 = 0; a0 < cn; a0 += TH / SUB) {
         const bool live = a0 + g < cn;
         const int i = live ? cell_atoms[cb + a0 + g] : 0;
         const double xi = live ? x[3 * i] : 0.0, yi = live ? x[3 * i + 1] : 0.0, zi = live ? x[3 * i + 2] : 0.0;
         int cnt = 0;
         for (int t0 = 0; t0 < total; t0 += NTILE) {
             const int nt = min(NTILE, total - t0);
-            __syncthreads();   // the previous pass has finished reading the tile
-            for (int t = lane; t < nt; t += 64) {
-                const int tt = t0 + t;
-                int k = 0;   // the cell holding candidate tt: k_off[k] <= tt < k_off[k + 1]
+            if (a0 == 0 || total > NTILE) {   // uniform
+                __syncthreads();   // the previous pass has finished reading the tile
+                for (int t = tid; t < nt; t += TH) {
+                    const int tt = t0 + t;
+                    int k = 0;   // the cell holding candidate tt: k_off[k] <= tt < k_off[k + 1]
 #pragma unroll
-                for (int step = 16; step > 0; step >>= 1)
-                    if (k + step < 27 && k_off[k + step] <= tt) k += step;
-                const int j = cell_atoms[k_base[k] + tt - k_off[k]];
-                {
+                    for (int step = 16; step > 0; step >>= 1)
+                        if (k + step < 27 && k_off[k + step] <= tt) k += step;
+                    const int j = cell_atoms[k_base[k] + tt - k_off[k]];
+                    {
 #pragma clang fp contract(off)
-                    tx[t] = x[3 * j] + k_dx[k];
-                    ty[t] = x[3 * j + 1] + k_dy[k];
-                    tz[t] = x[3 * j + 2] + k_dz[k];
+                        tx[t] = x[3 * j] + k_dx[k];
+                        ty[t] = x[3 * j + 1] + k_dy[k];
+                        tz[t] = x[3 * j + 2] + k_dz[k];
+                    }
+                    tj[t] = j;
+                    ts[t] = k_code[k];
                 }
-                tj[t] = j;
-                ts[t] = k_code[k];
+                __syncthreads();
             }
-            __syncthreads();
-            for (int m0 = 0; m0 < nt; m0 += NSUB) {   // uniform trip count
+            for (int m0 = 0; m0 < nt; m0 += SUB) {   // uniform trip count
                 const int m = m0 + sub;
                 bool acc = false;
                 int j = 0;
@@ -426,10 +441,7 @@ __global__ __launch_bounds__(64) void k_neighbors_tile(const double* __restrict_
                 const unsigned long long mk = __ballot(acc) & group;
                 if (acc) {
                     const int q = cnt + __popcll(mk & below);
-                    if (q < NBMAX) {
-                        nb_j[static_cast<size_t>(q) * N + i] = j;
-                        nb_s[static_cast<size_t>(q) * N + i] = ts[m];
-                    }
+                    if (q < NBMAX) nbr[static_cast<size_t>(i) * NBMAX + q] = make_int2(j, ts[m]);
                 }
                 cnt += __popcll(mk);
             }
@@ -441,81 +453,103 @@ __global__ __launch_bounds__(64) void k_neighbors_tile(const double* __restrict_
     }
 }
 
-// Small boxes (fewer than three cells along an axis): every atom against every periodic image.
-__global__ void k_neighbors_brute(const double* __restrict__ x, int* __restrict__ nb_cnt, int* __restrict__ nb_j,
-                                  int* __restrict__ nb_s, double Lx, double Ly, double Lz, double rcs, double rcs2,
-                                  int N, int* __restrict__ overflow) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
+// Small boxes (fewer than three cells along an axis): every atom against the periodic images that can reach it.
+// One wave per atom: images in the order (sz, sy, sx), 64 atoms j at a time, accepted ones ranked by a ballot, so
+// the list keeps the order image, then j.  Positions are wrapped into [0, L), so image s of an axis lies in
+// [sL, sL + L) and is skipped where that interval is out of reach of x_i (with a margin far above rounding):
+// about 6 of the 125 images of a 128-atom cell remain.  128 atoms at rcut + skin 5.1 A: 1,659 us with one lane
+// per atom walking all images.
+__global__ __launch_bounds__(256) void k_neighbors_brute(const double* __restrict__ x, int* __restrict__ nb_cnt,
+                                                         int2* __restrict__ nbr, double Lx, double Ly, double Lz,
+                                                         double rcs, double rcs2, int N, int* __restrict__ overflow) {
+    const int i = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= N) return;   // uniform over the wave
     const int rx = min(static_cast<int>(ceil(rcs / Lx)) + 1, SHK), ry = min(static_cast<int>(ceil(rcs / Ly)) + 1, SHK),
               rz = min(static_cast<int>(ceil(rcs / Lz)) + 1, SHK);
     const double xi = x[3 * i], yi = x[3 * i + 1], zi = x[3 * i + 2];
+    auto beyond = [&](int s, double L, double c) {
+        const double lo = s * L - c, far = rcs + 1e-9 * (rcs + L);
+        return lo > far || lo + L < -far;
+    };
+    const unsigned long long below = (1ull << lane) - 1;
     int cnt = 0;
-    for (int sz = -rz; sz <= rz; ++sz)
-        for (int sy = -ry; sy <= ry; ++sy)
-            for (int sx = -rx; sx <= rx; ++sx)
-                for (int j = 0; j < N; ++j) {
-                    if (j == i && sx == 0 && sy == 0 && sz == 0) continue;
-                    const double d2 = dist2_nc(image_nc(x[3 * j], sx, Lx, xi), image_nc(x[3 * j + 1], sy, Ly, yi),
-                                               image_nc(x[3 * j + 2], sz, Lz, zi));
-                    if (d2 <= rcs2) {
-                        if (cnt < NBMAX) {
-                            nb_j[static_cast<size_t>(cnt) * N + i] = j;
-                            nb_s[static_cast<size_t>(cnt) * N + i] = shift_code(sx, sy, sz);
-                        }
-                        ++cnt;
+    for (int sz = -rz; sz <= rz; ++sz) {
+        if (beyond(sz, Lz, zi)) continue;
+        for (int sy = -ry; sy <= ry; ++sy) {
+            if (beyond(sy, Ly, yi)) continue;
+            for (int sx = -rx; sx <= rx; ++sx) {
+                if (beyond(sx, Lx, xi)) continue;
+                const bool self = sx == 0 && sy == 0 && sz == 0;
+                const int code = shift_code(sx, sy, sz);
+                for (int j0 = 0; j0 < N; j0 += 64) {
+                    const int j = j0 + lane;
+                    bool acc = false;
+                    if (j < N) {
+                        const double d2 = dist2_nc(image_nc(x[3 * j], sx, Lx, xi), image_nc(x[3 * j + 1], sy, Ly, yi),
+                                                   image_nc(x[3 * j + 2], sz, Lz, zi));
+                        acc = d2 <= rcs2 && !(self && j == i);
                     }
+                    const unsigned long long mk = __ballot(acc);
+                    if (acc) {
+                        const int q = cnt + __popcll(mk & below);
+                        if (q < NBMAX) nbr[static_cast<size_t>(i) * NBMAX + q] = make_int2(j, code);
+                    }
+                    cnt += __popcll(mk);
                 }
-    if (cnt > NBMAX) atomicOr(overflow, 1);
-    nb_cnt[i] = min(cnt, NBMAX);
+            }
+        }
+    }
+    if (lane == 0) {
+        if (cnt > NBMAX) atomicOr(overflow, 1);
+        nb_cnt[i] = min(cnt, NBMAX);
+    }
 }
 
-// total of the per-atom entry counts: one atomic per workgroup
-__global__ __launch_bounds__(256) void k_sum_counts(const int* __restrict__ cnt, int N,
-                                                    unsigned long long* __restrict__ total) {
-    __shared__ unsigned long long part[4];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long v = i < N ? static_cast<unsigned long long>(cnt[i]) : 0ull;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(total, part[0] + part[1] + part[2] + part[3]);
-}
+// Incoming entries: every entry e = (i -> j) is appended to j's list (slot k of atom j at j*NBMAX + k), 16 lanes
+// per atom, one atomic per entry; each list is then put in ascending order, and the entries are counted.
+constexpr int PSUB = 16;   // lanes that share an atom in the per-atom kernels
 
-// incoming entries: for every entry e = (i -> j) append e to j's list, then sort each list.  The lists are
-// atom-major (slot k of atom j at j*NBMAX + k): the tally's 16 lanes per atom then read one contiguous run.
-__global__ void k_incoming(const int* __restrict__ nb_cnt, const int* __restrict__ nb_j, int* __restrict__ in_cnt,
-                           int* __restrict__ in_e, int N, int* __restrict__ overflow) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    for (int k = 0; k < nb_cnt[i]; ++k) {
-        const int e = k * N + i;
-        const int j = nb_j[e];
+__global__ __launch_bounds__(256) void k_incoming(const int* __restrict__ nb_cnt, const int2* __restrict__ nbr,
+                                                  int* __restrict__ in_cnt, int* __restrict__ in_e, int N,
+                                                  int* __restrict__ overflow, unsigned long long* __restrict__ total) {
+    __shared__ int part[256 / PSUB];
+    const int t = blockIdx.x * 256 + threadIdx.x, i = t / PSUB, sub = t % PSUB;
+    const int n = i < N ? nb_cnt[i] : 0;
+    for (int k = sub; k < n; k += PSUB) {
+        const int e = i * NBMAX + k, j = nbr[e].x;
         const int slot = atomicAdd(&in_cnt[j], 1);
         if (slot < NBMAX)
             in_e[static_cast<size_t>(j) * NBMAX + slot] = e;
         else
             atomicOr(overflow, 4);
     }
+    if (sub == 0) part[threadIdx.x / PSUB] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long v = 0;
+        for (int k = 0; k < 256 / PSUB; ++k) v += static_cast<unsigned long long>(part[k]);
+        if (v) atomicAdd(total, v);
+    }
 }
 
-__global__ void k_incoming_sort(int* __restrict__ in_cnt, int* __restrict__ in_e, int N) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int n = min(in_cnt[i], NBMAX);
-    in_cnt[i] = n;
-    int* a = in_e + static_cast<size_t>(i) * NBMAX;   // slot k at a[k]
-    const size_t st = 1;
-    for (int k = 1; k < n; ++k) {
-        const int v = a[k * st];
-        int m = k - 1;
-        while (m >= 0 && a[m * st] > v) {
-            a[(m + 1) * st] = a[m * st];
-            --m;
-        }
-        a[(m + 1) * st] = v;
+// ascending order of each atom's incoming list: 16 lanes per atom rank its entries from an LDS copy.  (One lane per
+// atom sorting by insertion took 20 us at 250 atoms and 63 us at 128,000.)
+__global__ __launch_bounds__(256) void k_incoming_sort(int* __restrict__ in_cnt, int* __restrict__ in_e, int N) {
+    constexpr int APB = 256 / PSUB;
+    __shared__ int list[APB][NBMAX];
+    const int t = blockIdx.x * 256 + threadIdx.x, i = t / PSUB, sub = t % PSUB;
+    int* __restrict__ a = in_e + static_cast<size_t>(i) * NBMAX;
+    int* l = list[threadIdx.x / PSUB];
+    const int n = i < N ? min(in_cnt[i], NBMAX) : 0;
+    for (int k = sub; k < n; k += PSUB) l[k] = a[k];
+    __syncthreads();
+    for (int k = sub; k < n; k += PSUB) {
+        const int v = l[k];
+        int rank = 0;
+        for (int m = 0; m < n; ++m) rank += l[m] < v;
+        a[rank] = v;
     }
+    if (i < N && sub == 0) in_cnt[i] = n;
 }
 
 __device__ __forceinline__ void entry_disp(const double* __restrict__ x, int i, int j, int code, double Lx, double Ly,
@@ -529,10 +563,10 @@ __device__ __forceinline__ void entry_disp(const double* __restrict__ x, int i, 
 
 // pairs per atom (entries within the pair cutoff); 16 lanes per atom as in k_pair_fill_md below
 __global__ __launch_bounds__(256) void k_pair_count_md(const double* __restrict__ x, const int* __restrict__ type,
-                                                       const int* __restrict__ nb_cnt, const int* __restrict__ nb_j,
-                                                       const int* __restrict__ nb_s, const double* __restrict__ rc2_tt,
-                                                       int ntypes, int* __restrict__ pcnt, double Lx, double Ly,
-                                                       double Lz, int N) {
+                                                       const int* __restrict__ nb_cnt, const int2* __restrict__ nbr,
+                                                       const double* __restrict__ rc2_tt, int ntypes,
+                                                       int* __restrict__ pcnt, double Lx, double Ly, double Lz,
+                                                       int N) {
     constexpr int SUB = 16;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int i = t / SUB, sub = t % SUB, lane = threadIdx.x & 63;
@@ -545,9 +579,10 @@ __global__ __launch_bounds__(256) void k_pair_count_md(const double* __restrict_
         const int k = k0 + sub;
         bool acc = false;
         if (k < n) {
-            const int e = k * N + i, j = nb_j[e];
+            const int2 nj = nbr[i * NBMAX + k];
+            const int j = nj.x;
             double dx, dy, dz;
-            entry_disp(x, i, j, nb_s[e], Lx, Ly, Lz, dx, dy, dz);
+            entry_disp(x, i, j, nj.y, Lx, Ly, Lz, dx, dy, dz);
             const double d2 = dist2_nc(dx, dy, dz);
             acc = d2 < rc2_tt[ti * (ntypes + 1) + type[j]] && d2 > 1e-20;
         }
@@ -560,12 +595,10 @@ __global__ __launch_bounds__(256) void k_pair_count_md(const double* __restrict_
 // consecutive pair slots from a ballot, so a wave's stores cover a few contiguous pair ranges (one per
 // atom) instead of 64 scattered slots.  Pair order within an atom is the entry order, as with one lane
 // per atom.
-constexpr int PSUB = 16;
-
 __global__ __launch_bounds__(256) void k_pair_fill_md(const double* __restrict__ x, const int* __restrict__ type,
-                                                      const int* __restrict__ nb_cnt, const int* __restrict__ nb_j,
-                                                      const int* __restrict__ nb_s, const double* __restrict__ rc2_tt,
-                                                      int ntypes, const int* __restrict__ poff, int* __restrict__ pi_,
+                                                      const int* __restrict__ nb_cnt, const int2* __restrict__ nbr,
+                                                      const double* __restrict__ rc2_tt, int ntypes,
+                                                      const int* __restrict__ poff, int* __restrict__ pi_,
                                                       int* __restrict__ pj, int* __restrict__ pti,
                                                       int* __restrict__ ptj, double* __restrict__ prij,
                                                       int* __restrict__ entry_pair, double Lx, double Ly, double Lz,
@@ -584,11 +617,12 @@ __global__ __launch_bounds__(256) void k_pair_fill_md(const double* __restrict__
         int j = 0, tjv = 0;
         double dx = 0.0, dy = 0.0, dz = 0.0;
         bool acc = false;
-        const int e = k * N + i;
+        const int e = i * NBMAX + k;
         if (valid) {
-            j = nb_j[e];
+            const int2 nj = nbr[e];
+            j = nj.x;
             tjv = type[j];
-            entry_disp(x, i, j, nb_s[e], Lx, Ly, Lz, dx, dy, dz);
+            entry_disp(x, i, j, nj.y, Lx, Ly, Lz, dx, dy, dz);
             const double d2 = dist2_nc(dx, dy, dz);
             acc = d2 < rc2_tt[ti * (ntypes + 1) + tjv] && d2 > 1e-20;
         }
@@ -711,8 +745,7 @@ __global__ void k_vv2(double* __restrict__ v, const double* __restrict__ f, cons
 // xij = x_j - x_i.  Each atom owns its sums, so there are no atomics; 16 lanes per atom take every 16th
 // entry and combine by a butterfly.  zacc[10 i + c]: force x, y, z, virial xx, yy, zz, xy, xz, yz, energy.
 __global__ __launch_bounds__(256) void k_zbl_md(const double* __restrict__ x, const int* __restrict__ nb_cnt,
-                                                const int* __restrict__ nb_j, const int* __restrict__ nb_s,
-                                                double Lx, double Ly, double Lz, int N, ZblParams zp,
+                                                const int2* __restrict__ nbr, double Lx, double Ly, double Lz, int N, ZblParams zp,
                                                 double* __restrict__ zacc) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int i = t / PSUB, sub = t % PSUB;
@@ -721,9 +754,9 @@ __global__ __launch_bounds__(256) void k_zbl_md(const double* __restrict__ x, co
     if (live) {
         const int n = nb_cnt[i];
         for (int k = sub; k < n; k += PSUB) {
-            const int e = k * N + i;
+            const int2 nj = nbr[i * NBMAX + k];
             double dx, dy, dz;
-            entry_disp(x, i, nb_j[e], nb_s[e], Lx, Ly, Lz, dx, dy, dz);
+            entry_disp(x, i, nj.x, nj.y, Lx, Ly, Lz, dx, dy, dz);
             const double d2 = dist2_nc(dx, dy, dz);
             if (d2 <= zp.rout2) {
                 const double r = sqrt(d2);
@@ -793,9 +826,22 @@ struct mdp_md {
     DevTables tab;
     std::vector<double> massinv_h, rc2_h;
     // device state
-    DevBuf x, v, f, type, massinv, xref, cell_of, cell_cnt, cell_start, cell_fill, cell_atoms, scan_tmp, nb_cnt, nb_j,
-        nb_s, in_cnt, in_e, pcnt, poff, pi, pj, pti, ptj, prij, entry_pair, Ur, Ui, Yr, Yi, epart, dedr, eatom, vir,
-        beta_t, rc2, flags, maxd2, row_order, yt, pair_sum, pgeo, zacc;
+    // cleared: what a rebuild starts from zero (ClearedPart), cleared by one fill
+    DevBuf x, v, f, type, massinv, xref, cell_of, cleared, cell_start, cell_atoms, scan_tmp, nb_cnt, nbr, in_e, pcnt, poff, pi, pj, pti, ptj, prij, entry_pair, Ur, Ui, Yr, Yi, epart, dedr, eatom, vir,
+        beta_t, rc2, row_order, yt, pair_sum, pgeo, zacc;
+    // Layout of `cleared`: the rebuild's report to the host (max displacement^2 bits, neighbour entries, flags),
+    // then incoming counts per atom, cell counts and cell fill positions.
+    struct Report {
+        unsigned long long maxd2, entries;
+        int flags[4];
+    };
+    Report* report_h = nullptr;   // pinned
+    Report* report() const { return static_cast<Report*>(cleared.p); }
+    int* in_cnt() const { return reinterpret_cast<int*>(report() + 1); }
+    size_t cell_count() const { return static_cast<size_t>(ncell[0]) * ncell[1] * ncell[2]; }
+    int* cell_cnt() const { return in_cnt() + N; }
+    int* cell_fill() const { return cell_cnt() + cell_count() + 1; }
+    size_t cleared_bytes() const { return sizeof(Report) + sizeof(int) * (N + 2 * (cell_count() + 1)); }
     // Nose-Hoover NVT (mdp_md_set_nvt); off: NVE
     bool nvt = false;
     double nvt_tstart = 0, nvt_tstop = 0, nvt_tfreq = 0, nvt_drag = 0, nvt_tdof = 0;
@@ -869,6 +915,7 @@ struct mdp_md {
         if (st) {
             (void)hipStreamSynchronize(st);
             for (auto e : ev_pool) (void)hipEventDestroy(e);
+            if (report_h) (void)hipHostFree(report_h);
             (void)hipStreamDestroy(st);
         }
     }
@@ -961,15 +1008,13 @@ struct mdp_md {
         MDP_HIP(hipMemsetAsync(f.p, 0, sizeof(double) * 3 * n, st));
         xref.ensure(sizeof(double) * 3 * n);
         cell_of.ensure(sizeof(int) * n);
-        cell_cnt.ensure(sizeof(int) * (ncells + 1));
+        cleared.ensure(cleared_bytes());
+        MDP_HIP(hipHostMalloc(reinterpret_cast<void**>(&report_h), sizeof(Report), hipHostMallocDefault));
         cell_start.ensure(sizeof(int) * (ncells + 1));
-        cell_fill.ensure(sizeof(int) * (ncells + 1));
         cell_atoms.ensure(sizeof(int) * n);
         scan_tmp.ensure(sizeof(int) * (scan_tmp_ints(static_cast<int>(std::max(n, ncells))) + 8));
         nb_cnt.ensure(sizeof(int) * n);
-        nb_j.ensure(sizeof(int) * n * NBMAX);
-        nb_s.ensure(sizeof(int) * n * NBMAX);
-        in_cnt.ensure(sizeof(int) * n);
+        nbr.ensure(sizeof(int2) * n * NBMAX);
         in_e.ensure(sizeof(int) * n * NBMAX);
         pcnt.ensure(sizeof(int) * n);
         poff.ensure(sizeof(int) * (n + 1));
@@ -981,8 +1026,6 @@ struct mdp_md {
         epart.ensure(sizeof(double) * n * nrows);
         eatom.ensure(sizeof(double) * n);
         vir.ensure(sizeof(double) * 6 * n);
-        flags.ensure(sizeof(int) * 4);
-        maxd2.ensure(2 * sizeof(unsigned long long));   // [0] max displacement^2 bits, [1] neighbour entries
         pair_sum.ensure(sizeof(unsigned long long));
         MDP_HIP(hipMemsetAsync(pair_sum.p, 0, sizeof(unsigned long long), st));
         MDP_HIP(hipMemsetAsync(Yr.p, 0, sizeof(double) * n * iu, st));
@@ -1002,77 +1045,74 @@ struct mdp_md {
         dedr.ensure(sizeof(double) * 3 * c);
     }
 
-    // the cell-list neighbour kernel: 0 = eight lanes per atom through L1, 1 = the per-wavefront LDS tile
+    // the cell-list neighbour kernel: 0 = eight lanes per atom through L1, 1 = the LDS tile on 128 lanes per cell,
+    // 2 = on 256 lanes
     void neighbors_launch(int v) {
         const double rcs = rcnb;
+        const dim3 cells(static_cast<unsigned>(cell_count()));
         if (v == 1)
-            hipLaunchKernelGGL(k_neighbors_tile, dim3(static_cast<unsigned>(ncell[0] * ncell[1] * ncell[2])), dim3(64), 0,
-                               st, x.as<double>(), cell_start.as<int>(), cell_atoms.as<int>(), nb_cnt.as<int>(),
-                               nb_j.as<int>(), nb_s.as<int>(), L[0], L[1], L[2], ncell[0], ncell[1], ncell[2],
-                               rcs * rcs, N, flags.as<int>());
+            hipLaunchKernelGGL((k_neighbors_tile<128, 8>), cells, dim3(128), 0, st, x.as<double>(), cell_start.as<int>(),
+                               cell_atoms.as<int>(), nb_cnt.as<int>(), nbr.as<int2>(), L[0], L[1], L[2], ncell[0],
+                               ncell[1], ncell[2], rcs * rcs, N, report()->flags);
+        else if (v == 2)
+            hipLaunchKernelGGL((k_neighbors_tile<256, 16>), cells, dim3(256), 0, st, x.as<double>(),
+                               cell_start.as<int>(), cell_atoms.as<int>(), nb_cnt.as<int>(), nbr.as<int2>(), L[0], L[1],
+                               L[2], ncell[0], ncell[1], ncell[2], rcs * rcs, N, report()->flags);
         else
             hipLaunchKernelGGL(k_neighbors_cell, dim3(nb(static_cast<long>(N) * NSUB, 256)), dim3(256), 0, st,
                                x.as<double>(), cell_of.as<int>(), cell_start.as<int>(), cell_atoms.as<int>(),
-                               nb_cnt.as<int>(), nb_j.as<int>(), nb_s.as<int>(), L[0], L[1], L[2], ncell[0], ncell[1],
-                               ncell[2], rcs * rcs, N, flags.as<int>());
+                               nb_cnt.as<int>(), nbr.as<int2>(), L[0], L[1], L[2], ncell[0], ncell[1], ncell[2],
+                               rcs * rcs, N, report()->flags);
     }
 
     void rebuild(bool check_disp) {
         const double rcs = rcnb;
-        const size_t ncells = static_cast<size_t>(ncell[0]) * ncell[1] * ncell[2];
-        MDP_HIP(hipMemsetAsync(cell_cnt.p, 0, sizeof(int) * (ncells + 1), st));
-        MDP_HIP(hipMemsetAsync(cell_fill.p, 0, sizeof(int) * (ncells + 1), st));
-        MDP_HIP(hipMemsetAsync(flags.p, 0, sizeof(int) * 4, st));
-        MDP_HIP(hipMemsetAsync(maxd2.p, 0, 2 * sizeof(unsigned long long), st));
-        MDP_HIP(hipMemsetAsync(in_cnt.p, 0, sizeof(int) * N, st));
+        const size_t ncells = cell_count();
+        MDP_HIP(hipMemsetAsync(cleared.p, 0, cleared_bytes(), st));
         hipLaunchKernelGGL(k_wrap_bin, dim3(nb(N, 256)), dim3(256), 0, st, x.as<double>(), xref.as<double>(),
-                           cell_of.as<int>(), cell_cnt.as<int>(), maxd2.as<unsigned long long>(), L[0], L[1], L[2],
-                           ncell[0], ncell[1], ncell[2], N, check_disp ? 1 : 0, flags.as<int>());
+                           cell_of.as<int>(), cell_cnt(), &report()->maxd2, L[0], L[1], L[2], ncell[0], ncell[1],
+                           ncell[2], N, check_disp ? 1 : 0, report()->flags);
         if (use_cells) {
-            exclusive_scan(cell_cnt.as<int>(), cell_start.as<int>(), static_cast<int>(ncells), scan_tmp.as<int>(), st);
+            exclusive_scan(cell_cnt(), cell_start.as<int>(), static_cast<int>(ncells), scan_tmp.as<int>(), st);
             hipLaunchKernelGGL(k_cell_fill, dim3(nb(N, 256)), dim3(256), 0, st, cell_of.as<int>(), cell_start.as<int>(),
-                               cell_fill.as<int>(), cell_atoms.as<int>(), N);
-            hipLaunchKernelGGL(k_cell_sort, dim3(nb(static_cast<long>(ncells), 256)), dim3(256), 0, st,
-                               cell_start.as<int>(), cell_atoms.as<int>(), static_cast<int>(ncells), flags.as<int>());
+                               cell_fill(), cell_atoms.as<int>(), N);
+            hipLaunchKernelGGL(k_cell_sort, dim3(nb(static_cast<long>(ncells), 4)), dim3(256), 0, st,
+                               cell_start.as<int>(), cell_atoms.as<int>(), static_cast<int>(ncells), report()->flags);
             neighbors_launch(nb_variant);
         } else {
-            hipLaunchKernelGGL(k_neighbors_brute, dim3(nb(N, 64)), dim3(64), 0, st, x.as<double>(), nb_cnt.as<int>(),
-                               nb_j.as<int>(), nb_s.as<int>(), L[0], L[1], L[2], rcs, rcs * rcs, N, flags.as<int>());
+            hipLaunchKernelGGL(k_neighbors_brute, dim3(nb(N, 4)), dim3(256), 0, st, x.as<double>(), nb_cnt.as<int>(),
+                               nbr.as<int2>(), L[0], L[1], L[2], rcs, rcs * rcs, N, report()->flags);
         }
-        hipLaunchKernelGGL(k_incoming, dim3(nb(N, 256)), dim3(256), 0, st, nb_cnt.as<int>(), nb_j.as<int>(),
-                           in_cnt.as<int>(), in_e.as<int>(), N, flags.as<int>());
-        hipLaunchKernelGGL(k_incoming_sort, dim3(nb(N, 256)), dim3(256), 0, st, in_cnt.as<int>(), in_e.as<int>(), N);
-        hipLaunchKernelGGL(k_sum_counts, dim3(nb(N, 256)), dim3(256), 0, st, nb_cnt.as<int>(), N,
-                           maxd2.as<unsigned long long>() + 1);
+        const dim3 per_atom(nb(static_cast<long>(N) * PSUB, 256));
+        hipLaunchKernelGGL(k_incoming, per_atom, dim3(256), 0, st, nb_cnt.as<int>(), nbr.as<int2>(), in_cnt(),
+                           in_e.as<int>(), N, report()->flags, &report()->entries);
+        hipLaunchKernelGGL(k_incoming_sort, per_atom, dim3(256), 0, st, in_cnt(), in_e.as<int>(), N);
         // a single small readback per rebuild: overflow flags, displacement and entry count
-        int fl[4];
-        unsigned long long md2[2] = {0, 0};
-        MDP_HIP(hipMemcpyAsync(fl, flags.p, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
-        MDP_HIP(hipMemcpyAsync(md2, maxd2.p, sizeof(md2), hipMemcpyDeviceToHost, st));
+        MDP_HIP(hipMemcpyAsync(report_h, report(), sizeof(Report), hipMemcpyDeviceToHost, st));
         MDP_HIP(hipStreamSynchronize(st));
-        if (fl[0]) {
+        const int fl = report_h->flags[0];
+        if (fl) {
             stats[5] += 1;
-            throw Error(std::string("neighbour build failed:") + ((fl[0] & 1) ? " >96 neighbours per atom" : "") +
-                        ((fl[0] & 2) ? " >48 atoms per cell" : "") + ((fl[0] & 4) ? " >96 incoming entries" : "") +
-                        ((fl[0] & 8) ? " non-finite or runaway positions" : ""));
+            throw Error(std::string("neighbour build failed:") + ((fl & 1) ? " >96 neighbours per atom" : "") +
+                        ((fl & 2) ? " >48 atoms per cell" : "") + ((fl & 4) ? " >96 incoming entries" : "") +
+                        ((fl & 8) ? " non-finite or runaway positions" : ""));
         }
         double d2;
-        std::memcpy(&d2, &md2[0], sizeof(d2));
+        std::memcpy(&d2, &report_h->maxd2, sizeof(d2));
         stats[2] += 1;
         if (check_disp && d2 > 0.25 * skin * skin) stats[3] += 1;
         // entry count bounds the pair count until the next rebuild
-        const long tot = static_cast<long>(md2[1]);
+        const long tot = static_cast<long>(report_h->entries);
         stats[1] = tot;
         ensure_pairs(static_cast<size_t>(tot));
     }
 
     void pairs() {
         hipLaunchKernelGGL(k_pair_count_md, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, x.as<double>(), type.as<int>(),
-                           nb_cnt.as<int>(), nb_j.as<int>(), nb_s.as<int>(), rc2.as<double>(), ntypes, pcnt.as<int>(),
-                           L[0], L[1], L[2], N);
+                           nb_cnt.as<int>(), nbr.as<int2>(), rc2.as<double>(), ntypes, pcnt.as<int>(), L[0], L[1], L[2], N);
         exclusive_scan(pcnt.as<int>(), poff.as<int>(), N, scan_tmp.as<int>(), st);
         hipLaunchKernelGGL(k_pair_fill_md, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, x.as<double>(), type.as<int>(),
-                           nb_cnt.as<int>(), nb_j.as<int>(), nb_s.as<int>(), rc2.as<double>(), ntypes, poff.as<int>(),
+                           nb_cnt.as<int>(), nbr.as<int2>(), rc2.as<double>(), ntypes, poff.as<int>(),
                            pi.as<int>(), pj.as<int>(), pti.as<int>(), ptj.as<int>(), prij.as<double>(),
                            entry_pair.as<int>(), L[0], L[1], L[2], N, tab.view, pgeo.as<double>());
     }
@@ -1095,8 +1135,7 @@ struct mdp_md {
         if (!zbl) return;
         timed(T_PAIRPOT, [&] {
             hipLaunchKernelGGL(k_zbl_md, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, x.as<double>(),
-                               nb_cnt.as<int>(), nb_j.as<int>(), nb_s.as<int>(), L[0], L[1], L[2], N, zp,
-                               zacc.as<double>());
+                               nb_cnt.as<int>(), nbr.as<int2>(), L[0], L[1], L[2], N, zp, zacc.as<double>());
         });
     }
 
@@ -1112,12 +1151,11 @@ struct mdp_md {
         const bool cells = nc[0] >= 3 && nc[1] >= 3 && nc[2] >= 3;
         if (!cells && N > 200000) throw Error("mdp_md_set_zbl: box too small for cell lists at this atom count");
         const size_t ncells = static_cast<size_t>(nc[0]) * nc[1] * nc[2];
-        cell_cnt.ensure(sizeof(int) * (ncells + 1));
         cell_start.ensure(sizeof(int) * (ncells + 1));
-        cell_fill.ensure(sizeof(int) * (ncells + 1));
         scan_tmp.ensure(sizeof(int) * (scan_tmp_ints(static_cast<int>(std::max(static_cast<size_t>(N), ncells))) + 8));
         zacc.ensure(sizeof(double) * 10 * static_cast<size_t>(N));
         for (int d = 0; d < 3; ++d) ncell[d] = nc[d];
+        cleared.ensure(cleared_bytes());
         use_cells = cells;
         rcnb = rcs;
         zp = zbl_params(cut_inner, cut_outer, z);
@@ -1153,7 +1191,7 @@ struct mdp_md {
         pair_potential();
         timed(T_TALLY, [&] {
             hipLaunchKernelGGL(k_tally, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, dedr.as<double>(), prij.as<double>(),
-                               poff.as<int>(), in_cnt.as<int>(), in_e.as<int>(), entry_pair.as<int>(),
+                               poff.as<int>(), in_cnt(), in_e.as<int>(), entry_pair.as<int>(),
                                epart.as<double>(), nrows, e0, nullptr, fo, vo, eo, v.as<double>(), type.as<int>(),
                                massinv.as<double>(), dtf, integrate ? 1 : 0, N, count ? pair_sum.as<unsigned long long>() : nullptr,
                                zbl ? zacc.as<double>() : nullptr);
@@ -1239,7 +1277,7 @@ struct mdp_md {
         pair_potential();
         timed(T_TALLY, [&] {
             hipLaunchKernelGGL(k_tally, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, dedr.as<double>(), prij.as<double>(),
-                               poff.as<int>(), in_cnt.as<int>(), in_e.as<int>(), entry_pair.as<int>(),
+                               poff.as<int>(), in_cnt(), in_e.as<int>(), entry_pair.as<int>(),
                                epart.as<double>(), 0, 0.0, sE.as<double>(), f.as<double>(), vir.as<double>(),
                                eatom.as<double>(), v.as<double>(), type.as<int>(), massinv.as<double>(), dtf,
                                integrate ? 1 : 0, N, pair_sum.as<unsigned long long>(), zbl ? zacc.as<double>() : nullptr);
@@ -1362,13 +1400,13 @@ struct mdp_md {
             if (t < best) { best = t; ui_variant = uids[k]; }
         }
         // cell-list neighbour kernel (when the box has cell lists): both write the same lists from the
-        // cell arrays of the last rebuild; MDP_NB_VARIANT pins 0 or 1
+        // cell arrays of the last rebuild; MDP_NB_VARIANT pins one of 0, 1, 2
         if (use_cells) {
             js += "}, \"neighbor_build\": {";
-            int nids[2] = {0, 1}, nn = 2;
+            int nids[3] = {0, 1, 2}, nn = 3;
             if (const char* np_ = std::getenv("MDP_NB_VARIANT")) {
                 const int v = std::atoi(np_);
-                if (v != 0 && v != 1) throw Error("MDP_NB_VARIANT is not a neighbour kernel variant (0 or 1)");
+                if (v < 0 || v > 2) throw Error("MDP_NB_VARIANT is not a neighbour kernel variant (0, 1 or 2)");
                 nids[0] = v;
                 nn = 1;
             }
@@ -1630,21 +1668,22 @@ int mdp_md_neighbors(mdp_md* md, int* off, int* nbj, int* nbshift, long* nentrie
     return api([&] {
         const int N = md->N;
         MDP_HIP(hipStreamSynchronize(md->st));
-        std::vector<int> cnt(N), js(static_cast<size_t>(N) * NBMAX), ss(static_cast<size_t>(N) * NBMAX);
+        std::vector<int> cnt(N);
+        std::vector<int2> entries(static_cast<size_t>(N) * NBMAX);
         MDP_HIP(hipMemcpy(cnt.data(), md->nb_cnt.p, sizeof(int) * N, hipMemcpyDeviceToHost));
         long tot = 0;
         for (int c : cnt) tot += c;
         if (nentries) *nentries = tot;
         if (!nbj) return;
-        MDP_HIP(hipMemcpy(js.data(), md->nb_j.p, sizeof(int) * js.size(), hipMemcpyDeviceToHost));
-        MDP_HIP(hipMemcpy(ss.data(), md->nb_s.p, sizeof(int) * ss.size(), hipMemcpyDeviceToHost));
+        MDP_HIP(hipMemcpy(entries.data(), md->nbr.p, sizeof(int2) * entries.size(), hipMemcpyDeviceToHost));
         long k = 0;
         for (int i = 0; i < N; ++i) {
             off[i] = static_cast<int>(k);
             for (int m = 0; m < cnt[i]; ++m, ++k) {
-                nbj[k] = js[static_cast<size_t>(m) * N + i];
+                const int2 e = entries[static_cast<size_t>(i) * NBMAX + m];
+                nbj[k] = e.x;
                 int sx, sy, sz;
-                shift_decode(ss[static_cast<size_t>(m) * N + i], sx, sy, sz);
+                shift_decode(e.y, sx, sy, sz);
                 nbshift[3 * k] = sx;
                 nbshift[3 * k + 1] = sy;
                 nbshift[3 * k + 2] = sz;

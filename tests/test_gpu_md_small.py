@@ -1,0 +1,56 @@
+"""MD engine kernels whose work is split for systems too small to fill the GPU, at the sizes where the split can
+go wrong: one atom, a block of 64 atoms less one and plus one, boxes with a single cell along an axis.
+
+Neighbour lists are compared as sorted sets, bit for bit, with the oracle's brute force; energies, forces and
+virials with the oracle's force chain within 1e-10 of the max norm, as in test_gpu_md.py.
+"""
+import numpy as np
+import pytest
+
+from mdp_amd import lattice
+from test_gpu_md import RCUTFAC, _coeff, _engine, _oracle_bruteforce
+
+pytestmark = pytest.mark.gpu
+
+
+def _atoms(n, seed):
+    """n atoms of a displaced BCC crystal with vacancies (n = 1: alone in its box)"""
+    cells = max(1, int(np.ceil((n / 2) ** (1 / 3))))
+    x, box = lattice.crystal("bcc", cells, 3.316, 0.1, seed)
+    keep = np.sort(np.random.default_rng(seed).permutation(len(x))[:n])
+    return np.ascontiguousarray(x[keep]), box
+
+
+def test_neighbor_tile_of_256_lanes_identical(oracle, monkeypatch):
+    """The tile kernel on 256 lanes per cell writes the lists of the L1 kernel entry for entry: ragged cells, empty
+    cells, and cells whose surroundings need more than one tile."""
+    rng = np.random.default_rng(6)
+    x1, box1 = lattice.crystal("bcc", 9, 3.316, 0.35, 62)
+    x2 = rng.uniform(0.0, 40.0, size=(400, 3))
+    x3, box3 = lattice.crystal("bcc", 8, 2.75, 0.2, 63)
+    for x, box in ((x1, box1), (x2, np.full(3, 40.0)), (x3, box3)):
+        lists = []
+        for v in ("0", "1", "2"):
+            monkeypatch.setenv("MDP_NB_VARIANT", v)
+            md = _engine(x, box, 4, _coeff(oracle, 4, 1))
+            md.compute()
+            lists.append(md.neighbors())
+            md.close()
+        for other in lists[1:]:
+            for a, b in zip(lists[0], other):
+                assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("cells", [(1, 1, 1), (1, 4, 5), (2, 2, 7), (4, 4, 4)])
+def test_small_box_lists_vs_bruteforce(oracle, cells):
+    """The small-box kernel where images are skipped: flat and long boxes, one cell along an axis."""
+    x, box = lattice.crystal("bcc", cells, 3.316, 0.15, 17)
+    x[0] = 0.0   # on the lower faces
+    md = _engine(x, box, 4, _coeff(oracle, 4, 1))
+    md.compute()
+    off, nj, ns = md.neighbors()
+    o2, j2, s2 = _oracle_bruteforce(oracle, x, box, RCUTFAC + 0.3)
+    for i in range(len(x)):
+        a = sorted(zip(nj[off[i]:off[i + 1]].tolist(), map(tuple, ns[off[i]:off[i + 1]].tolist())))
+        b = sorted(zip(j2[o2[i]:o2[i + 1]].tolist(), map(tuple, s2[o2[i]:o2[i + 1]].tolist())))
+        assert a == b, i
