@@ -23,6 +23,12 @@ YH_DECL(8, 12c)
 YH_DECL(8, 12y)
 YH_DECL(8, 12u1)
 #undef YH_DECL
+void launch_yi_rows_8(const SnapDev&, const double*, const double*, const double*, double*, double*, double*, const int*,
+                      int, hipStream_t);
+void launch_yi_rows_small(const SnapDev&, const double*, const double*, const double*, double*, double*, double*,
+                          const int*, int, hipStream_t);
+
+constexpr int YI_ROWS = 208;   // variant id of k_yi_rows
 
 void yi_row_order(int J, int* out) {
     auto cgn = [](int m, int j1, int j2, int j) {
@@ -51,17 +57,25 @@ void yi_row_order(int J, int* out) {
 int yi_half_variants(int J, int* ids) {
     if (J == 8) {   // waves per workgroup; 112: 12 waves, the larger layer's U rows shared across couplings;
                     // 113: the same with (re, im) adjacent in LDS; 115: 113 with the swap symmetry of the
-                    // (j1, j1) couplings; 116: 115 with the row index made wave-uniform explicitly
-        ids[0] = 8; ids[1] = 12; ids[2] = 4; ids[3] = 112; ids[4] = 113; ids[5] = 115; ids[6] = 116;
-        return 7;
+                    // (j1, j1) couplings; 116: 115 with the row index made wave-uniform explicitly;
+                    // 208: a workgroup per output row (k_yi_rows)
+        ids[0] = 8; ids[1] = 12; ids[2] = 4; ids[3] = 112; ids[4] = 113; ids[5] = 115; ids[6] = 116; ids[7] = YI_ROWS;
+        return 8;
     }
-    ids[0] = 8;
-    return 1;
+    ids[0] = 8; ids[1] = YI_ROWS;
+    return 2;
 }
 
 void launch_yi_half(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
                     double* epart, const int* order, int N, hipStream_t st, int waves) {
     if (N <= 0) return;
+    if (waves == YI_ROWS) {
+        if (s.J == 8)
+            launch_yi_rows_8(s, Ur, Ui, beta_t, Yr, Yi, epart, order, N, st);
+        else
+            launch_yi_rows_small(s, Ur, Ui, beta_t, Yr, Yi, epart, order, N, st);
+        return;
+    }
     switch (s.J) {
         case 2: launch_yi_half_2_8(s, Ur, Ui, beta_t, Yr, Yi, epart, order, N, st); break;
         case 4: launch_yi_half_4_8(s, Ur, Ui, beta_t, Yr, Yi, epart, order, N, st); break;

@@ -147,12 +147,14 @@ __device__ __forceinline__ void z_row_lds(int mb, int malim, const double* __res
 // SYM: a coupling (J1, J1) takes each unordered pair of rows {mb1, mb2} once (the sum is symmetric under
 // the swap of its two U factors): mb1 > mb2 is skipped, mb1 < mb2 counts twice, mb1 = mb2 through
 // z_terms_same_row -- 17% fewer terms at twojmax 8.
-template <int J, int JO, bool CX = false, bool SYM = false, int UNI = 0>
+// PARTS > 1: only the rows (J1, mb1) numbered part, part + PARTS, ... are taken (k_yi_rows).
+template <int J, int JO, bool CX = false, bool SYM = false, int UNI = 0, int PARTS = 1>
 __device__ __forceinline__ void y_couplings_shared_a(int mb, int malim, const double* __restrict__ lr,
                                                      const double* __restrict__ li, int lane,
                                                      const double* __restrict__ cg,
                                                      const double* __restrict__ beta_t, double (&yr)[JO + 1],
-                                                     double (&yi)[JO + 1]) {
+                                                     double (&yi)[JO + 1], int part = 0) {
+    int turn = 0;
     static_for<0, J + 1>([&](auto J1c) {
         constexpr int J1 = decltype(J1c)::value;
         int lo = J1 + 1, hi = -1;   // mb1 range over this layer's couplings
@@ -164,6 +166,11 @@ __device__ __forceinline__ void y_couplings_shared_a(int mb, int malim, const do
             }
         });
         for (int mb1v = lo; mb1v <= hi; ++mb1v) {
+            if constexpr (PARTS > 1) {
+                const bool mine = turn == part;
+                turn = turn + 1 == PARTS ? 0 : turn + 1;
+                if (!mine) continue;
+            }
             // UNI: the row index made wave-uniform explicitly (scalar branches for the row tests below)
             const int mb1 = UNI ? __builtin_amdgcn_readfirstlane(mb1v) : mb1v;
             double ar[J1 + 1], ai[J1 + 1];
@@ -288,6 +295,97 @@ __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ c
                                                       epart);
         });
     }
+}
+
+// compute_yi where 64-atom blocks are too few to fill the chip: one workgroup per (block, output row).  Its W waves
+// split the row's terms by the U rows (J1, mb1) of the larger layer, and the W partial rows are added in LDS in
+// wave order.  k_yi_half keeps a whole output row on one wave and a whole block on one CU, so on a few blocks its
+// time is that of a block (129 us at twojmax 8, 63 us at 6) whatever their number; here n_half_rows times as many
+// CUs work on it, at the price of staging the block's U once per row.  That staging (about 1 us of L2 reads a
+// workgroup) is why k_yi_half stays the better one from some 150 blocks on; the engine times both.
+// Workgroups are dealt to the 8 XCDs round-robin, so workgroup b takes a block of index b mod 8: the rows of one
+// block read its U through one L2.
+template <int J, int W>
+constexpr int yi_rows_lds() {   // doubles: the staged U, or the partial rows and energies that replace it
+    return 2 * n_half_elems(J) * 64 > (2 * (J + 1) + 1) * W * 64 ? 2 * n_half_elems(J) * 64 : (2 * (J + 1) + 1) * W * 64;
+}
+
+template <int J, int W>
+__global__ __launch_bounds__(64 * W) void k_yi_rows(const double* __restrict__ cg, const double* __restrict__ Ur,
+                                                    const double* __restrict__ Ui, const double* __restrict__ beta_t,
+                                                    double* __restrict__ Yr, double* __restrict__ Yi,
+                                                    double* __restrict__ epart, const int* __restrict__ order, int N) {
+    constexpr int HE = n_half_elems(J), NR = n_half_rows(J);
+    __shared__ double lbuf[yi_rows_lds<J, W>()];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = blockIdx.x / 8, block = (q / NR) * 8 + blockIdx.x % 8;
+    if (block * 64 >= N) return;   // uniform over the workgroup
+    const int row = __builtin_amdgcn_readfirstlane(order[q % NR]);
+    const int atom = block * 64 + lane;
+    const bool live = atom < N;
+    const size_t n = static_cast<size_t>(N);
+    double2* const lc = reinterpret_cast<double2*>(lbuf);
+    for (int e = wave; e < HE; e += W)
+        lc[e * 64 + lane] = live ? make_double2(Ur[static_cast<size_t>(e) * n + atom], Ui[static_cast<size_t>(e) * n + atom])
+                                 : make_double2(0.0, 0.0);
+    __syncthreads();
+    const int jo = half_row_j(row), mb = half_row_mb(row);
+    static_for<0, J + 1>([&](auto JOc) {
+        constexpr int JO = decltype(JOc)::value;
+        if (jo == JO) {   // uniform over the workgroup
+            constexpr int PER = (JO + W) / W;   // elements of the row that a wave finishes: ma = wave + W h
+            const int malim = (2 * mb == JO) ? mb : JO;
+            const int hrow = h_block(JO) + (JO + 1) * mb;
+            double yr[JO + 1], yi[JO + 1];
+#pragma unroll
+            for (int m = 0; m <= JO; ++m) { yr[m] = 0.0; yi[m] = 0.0; }
+            y_couplings_shared_a<J, JO, true, true, 1, W>(mb, malim, lbuf, nullptr, lane, cg, beta_t, yr, yi, wave);
+            double2 u[PER];
+#pragma unroll
+            for (int h = 0; h < PER; ++h) u[h] = lc[(hrow + min(wave + W * h, JO)) * 64 + lane];
+            __syncthreads();   // every wave has read what it needs of U
+#pragma unroll
+            for (int m = 0; m <= JO; ++m) lc[(m * W + wave) * 64 + lane] = make_double2(yr[m], yi[m]);
+            __syncthreads();
+            double e = 0.0;
+#pragma unroll
+            for (int h = 0; h < PER; ++h) {
+                const int ma = wave + W * h;
+                if (ma <= malim) {
+                    double2 y = lc[ma * W * 64 + lane];
+#pragma unroll
+                    for (int w = 1; w < W; ++w) {
+                        const double2 p = lc[(ma * W + w) * 64 + lane];
+                        y.x += p.x;
+                        y.y += p.y;
+                    }
+                    if (live) {
+                        Yr[static_cast<size_t>(hrow + ma) * n + atom] = y.x;
+                        Yi[static_cast<size_t>(hrow + ma) * n + atom] = y.y;
+                    }
+                    const double wt = (2 * mb < JO || ma < mb) ? 1.0 : 0.5;
+                    e += wt * (u[h].x * y.x + u[h].y * y.y);
+                }
+            }
+            double* const es = lbuf + 2 * (J + 1) * W * 64;
+            es[wave * 64 + lane] = e;
+            __syncthreads();
+            if (wave == 0 && live) {
+                double sum = es[lane];
+#pragma unroll
+                for (int w = 1; w < W; ++w) sum += es[w * 64 + lane];
+                epart[static_cast<size_t>(row) * n + atom] = sum;
+            }
+        }
+    });
+}
+
+template <int J, int W>
+void launch_yi_rows(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
+                    double* epart, const int* order, int N, hipStream_t st) {
+    const int blocks = ((N + 63) / 64 + 7) / 8 * 8;   // whole XCD rounds; workgroups past the last block return
+    hipLaunchKernelGGL((k_yi_rows<J, W>), dim3(blocks * n_half_rows(J)), dim3(64 * W), 0, st, s.cg, Ur, Ui, beta_t, Yr, Yi,
+                       epart, order, N);
 }
 
 // B of every bispectrum triple (j >= j1) from the half U of 64 atoms staged in LDS, as k_yi_half stages

@@ -972,6 +972,9 @@ struct mdp_md {
             }
         }
         nrows = n_half_rows(J);
+        // until (or without) the autotuner: a workgroup per output row where a workgroup per 64 atoms would leave
+        // most CUs idle (it loses from some 150 blocks on)
+        yi_waves = N <= 64 * 128 ? 208 : 8;
         massinv_h.assign(ntypes + 1, 0.0);
         for (int t = 1; t <= ntypes; ++t) massinv_h[t] = 1.0 / p->mass[t - 1];
         rc2_h.assign((ntypes + 1) * (ntypes + 1), 0.0);

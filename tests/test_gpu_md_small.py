@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from mdp_amd import lattice
-from test_gpu_md import RCUTFAC, _coeff, _engine, _oracle_bruteforce
+from test_gpu_md import RCUTFAC, _coeff, _engine, _first_step_vs_oracle, _oracle_bruteforce
 
 pytestmark = pytest.mark.gpu
 
@@ -19,6 +19,16 @@ def _atoms(n, seed):
     x, box = lattice.crystal("bcc", cells, 3.316, 0.1, seed)
     keep = np.sort(np.random.default_rng(seed).permutation(len(x))[:n])
     return np.ascontiguousarray(x[keep]), box
+
+
+@pytest.mark.parametrize("n", [1, 63, 65])
+@pytest.mark.parametrize("J", [2, 4, 6, 8])
+def test_yi_row_workgroups_vs_oracle(oracle, monkeypatch, J, n):
+    """compute_yi with a workgroup per output row (variant 208)."""
+    monkeypatch.setenv("MDP_YI_VARIANT", "208")
+    x, box = _atoms(n, 7 + n + J)
+    md = _first_step_vs_oracle(oracle, x, box, J, 3)
+    assert md.tuning()["chosen"]["compute_yi_waves"] == 208
 
 
 def test_neighbor_tile_of_256_lanes_identical(oracle, monkeypatch):
