@@ -39,6 +39,9 @@ struct mdp_fit {
     std::vector<int> a0_h;   // [C+1]
     std::vector<double> boxes_h, tilts_h;   // tilts_h empty: every cell orthogonal
     DevBuf x, type, cfg_of, cfg_a0, cfg_L, cfg_T, cfg_p0, rc2, pcnt, poff, scan_tmp, flags, counter;
+    std::vector<int> cfg_ord_h;
+    int n_large = 0;    // how many of them the tallies treat as large (lsq_large_configuration)
+    DevBuf cfg_ord;     // configurations, most atoms first
     DevBuf chunk_ord;   // 64-atom chunks of the pair build, most candidate tests first
     DevBuf pi, pj, pti, ptj, rij, Ur, Ui, zt, blist, bpart, dblist, bzero, t_lo, t_b, t_z, t_w, zorder, t_wtab, t_hlo, t_hb, t_hz,
         t_hw, t_mz, t_mw, t_mcomb, pgeo;
@@ -176,6 +179,15 @@ struct mdp_fit {
             for (int k = 0; k < nch; ++k) ord[k] = k;
             std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return cost[a] > cost[b]; });
             put(chunk_ord, ord.data(), sizeof(int) * std::max(nch, 1));
+        }
+        cfg_ord_h.resize(C);
+        for (int c = 0; c < C; ++c) cfg_ord_h[c] = c;
+        std::stable_sort(cfg_ord_h.begin(), cfg_ord_h.end(),
+                         [&](int a, int b) { return a0_h[a + 1] - a0_h[a] > a0_h[b + 1] - a0_h[b]; });
+        put(cfg_ord, cfg_ord_h.data(), sizeof(int) * C);
+        for (n_large = 0; n_large < C; ++n_large) {
+            const int c = cfg_ord_h[n_large];
+            if (a0_h[c + 1] - a0_h[c] <= lsq_large_configuration()) break;
         }
         put(bzero, bz.data(), sizeof(double) * bz.size());
         put(t_lo, lo.data(), sizeof(int) * lo.size());
@@ -494,7 +506,7 @@ struct mdp_fit {
                             scan_tmp.as<int>(), st);
         launch_lsq_tallies(blist.as<double>(), dblist.as<double>(), rij.as<double>(), poff.as<int>(), l_off.as<int>(),
                            l_idx.as<int>(), pti.as<int>(), type.as<int>(), cfg_of.as<int>(), cfg_a0.as<int>(),
-                           cfg_p0.as<int>(), C, N, IB, ntypes, max_natoms(), l_bi.as<double>(), l_bd.as<double>(),
+                           cfg_p0.as<int>(), cfg_ord.as<int>(), n_large, C, N, IB, ntypes, max_natoms(), l_bi.as<double>(), l_bd.as<double>(),
                            l_bv.as<double>(), l_as.as<double>(), st);
         MDP_HIP(hipGetLastError());
     }
@@ -508,19 +520,8 @@ struct mdp_fit {
                     const double* ws, int normalizeenergy, double* L, double* hv) {
         lsq_tallies();
         const int K = ntypes * tab.idx.idxb_max;
-        if (lsq_gram_lds(K) > 65536) throw Error("mdp_fit_normal_equations: too many descriptor columns");
+        if (K > lsq_gram_max_columns()) throw Error("mdp_fit_normal_equations: too many descriptor columns");
         const int ntri = K * (K + 1) / 2, nout = ntri + K, G = 1024;
-        if (l_ekl_k != K) {
-            std::vector<int2> ekl(nout);
-            int e0 = 0;
-            for (int k = 0; k < K; ++k)
-                for (int l = k; l < K; ++l) ekl[e0++] = make_int2(k, l);
-            for (int k = 0; k < K; ++k) ekl[ntri + k] = make_int2(k, -1);
-            l_ekl.ensure(sizeof(int2) * nout);
-            MDP_HIP(hipMemcpyAsync(l_ekl.p, ekl.data(), sizeof(int2) * nout, hipMemcpyHostToDevice, st));
-            MDP_HIP(hipStreamSynchronize(st));
-            l_ekl_k = K;
-        }
         l_part.ensure(sizeof(double) * static_cast<size_t>(G) * nout);
         l_out.ensure(sizeof(double) * nout);
         std::fill(L, L + 3 * static_cast<size_t>(K) * K, 0.0);
@@ -535,7 +536,7 @@ struct mdp_fit {
             MDP_HIP(hipMemcpyAsync(l_T.p, T, sizeof(double) * nT, hipMemcpyHostToDevice, st));
             MDP_HIP(hipMemcpyAsync(l_W.p, W.data(), sizeof(double) * W.size(), hipMemcpyHostToDevice, st));
             launch_lsq_gram(l_chunks.as<LsqChunk>(), static_cast<int>(ch.size()), A, l_T.as<double>(), l_W.as<double>(),
-                            K, l_ekl.as<int2>(), l_part.as<double>(), G, l_out.as<double>(), st);
+                            K, l_part.as<double>(), G, l_out.as<double>(), st);
             std::vector<double> o(nout);
             MDP_HIP(hipMemcpyAsync(o.data(), l_out.p, sizeof(double) * nout, hipMemcpyDeviceToHost, st));
             MDP_HIP(hipStreamSynchronize(st));

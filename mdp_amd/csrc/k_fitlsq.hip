@@ -39,19 +39,37 @@ __global__ void k_lsq_in_fill(const int* __restrict__ pj, long P, const int* __r
     in_idx[in_off[a] + atomicAdd(cursor + a, 1)] = static_cast<int>(p);
 }
 
-// the fill order depends on scheduling: sort each atom's short list
-__global__ void k_lsq_in_sort(const int* __restrict__ in_off, int* __restrict__ in_idx, int N) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= N) return;
-    const int lo = in_off[a], hi = in_off[a + 1];
-    for (int i = lo + 1; i < hi; ++i) {
-        const int v = in_idx[i];
-        int k = i - 1;
-        while (k >= lo && in_idx[k] > v) {
-            in_idx[k + 1] = in_idx[k];
-            --k;
+// The fill order depends on scheduling: each atom's list is put in ascending order, 16 lanes per atom ranking its
+// entries from an LDS copy (105,000 atoms of 20 pairs: 13 us; 99 us with one lane per atom sorting by insertion).  A list
+// longer than the copy is sorted in place by one lane.
+constexpr int SORT_SUB = 16, SORT_MAX = 128;
+
+__global__ __launch_bounds__(256) void k_lsq_in_sort(const int* __restrict__ in_off, int* __restrict__ in_idx, int N) {
+    __shared__ int list[256 / SORT_SUB][SORT_MAX];
+    const int t = blockIdx.x * 256 + threadIdx.x, a = t / SORT_SUB, sub = t % SORT_SUB;
+    const int lo = a < N ? in_off[a] : 0, n = a < N ? in_off[a + 1] - lo : 0;
+    int* l = list[threadIdx.x / SORT_SUB];
+    int* __restrict__ x = in_idx + lo;
+    if (n <= SORT_MAX)
+        for (int k = sub; k < n; k += SORT_SUB) l[k] = x[k];
+    __syncthreads();
+    if (n <= SORT_MAX) {
+        for (int k = sub; k < n; k += SORT_SUB) {
+            const int v = l[k];
+            int rank = 0;
+            for (int m = 0; m < n; ++m) rank += l[m] < v;
+            x[rank] = v;
         }
-        in_idx[k + 1] = v;
+    } else if (sub == 0) {
+        for (int i = 1; i < n; ++i) {
+            const int v = x[i];
+            int k = i - 1;
+            while (k >= 0 && x[k] > v) {
+                x[k + 1] = x[k];
+                --k;
+            }
+            x[k + 1] = v;
+        }
     }
 }
 
@@ -63,7 +81,8 @@ void launch_lsq_incoming(const int* pj, long P, int N, int* in_cnt, int* in_off,
     if (P > 0) hipLaunchKernelGGL(k_lsq_in_count, dim3(nblocks(P, 256)), dim3(256), 0, st, pj, P, in_cnt);
     exclusive_scan(in_cnt, in_off, N, scan_tmp, st);
     if (P > 0) hipLaunchKernelGGL(k_lsq_in_fill, dim3(nblocks(P, 256)), dim3(256), 0, st, pj, P, in_off, cursor, in_idx);
-    hipLaunchKernelGGL(k_lsq_in_sort, dim3(nblocks(N, 128)), dim3(128), 0, st, in_off, in_idx, N);
+    hipLaunchKernelGGL(k_lsq_in_sort, dim3(nblocks(static_cast<long>(N) * SORT_SUB, 256)), dim3(256), 0, st, in_off,
+                       in_idx, N);
 }
 
 // ---- tallies ------------------------------------------------------------------------------------
@@ -108,53 +127,110 @@ __global__ void k_lsq_bd(const double* __restrict__ dblist, const int* __restric
     }
 }
 
-// The same tally for one element type, one block per (configuration, comp + 3 k): the block streams
-// that plane of dB/dr (pair-contiguous) through LDS in tiles of LSQ_TILE pairs with coalesced loads, and
-// each atom adds its own pairs and subtracts its incoming ones (both ascending) into an LDS accumulator
-// only it touches.  Every dB/dr value is read from HBM once.  LDS: LSQ_TILE + N_c doubles, N_c ints;
-// 1024 threads per block keep the CU busy although only two such blocks fit in its LDS.
-constexpr int LSQ_TILE = 4096;
-__global__ __launch_bounds__(1024) void k_lsq_bd_tiled(const double* __restrict__ dblist, const int* __restrict__ poff,
-                                                      const int* __restrict__ in_off, const int* __restrict__ in_idx,
-                                                      const int* __restrict__ cfg_a0, const int* __restrict__ cfg_p0,
-                                                      int IB, double* __restrict__ bd) {
-    extern __shared__ double sm[];
-    const int c = blockIdx.x / (3 * IB), plane = blockIdx.x % (3 * IB);
-    const int comp = plane % 3, k = plane / 3;
-    const int a0 = cfg_a0[c], nc = cfg_a0[c + 1] - a0, p0 = cfg_p0[c];
-    const int pc = cfg_p0[c + 1] - p0;
-    double* tile = sm;
-    double* acc = sm + LSQ_TILE;
-    int* cur = reinterpret_cast<int*>(acc + nc);
-    const double* __restrict__ db = dblist + static_cast<size_t>(p0) * 3 * IB + static_cast<size_t>(pc) * (comp + 3 * k);
-    for (int a = threadIdx.x; a < nc; a += 1024) {
-        acc[a] = 0.0;
-        cur[a] = in_off[a0 + a];
+// The tallies of dB/dr for one element type: bd (as above) and the virial v = -r (x) dB/dr in one pass over dB/dr.
+// Bound: that one read (24 IB bytes per pair).  One workgroup per (configuration, k): it streams the three planes
+// of k through LDS in tiles of BD_TILE pairs, adds each pair's virial on the way, and then every atom adds its own
+// pairs of the tile and subtracts its incoming ones (both ascending), in registers of the thread that owns it: up to
+// H atoms per thread.  The indices of an atom's next two incoming pairs are kept loaded: a tile without one costs no
+// memory access, and one load's latency passes behind the other's pair.  Configurations come largest first (cfg_ord),
+// those of more than BD_TH atoms in a launch of their own.  105,000 atoms, 2.1 M pairs, twojmax 8:
+// 1,312 us (2.1 TB/s); a pass per plane for bd and a second read of dB/dr for the virial took 1,841 + 813 us.
+// bv[c*6*Kt + 6*k + m], components m = (xx, yy, zz, xy, xz, yz); as[(6c + m')*Kt + k] are the same as the stress rows of
+// the fit, in the upstream row order m' -> m = (0, 1, 2, 5, 4, 3) (snapcpp.jl:660-662).
+constexpr int BD_TILE = 1280, BD_TH = 512, BD_MAXH = 4;
+
+template <int H>
+__global__ __launch_bounds__(BD_TH) void k_lsq_bd_bv(const double* __restrict__ dblist, const double* __restrict__ rij,
+                                                     const int* __restrict__ poff, const int* __restrict__ in_off,
+                                                     const int* __restrict__ in_idx, const int* __restrict__ cfg_a0,
+                                                     const int* __restrict__ cfg_p0, const int* __restrict__ cfg_ord,
+                                                     int IB, double* __restrict__ bd, double* __restrict__ bv,
+                                                     double* __restrict__ as) {
+    __shared__ double tile[3][BD_TILE];
+    __shared__ double red[BD_TH / 64][6];
+    const int c = cfg_ord[blockIdx.x / IB], k = blockIdx.x % IB, t = threadIdx.x;
+    const int a0 = cfg_a0[c], nc = cfg_a0[c + 1] - a0, p0 = cfg_p0[c], pc = cfg_p0[c + 1] - p0;
+    const double* __restrict__ db = dblist + static_cast<size_t>(p0) * 3 * IB + 3 * static_cast<size_t>(pc) * k;
+    const double* __restrict__ r = rij + 3 * static_cast<size_t>(p0);
+    double s[H][3], v[6] = {0, 0, 0, 0, 0, 0};
+    int q0[H], q1[H], m[H], mend[H], next[H], after[H];   // own pairs; incoming list position and end, next two pairs
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        const int a = t + h * BD_TH;
+        const bool live = a < nc;
+        s[h][0] = s[h][1] = s[h][2] = 0.0;
+        q0[h] = live ? poff[a0 + a] - p0 : 0;
+        q1[h] = live ? poff[a0 + a + 1] - p0 : 0;
+        m[h] = live ? in_off[a0 + a] : 0;
+        mend[h] = live ? in_off[a0 + a + 1] : 0;
+        next[h] = m[h] < mend[h] ? in_idx[m[h]] - p0 : pc;
+        after[h] = m[h] + 1 < mend[h] ? in_idx[m[h] + 1] - p0 : pc;
     }
-    for (int t0 = 0; t0 < pc; t0 += LSQ_TILE) {
-        const int t1 = min(pc, t0 + LSQ_TILE);
+    for (int t0 = 0; t0 < pc; t0 += BD_TILE) {
+        const int t1 = min(pc, t0 + BD_TILE);
+        __syncthreads();   // the previous tile's readers are done
+        for (int q = t0 + t; q < t1; q += BD_TH) {
+            const double bx = db[q], by = db[q + static_cast<size_t>(pc)], bz = db[q + 2 * static_cast<size_t>(pc)];
+            const double dx = -r[3 * q], dy = -r[3 * q + 1], dz = -r[3 * q + 2];
+            tile[0][q - t0] = bx;
+            tile[1][q - t0] = by;
+            tile[2][q - t0] = bz;
+            v[0] += dx * bx;
+            v[1] += dy * by;
+            v[2] += dz * bz;
+            v[3] += dx * by;
+            v[4] += dx * bz;
+            v[5] += dy * bz;
+        }
         __syncthreads();
-        for (int i = threadIdx.x; i < t1 - t0; i += 1024) tile[i] = db[t0 + i];
-        __syncthreads();
-        for (int a = threadIdx.x; a < nc; a += 1024) {
-            const int g = a0 + a;
-            double s = acc[a];
-            const int q0 = max(poff[g] - p0, t0), q1 = min(poff[g + 1] - p0, t1);
-            for (int q = q0; q < q1; ++q) s += tile[q - t0];
-            int m = cur[a];
-            const int mend = in_off[g + 1];
-            for (; m < mend; ++m) {
-                const int q = in_idx[m] - p0;
-                if (q >= t1) break;
-                s -= tile[q - t0];
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const int lo = max(q0[h], t0) - t0, hi = min(q1[h], t1) - t0;
+#pragma unroll 4
+            for (int q = lo; q < hi; ++q) {
+                s[h][0] += tile[0][q];
+                s[h][1] += tile[1][q];
+                s[h][2] += tile[2][q];
             }
-            cur[a] = m;
-            acc[a] = s;
+            while (next[h] < t1) {
+                const int q = next[h] - t0;
+                ++m[h];
+                next[h] = after[h];
+                after[h] = m[h] + 1 < mend[h] ? in_idx[m[h] + 1] - p0 : pc;
+                s[h][0] -= tile[0][q];
+                s[h][1] -= tile[1][q];
+                s[h][2] -= tile[2][q];
+            }
         }
     }
+    double* __restrict__ out = bd + 3 * static_cast<size_t>(a0) * IB + 3 * static_cast<size_t>(nc) * k;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        const int a = t + h * BD_TH;
+        if (a < nc) {
+            out[3 * a] = s[h][0];
+            out[3 * a + 1] = s[h][1];
+            out[3 * a + 2] = s[h][2];
+        }
+    }
+#pragma unroll
+    for (int w = 32; w >= 1; w /= 2)
+#pragma unroll
+        for (int i = 0; i < 6; ++i) v[i] += __shfl_xor(v[i], w);
+    if ((t & 63) == 0)
+#pragma unroll
+        for (int i = 0; i < 6; ++i) red[t >> 6][i] = v[i];
     __syncthreads();
-    for (int a = threadIdx.x; a < nc; a += 1024)
-        bd[3 * static_cast<size_t>(a0) * IB + comp + 3 * a + 3 * static_cast<size_t>(nc) * k] = acc[a];
+    if (t < 6) {
+        constexpr int ord[6] = {0, 1, 2, 5, 4, 3};
+        double raw = 0.0, row = 0.0;
+        for (int w = 0; w < BD_TH / 64; ++w) {
+            raw += red[w][t];
+            row += red[w][ord[t]];
+        }
+        bv[static_cast<size_t>(c) * 6 * IB + 6 * k + t] = raw;
+        as[(static_cast<size_t>(c) * 6 + t) * IB + k] = row;
+    }
 }
 
 // bi[c*Kt + col] = sum of B_k over the atoms of type t of configuration c: one block per (c, col), its
@@ -180,7 +256,8 @@ __global__ __launch_bounds__(256) void k_lsq_bi(const double* __restrict__ blist
     if (threadIdx.x == 0) bi[blockIdx.x] = red[0];
 }
 
-// virial tally of configuration c and column col (one block): v = -r (x) dB/dr summed over the pairs
+// virial tally of configuration c and column col (one block; several element types, or configurations too large for
+// k_lsq_bd_bv): v = -r (x) dB/dr summed over the pairs
 // whose owner has the column's type, components (xx, yy, zz, xy, xz, yz) as upstream; written raw,
 // bv[c*6*Kt + 6*col + m], and as the stress rows of the fit, as[(6c + m')*Kt + col] with the upstream
 // row order m' -> m = (0, 1, 2, 5, 4, 3) (snapcpp.jl:660-662).  Fixed-order tree reduction.
@@ -226,82 +303,145 @@ __global__ __launch_bounds__(256) void k_lsq_bv(const double* __restrict__ dblis
 
 void launch_lsq_tallies(const double* blist, const double* dblist, const double* rij, const int* poff,
                         const int* in_off, const int* in_idx, const int* pti, const int* type, const int* cfg_of,
-                        const int* cfg_a0, const int* cfg_p0, int C, int N, int IB, int ntypes, int max_natoms,
-                        double* bi, double* bd, double* bv, double* as, hipStream_t st) {
+                        const int* cfg_a0, const int* cfg_p0, const int* cfg_ord, int n_large, int C, int N, int IB,
+                        int ntypes, int max_natoms, double* bi, double* bd, double* bv, double* as, hipStream_t st) {
     const int kt = ntypes * IB;
-    const size_t lds = sizeof(double) * (LSQ_TILE + static_cast<size_t>(max_natoms)) + sizeof(int) * max_natoms;
-    if (ntypes == 1 && lds <= 65536)
-        hipLaunchKernelGGL(k_lsq_bd_tiled, dim3(static_cast<unsigned>(C) * 3 * IB), dim3(1024), lds, st, dblist, poff,
-                           in_off, in_idx, cfg_a0, cfg_p0, IB, bd);
-    else
+    // one element type and at most BD_MAXH atoms per thread: one read of dB/dr for both tallies
+    const int per_thread = (max_natoms + BD_TH - 1) / BD_TH;
+    const bool fused = ntypes == 1 && per_thread <= BD_MAXH;
+    if (fused) {
+        if (n_large > 0)
+            hipLaunchKernelGGL(k_lsq_bd_bv<BD_MAXH>, dim3(static_cast<unsigned>(n_large) * IB), dim3(BD_TH), 0, st, dblist,
+                               rij, poff, in_off, in_idx, cfg_a0, cfg_p0, cfg_ord, IB, bd, bv, as);
+        if (n_large < C)
+            hipLaunchKernelGGL(k_lsq_bd_bv<1>, dim3(static_cast<unsigned>(C - n_large) * IB), dim3(BD_TH), 0, st, dblist,
+                               rij, poff, in_off, in_idx, cfg_a0, cfg_p0, cfg_ord + n_large, IB, bd, bv, as);
+    } else {
         hipLaunchKernelGGL(k_lsq_bd, dim3(nblocks(static_cast<long>(N) * IB, 256)), dim3(256), 0, st, dblist, poff,
                            in_off, in_idx, pti, type, cfg_of, cfg_a0, cfg_p0, N, IB, ntypes, bd);
+    }
     hipLaunchKernelGGL(k_lsq_bi, dim3(static_cast<unsigned>(C) * kt), dim3(256), 0, st, blist, type, cfg_a0, IB, ntypes,
                        bi);
-    hipLaunchKernelGGL(k_lsq_bv, dim3(static_cast<unsigned>(C) * kt), dim3(256), 0, st, dblist, rij, pti, cfg_p0, IB,
-                       ntypes, bv, as);
+    if (!fused)
+        hipLaunchKernelGGL(k_lsq_bv, dim3(static_cast<unsigned>(C) * kt), dim3(256), 0, st, dblist, rij, pti, cfg_p0, IB,
+                           ntypes, bv, as);
 }
 
 // ---- weighted normal equations --------------------------------------------------------------------
 
-// Chunk ch covers rows r < nrows: a(r, k) = A[abase + r*rs + k*cs], target T[tbase + r], weight
-// W[wbase + r / wdiv].  Outputs e < K(K+1)/2 are L(k, l), k <= l (row-major upper triangle), then
-// K entries of h.  Block b takes chunks b, b + G, ... and writes its partial sums to part[b]; each
-// thread owns a fixed set of outputs, accumulated in LDS.
+// Chunk ch covers rows r < nrows <= 64: a(r, k) = A[abase + r*rs + k*cs], target T[tbase + r], weight
+// W[wbase + r / wdiv].  Outputs e < K(K+1)/2 are L(k, l), k <= l (row-major upper triangle), then K entries of h.
+//
+// The sum over rows of w^2 [a | b]^T [a | b] on the FP64 matrix cores: the K + 1 columns of a chunk are staged column
+// by column in LDS (row length 66: the operand reads of a half wave cover all banks), and each wave owns every
+// fourth of the upper 16 x 16 tiles, one v_mfma_f64_16x16x4 per tile and four rows (operands A[m][k], B[k][n] at lanes
+// m + 16k, n + 16k; the accumulator's register i of lane (m, g) is row 4i + g, column m).  Workgroup b takes chunks b,
+// b + G, ... in order and writes its partial sums to part[b].  Bound: one read of the rows; the three groups of a batch
+// with 315,000 force rows of 55 columns take 100 us, 430 us with one output per thread.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int GR_LD = 66, GR_MAXT = 5;   // at most 5 x 16 columns (K <= 79)
+
+template <int NT>
 __global__ __launch_bounds__(256) void k_lsq_gram(const LsqChunk* __restrict__ chunks, int nchunks,
                                                   const double* __restrict__ A, const double* __restrict__ T,
-                                                  const double* __restrict__ W, int K,
-                                                  const int2* __restrict__ ekl, double* __restrict__ part) {
-    extern __shared__ double sm[];
+                                                  const double* __restrict__ W, int K, double* __restrict__ part) {
+    constexpr int TILES = NT * (NT + 1) / 2, PER = (TILES + 3) / 4;
+    __shared__ double tile[NT * 16 * GR_LD];
+    __shared__ double w2[64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m16 = lane & 15, g4 = lane >> 4;
     const int nout = K * (K + 1) / 2 + K;
-    double* acc = sm;                        // nout
-    double* tile = sm + nout;                // 64 * (K + 1): a(r, k) at r*(K+1) + k, w^2 b at r*(K+1) + K
-    double* w2 = tile + 64 * (K + 1);        // 64
-    for (int e = threadIdx.x; e < nout; e += 256) acc[e] = 0.0;
+    int ti[PER], tj[PER];   // this wave's tiles, (row, column) of the upper triangle in row-major order
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        int id = min(wave + 4 * u, TILES - 1), i = 0;
+        while (id >= NT - i) id -= NT - i++;
+        ti[u] = i;
+        tj[u] = i + id;
+    }
+    f64x4 acc[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) acc[u] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < NT * 16 * GR_LD; i += 256) tile[i] = 0.0;   // the columns past K stay zero
     for (int ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
         const LsqChunk q = chunks[ch];
         __syncthreads();
-        for (int i = threadIdx.x; i < q.nrows * K; i += 256) {
-            const int k = i / q.nrows, r = i % q.nrows;   // rows fastest: contiguous reads when rs == 1
-            tile[r * (K + 1) + k] = A[q.abase + static_cast<long>(r) * q.rs + static_cast<long>(k) * q.cs];
+        for (int i = threadIdx.x; i < 64 * K; i += 256) {   // rows fastest: contiguous reads when rs == 1
+            const int k = i / 64, r = i % 64;
+            tile[k * GR_LD + r] =
+                r < q.nrows ? A[q.abase + static_cast<long>(r) * q.rs + static_cast<long>(k) * q.cs] : 0.0;
         }
-        for (int r = threadIdx.x; r < q.nrows; r += 256) {
-            const double w = W[q.wbase + r / q.wdiv];
+        if (threadIdx.x < 64) {
+            const int r = threadIdx.x;
+            const double w = r < q.nrows ? W[q.wbase + r / q.wdiv] : 0.0;
             w2[r] = w * w;
-            tile[r * (K + 1) + K] = w * w * T[q.tbase + r];
+            tile[K * GR_LD + r] = r < q.nrows ? T[q.tbase + r] : 0.0;
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < nout; e += 256) {
-            const int2 kl = ekl[e];
-            double s = 0.0;
-            if (kl.y >= 0) {
-                for (int r = 0; r < q.nrows; ++r) s += w2[r] * tile[r * (K + 1) + kl.x] * tile[r * (K + 1) + kl.y];
-            } else {
-                for (int r = 0; r < q.nrows; ++r) s += tile[r * (K + 1) + kl.x] * tile[r * (K + 1) + K];
+#pragma unroll 4
+        for (int st = 0; st < 16; ++st) {
+            const int r = 4 * st + g4;
+            const double w = w2[r];
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const double a = w * tile[(16 * ti[u] + m16) * GR_LD + r];
+                const double b = tile[(16 * tj[u] + m16) * GR_LD + r];
+                acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[u], 0, 0, 0);
             }
-            acc[e] += s;
         }
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < nout; e += 256) part[static_cast<size_t>(blockIdx.x) * nout + e] = acc[e];
+    double* __restrict__ o = part + static_cast<size_t>(blockIdx.x) * nout;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (wave + 4 * u >= TILES) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = 16 * ti[u] + 4 * i + g4, l = 16 * tj[u] + m16;
+            if (k < K && l == K) o[K * (K + 1) / 2 + k] = acc[u][i];
+            if (k <= l && l < K) o[k * K - k * (k - 1) / 2 + l - k] = acc[u][i];
+        }
+    }
 }
 
-// out[e] = sum over blocks b = 0..G-1 of part[b][e], in block order
-__global__ void k_lsq_gram_sum(const double* __restrict__ part, int G, int nout, double* __restrict__ out) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nout) return;
+// out[e] = sum over b = 0..G-1 of part[b][e]: 64 outputs per workgroup, wave w adds partials w, w + 16, ... and the 16
+// sums are added in wave order (1,024 partials: 7 us; 245 us when one lane added a whole output)
+__global__ __launch_bounds__(1024) void k_lsq_gram_sum(const double* __restrict__ part, int G, int nout,
+                                                       double* __restrict__ out) {
+    __shared__ double sum[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, e = blockIdx.x * 64 + lane;
     double s = 0.0;
-    for (int b = 0; b < G; ++b) s += part[static_cast<size_t>(b) * nout + e];
+    if (e < nout) {
+#pragma unroll 8
+        for (int b = w; b < G; b += 16) s += part[static_cast<size_t>(b) * nout + e];
+    }
+    sum[w][lane] = s;
+    __syncthreads();
+    if (w != 0 || e >= nout) return;
+    s = sum[0][lane];
+#pragma unroll
+    for (int k = 1; k < 16; ++k) s += sum[k][lane];
     out[e] = s;
 }
 
-size_t lsq_gram_lds(int K) { return sizeof(double) * (K * (K + 1) / 2 + K + 64 * (K + 1) + 64); }
+int lsq_large_configuration() { return BD_TH; }
+
+int lsq_gram_max_columns() { return 77; }
 
 void launch_lsq_gram(const LsqChunk* chunks, int nchunks, const double* A, const double* T, const double* W, int K,
-                     const int2* ekl, double* part, int G, double* out, hipStream_t st) {
-    const int nout = K * (K + 1) / 2 + K;
-    hipLaunchKernelGGL(k_lsq_gram, dim3(G), dim3(256), lsq_gram_lds(K), st, chunks, nchunks, A, T, W, K, ekl, part);
-    hipLaunchKernelGGL(k_lsq_gram_sum, dim3(nblocks(nout, 256)), dim3(256), 0, st, part, G, nout, out);
+                     double* part, int G, double* out, hipStream_t st) {
+    const int nout = K * (K + 1) / 2 + K, NT = (K + 1 + 15) / 16;
+    static_assert(GR_MAXT * 16 >= 78, "the columns and the target fit the tiles");
+    G = G < nchunks ? G : nchunks;
+    switch (NT) {
+#define GRAM(NTV)                                                                                                       case NTV:                                                                                                               hipLaunchKernelGGL(k_lsq_gram<NTV>, dim3(G), dim3(256), 0, st, chunks, nchunks, A, T, W, K, part);                   break;
+        GRAM(1)
+        GRAM(2)
+        GRAM(3)
+        GRAM(4)
+        GRAM(5)
+#undef GRAM
+        default: return;
+    }
+    hipLaunchKernelGGL(k_lsq_gram_sum, dim3(nblocks(nout, 64)), dim3(1024), 0, st, part, G, nout, out);
 }
 
 }  // namespace mdp
