@@ -15,15 +15,41 @@ namespace mdp {
 
 bool templated_j(int J) { return J == 2 || J == 4 || J == 6 || J == 8; }
 
+// Sum over the SUB adjacent lanes that share an atom, by DPP within a row of 16 lanes; every lane gets the same sum
+// (quad permutes swap neighbours 1 and 2 apart; the half-row and row mirrors then pair quads and octets).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
+    return v + __hiloint2double(hi, lo);
+}
+template <int SUB>
+__device__ __forceinline__ double sub_sum(double v) {
+    static_assert(SUB == 1 || SUB == 4 || SUB == 16, "lanes per atom");
+    if constexpr (SUB >= 4) {
+        v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+        v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    }
+    if constexpr (SUB >= 16) {
+        v = dpp_add<0x141>(v);   // row_half_mirror
+        v = dpp_add<0x140>(v);   // row_mirror
+    }
+    return v;
+}
+
 // GEO: the pair's Cayley-Klein parameters and weighted switching factor come precomputed from
 // pgeo[5q..5q+4] = (a_r, a_i, b_r, b_i, sfac * w_j) (the MD pair list writes them once per step with the
 // same pair_geometry), instead of being derived here from r_ij in every row group.
-template <int J, int RLO, int RHI, int MODE, bool GEO = false>
+// SUB > 1 (with GEO, UI_HALF_WSELF): SUB adjacent lanes share an atom and take every SUB-th of its pairs, so that a
+// small system puts SUB times as many waves on the chip and each walks a SUB-th of the serial chain of pairs; the
+// partial sums are added across the lanes at the end and lane k % SUB stores element k.
+template <int J, int RLO, int RHI, int MODE, bool GEO = false, int SUB = 1>
 __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ Ur, double* __restrict__ Ui,
                                         const double* __restrict__ rij, const int* __restrict__ pair_off,
                                         const int* __restrict__ perm, const int* __restrict__ ti,
                                         const int* __restrict__ tj, int N, double wself, int elem_sel, int atom,
-                                        const double* __restrict__ pgeo = nullptr) {
+                                        const double* __restrict__ pgeo = nullptr, int sub = 0) {
+    static_assert(SUB == 1 || (GEO && MODE == UI_HALF_WSELF), "lanes share an atom in the MD and fitting form only");
     constexpr int NE = rows_elems(J, RLO, RHI);
     double accr[NE], acci[NE];
 #pragma unroll
@@ -41,22 +67,22 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
     };
 
     // the next pair's data are loaded while the current pair's recursion runs
-    const int q0 = pair_off[atom], q1 = pair_off[atom + 1];
+    const int q0 = SUB == 1 || atom < N ? pair_off[atom] : 0, q1 = SUB == 1 || atom < N ? pair_off[atom + 1] : 0;
     if constexpr (GEO) {
         double n[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (q0 < q1)
+        if (q0 + sub < q1)
 #pragma unroll
-            for (int k = 0; k < 5; ++k) n[k] = pgeo[5 * static_cast<size_t>(q0) + k];
-        for (int q = q0; q < q1; ++q) {
+            for (int k = 0; k < 5; ++k) n[k] = pgeo[5 * static_cast<size_t>(q0 + sub) + k];
+        for (int q = q0 + sub; q < q1; q += SUB) {
             PairGeom g;
             g.ar = n[0];
             g.ai = n[1];
             g.br = n[2];
             g.bi = n[3];
             const double sf = n[4];
-            if (q + 1 < q1)
+            if (q + SUB < q1)
 #pragma unroll
-                for (int k = 0; k < 5; ++k) n[k] = pgeo[5 * static_cast<size_t>(q + 1) + k];
+                for (int k = 0; k < 5; ++k) n[k] = pgeo[5 * static_cast<size_t>(q + SUB) + k];
             accumulate(g, sf);
         }
     } else {
@@ -83,6 +109,14 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
         }
     }
 
+    if constexpr (SUB > 1) {
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+            accr[k] = sub_sum<SUB>(accr[k]);
+            acci[k] = sub_sum<SUB>(acci[k]);
+        }
+        if (atom >= N) return;   // lanes past the last atom took part in no other atom's sum
+    }
     const size_t n = static_cast<size_t>(N);
     static_for<RLO, RHI + 1>([&](auto MBc) {
         constexpr int MB = decltype(MBc)::value;
@@ -97,6 +131,7 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
                     Ur[o] += accr[base + ma];
                     Ui[o] += acci[base + ma];
                 } else if constexpr (MODE == UI_HALF_WSELF) {
+                    if (SUB > 1 && sub != (base + ma) % SUB) continue;
                     const size_t oh = static_cast<size_t>(h_block(JJ) + (JJ + 1) * MB + ma) * n + atom;
                     Ur[oh] = accr[base + ma] + (ma == MB ? wself : 0.0);
                     Ui[oh] = acci[base + ma];
@@ -124,7 +159,7 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
 template <int J>
 constexpr int ui_ngroups() { return J == 8 ? 4 : (J == 6 ? 3 : 1); }
 
-template <int J, int MODE, bool GEO = false>
+template <int J, int MODE, bool GEO = false, int SUB = 1>
 __global__ __launch_bounds__(64) void k_ui(SnapDev s, double* __restrict__ Ur, double* __restrict__ Ui,
                                            const double* __restrict__ rij, const int* __restrict__ pair_off,
                                            const int* __restrict__ perm, const int* __restrict__ ti,
@@ -133,29 +168,30 @@ __global__ __launch_bounds__(64) void k_ui(SnapDev s, double* __restrict__ Ur, d
     constexpr int NG = ui_ngroups<J>();
     const int b = blockIdx.x, k = b / 8;
     const int group = k % NG, ablock = (k / NG) * 8 + b % 8;
-    const int atom = ablock * 64 + threadIdx.x;
-    if (atom >= N) return;
+    const int atom = ablock * (64 / SUB) + static_cast<int>(threadIdx.x) / SUB, sub = threadIdx.x % SUB;
+    if (SUB == 1 && atom >= N) return;
     if constexpr (J == 8) {
-        if (group == 0) ui_rows<8, 0, 0, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
-        else if (group == 1) ui_rows<8, 1, 1, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
-        else if (group == 2) ui_rows<8, 2, 2, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
-        else ui_rows<8, 3, 4, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
+        if (group == 0) ui_rows<8, 0, 0, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else if (group == 1) ui_rows<8, 1, 1, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else if (group == 2) ui_rows<8, 2, 2, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else ui_rows<8, 3, 4, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
     } else if constexpr (J == 6) {
-        if (group == 0) ui_rows<6, 0, 0, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
-        else if (group == 1) ui_rows<6, 1, 1, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
-        else ui_rows<6, 2, 3, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
+        if (group == 0) ui_rows<6, 0, 0, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else if (group == 1) ui_rows<6, 1, 1, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else ui_rows<6, 2, 3, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
     } else {
-        ui_rows<J, 0, J / 2, MODE, GEO>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo);
+        ui_rows<J, 0, J / 2, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
     }
 }
 
-template <int J, int MODE, bool GEO = false>
+template <int J, int MODE, bool GEO = false, int SUB = 1>
 static void ui_groups(const SnapDev& s, double* Ur, double* Ui, const double* rij, const int* off, const int* perm,
                       const int* ti, const int* tj, int N, double wself, int esel, hipStream_t st,
                       const double* pgeo = nullptr) {
     constexpr int NG = ui_ngroups<J>();
-    const int ablocks = ((N + 63) / 64 + 7) / 8 * 8;   // padded to whole XCD rounds; excess blocks return
-    hipLaunchKernelGGL((k_ui<J, MODE, GEO>), dim3(ablocks * NG), dim3(64), 0, st, s, Ur, Ui, rij, off, perm, ti, tj,
+    constexpr int A = 64 / SUB;   // atoms per workgroup
+    const int ablocks = ((N + A - 1) / A + 7) / 8 * 8;   // padded to whole XCD rounds; excess blocks return
+    hipLaunchKernelGGL((k_ui<J, MODE, GEO, SUB>), dim3(ablocks * NG), dim3(64), 0, st, s, Ur, Ui, rij, off, perm, ti, tj,
                        N, wself, esel, pgeo);
 }
 
@@ -294,16 +330,41 @@ void launch_ui_geo_lds(const SnapDev& s, double* Ur, double* Ui, const double* p
     }
 }
 
+// Measured on displaced BCC crystals, us with 1 / 4 / 16 lanes per atom: twojmax 4, 128 atoms 16 / 9 / 9, 16,000 atoms
+// 20 / 15 / 48, 65,536 atoms 27 / 45 / 163; twojmax 6, 128 atoms 17 / 9 / 7, 8,192 atoms 20 / 16 / 34, 31,250 atoms
+// 39 / 40 / 102; twojmax 8, 432 atoms 33 / 15 / 14, 8,192 atoms 36 / 32 / 103, 16,000 atoms 39 / 59 / 197.  The lines
+// lie where one lane per atom would leave most (24 waves) or half (512 waves) of the 1,024 SIMDs idle.
+int ui_lanes_per_atom(int J, int N) {
+    const long groups = J == 8 ? 4 : (J == 6 ? 3 : 1);
+    const long waves = (N + 63L) / 64 * groups;
+    return waves <= 24 ? 16 : (waves <= 512 ? 4 : 1);
+}
+
 void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int N,
-                   double wself, hipStream_t st) {
+                   double wself, hipStream_t st, int lanes) {
     if (N <= 0) return;
+    if (lanes == 0) lanes = ui_lanes_per_atom(s.J, N);
+#define UG(JV, SUBV)                                                                                                 \
+    ui_groups<JV, UI_HALF_WSELF, true, SUBV>(s, Ur, Ui, nullptr, pair_off, nullptr, nullptr, nullptr, N, wself, -1, st, \
+                                             pgeo)
+#define UG_CASE(JV)                                                        \
+    case JV:                                                               \
+        if (lanes == 16)                                                   \
+            UG(JV, 16);                                                    \
+        else if (lanes == 4)                                               \
+            UG(JV, 4);                                                     \
+        else                                                               \
+            UG(JV, 1);                                                     \
+        break;
     switch (s.J) {
-        case 2: ui_groups<2, UI_HALF_WSELF, true>(s, Ur, Ui, nullptr, pair_off, nullptr, nullptr, nullptr, N, wself, -1, st, pgeo); break;
-        case 4: ui_groups<4, UI_HALF_WSELF, true>(s, Ur, Ui, nullptr, pair_off, nullptr, nullptr, nullptr, N, wself, -1, st, pgeo); break;
-        case 6: ui_groups<6, UI_HALF_WSELF, true>(s, Ur, Ui, nullptr, pair_off, nullptr, nullptr, nullptr, N, wself, -1, st, pgeo); break;
-        case 8: ui_groups<8, UI_HALF_WSELF, true>(s, Ur, Ui, nullptr, pair_off, nullptr, nullptr, nullptr, N, wself, -1, st, pgeo); break;
+        UG_CASE(2)
+        UG_CASE(4)
+        UG_CASE(6)
+        UG_CASE(8)
         default: break;
     }
+#undef UG_CASE
+#undef UG
 }
 
 }  // namespace mdp

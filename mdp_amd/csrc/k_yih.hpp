@@ -300,7 +300,7 @@ __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ c
 // compute_yi where 64-atom blocks are too few to fill the chip: one workgroup per (block, output row).  Its W waves
 // split the row's terms by the U rows (J1, mb1) of the larger layer, and the W partial rows are added in LDS in
 // wave order.  k_yi_half keeps a whole output row on one wave and a whole block on one CU, so on a few blocks its
-// time is that of a block (129 us at twojmax 8, 63 us at 6) whatever their number; here n_half_rows times as many
+// time is that of a block (125 us at twojmax 8, 64 us at 6) whatever their number (128 atoms here: 18 and 12 us); here n_half_rows times as many
 // CUs work on it, at the price of staging the block's U once per row.  That staging (about 1 us of L2 reads a
 // workgroup) is why k_yi_half stays the better one from some 150 blocks on; the engine times both.
 // Workgroups are dealt to the 8 XCDs round-robin, so workgroup b takes a block of index b mod 8: the rows of one

@@ -864,7 +864,8 @@ struct mdp_md {
     double rmse_last = 0, rmse_max = 0, rmse_sum = 0;
     // autotuned launch variants (see autotune())
     int dedr_variant = 3, yi_waves = 8;
-    int ui_variant = 0;   // compute_ui: 0 = one thread per atom and row group, G > 0 = LDS sums on G workgroups
+    // compute_ui: 0, 4, 16 = 1, 4, 16 lanes per atom and row group, G >= 256: LDS sums on G workgroups
+    int ui_variant = 0;
     int nb_variant = 0;   // cell-list neighbour kernel (neighbors_launch)
     bool tuned = false;
     std::string tuning_json = "{}";
@@ -973,8 +974,11 @@ struct mdp_md {
         }
         nrows = n_half_rows(J);
         // until (or without) the autotuner: a workgroup per output row where a workgroup per 64 atoms would leave
-        // most CUs idle (it loses from some 150 blocks on)
-        yi_waves = N <= 64 * 128 ? 208 : 8;
+        // most CUs idle (us, per row / per block: twojmax 8, 4,394 atoms 106 / 132, 8,192 atoms 184 / 144; twojmax 6,
+        // 8,192 atoms 56 / 72, 16,000 atoms 105 / 82)
+        yi_waves = N <= 64 * (J == 8 ? 80 : 128) ? 208 : (J == 8 ? 116 : 8);
+        const int lanes = ui_lanes_per_atom(J, N);
+        ui_variant = lanes > 1 ? lanes : 0;
         massinv_h.assign(ntypes + 1, 0.0);
         for (int t = 1; t <= ntypes; ++t) massinv_h[t] = 1.0 / p->mass[t - 1];
         rc2_h.assign((ntypes + 1) * (ntypes + 1), 0.0);
@@ -1168,8 +1172,9 @@ struct mdp_md {
     }
 
     void ui_launch(int v) {
-        if (v == 0)
-            launch_ui_geo(tab.view, Ur.as<double>(), Ui.as<double>(), pgeo.as<double>(), poff.as<int>(), N, 1.0, st);
+        if (v < 256)
+            launch_ui_geo(tab.view, Ur.as<double>(), Ui.as<double>(), pgeo.as<double>(), poff.as<int>(), N, 1.0, st,
+                          v > 0 ? v : 1);
         else
             launch_ui_geo_lds(tab.view, Ur.as<double>(), Ui.as<double>(), pgeo.as<double>(), poff.as<int>(), N, 1.0,
                               v, st);
@@ -1385,14 +1390,14 @@ struct mdp_md {
             js += (k ? ", " : "") + std::string("\"") + std::to_string(ids[k]) + "\": " + std::to_string(t);
             if (t < best) { best = t; yi_waves = ids[k]; }
         }
-        // compute_ui: the per-atom kernel, or the LDS-sum kernel on 256, 512 or 1024 workgroups;
-        // MDP_UI_VARIANT pins one of 0, 256, 512, 1024
+        // compute_ui: the per-atom kernel on 1 (variant 0), 4 or 16 lanes per atom, or the LDS-sum kernel on 256, 512
+        // or 1024 workgroups; MDP_UI_VARIANT pins one of 0, 4, 16, 256, 512, 1024
         js += "}, \"compute_ui\": {";
-        int uids[4] = {0, 256, 512, 1024}, nu = 4;
+        int uids[6] = {0, 4, 16, 256, 512, 1024}, nu = 6;
         if (const char* up = std::getenv("MDP_UI_VARIANT")) {
             const int v = std::atoi(up);
-            if (v != 0 && v != 256 && v != 512 && v != 1024)
-                throw Error("MDP_UI_VARIANT is not a compute_ui variant (0, 256, 512 or 1024)");
+            if (v != 0 && v != 4 && v != 16 && v != 256 && v != 512 && v != 1024)
+                throw Error("MDP_UI_VARIANT is not a compute_ui variant (0, 4, 16, 256, 512 or 1024)");
             uids[0] = v;
             nu = 1;
         }

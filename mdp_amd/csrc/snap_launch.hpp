@@ -41,9 +41,10 @@ void launch_ui(const SnapDev& s, UiMode mode, double* Ur, double* Ui, const doub
                hipStream_t st);
 // compute_ui on the half layout with wself (UI_HALF_WSELF) from per-pair geometry written by the MD
 // pair list: pgeo[5p..5p+4] = (a_r, a_i, b_r, b_i, sfac * w_j) of pair p, pairs of atom i in
-// [pair_off[i], pair_off[i+1]).
+// [pair_off[i], pair_off[i+1]).  lanes: 1, 4 or 16 lanes share an atom's pairs (0: by ui_lanes_per_atom).
 void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int natoms,
-                   double wself, hipStream_t st);
+                   double wself, hipStream_t st, int lanes = 0);
+int ui_lanes_per_atom(int J, int natoms);
 // pgeo[5q..5q+4] = (a_r, a_i, b_r, b_i, sfac w_j) of every pair q < *np_dev (cap: the launch's pair capacity)
 void launch_pair_geo(const SnapDev& s, const double* rij, const int* ti, const int* tj, const int* np_dev, int cap,
                      double* pgeo, hipStream_t st);

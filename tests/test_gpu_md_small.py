@@ -31,6 +31,16 @@ def test_yi_row_workgroups_vs_oracle(oracle, monkeypatch, J, n):
     assert md.tuning()["chosen"]["compute_yi_waves"] == 208
 
 
+@pytest.mark.parametrize("variant", ["4", "16"])
+@pytest.mark.parametrize("J,n", [(2, 1), (4, 63), (6, 65), (8, 17), (8, 250)])
+def test_ui_lanes_per_atom_vs_oracle(oracle, monkeypatch, J, n, variant):
+    """compute_ui with 4 or 16 lanes sharing an atom's pairs: fewer and more pairs than lanes, ragged last waves."""
+    monkeypatch.setenv("MDP_UI_VARIANT", variant)
+    x, box = _atoms(n, 70 + n + J)
+    md = _first_step_vs_oracle(oracle, x, box, J, 5)
+    assert md.tuning()["chosen"]["compute_ui"] == int(variant)
+
+
 def test_neighbor_tile_of_256_lanes_identical(oracle, monkeypatch):
     """The tile kernel on 256 lanes per cell writes the lists of the L1 kernel entry for entry: ragged cells, empty
     cells, and cells whose surroundings need more than one tile."""
