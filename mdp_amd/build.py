@@ -30,11 +30,12 @@ FLAGS = ["-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC", "-Wall", "-Wno-
 
 # Per-file flags.  The Z/Y row kernels read their inner Clebsch-Gordan coefficients as compile-time
 # constants; machine-level loop-invariant code motion would hoist thousands of them out of the row loop
-# into SGPRs and spill those to VGPR lanes, so it is disabled for these translation units.
+# into SGPRs and spill those to VGPR lanes, so it is disabled for these translation units.  In the MD engine the
+# same motion keeps the constants of tan, sincos and exp in VGPRs across the pair list's loop (120 instead of 70).
 FILE_FLAGS = {f: ["-mllvm", "-disable-machine-licm"]
               for f in ("k_yih_8_8.hip", "k_yih_8_12.hip", "k_yih_8_4.hip", "k_yih_8_12s.hip", "k_yih_8_12c.hip",
                         "k_yih_8_12y.hip", "k_yih_8_12u1.hip", "k_yih_rows_8.hip", "k_yih_rows.hip", "k_yih_small.hip",
-                        "k_fit_zb.hip")}
+                        "k_fit_zb.hip", "md_engine.hip")}
 
 
 def hipcc():

@@ -316,7 +316,8 @@ struct mdp_fit {
                 if (zb_lds) {   // half U + wself from the per-pair geometry (one geometry per pair)
                     launch_pair_geo(s, rij.as<double>(), pti.as<int>(), ptj.as<int>(), poff.as<int>() + N,
                                     static_cast<int>(cap), pgeo.as<double>(), st);
-                    launch_ui_geo(s, Ur.as<double>(), Ui.as<double>(), pgeo.as<double>(), poff.as<int>(), N, 1.0, st);
+                    launch_ui_geo(s, Ur.as<double>(), Ui.as<double>(), pgeo.as<double>(), poff.as<int>(),
+                                  poff.as<int>() + 1, N, 1.0, st);
                 } else {
                     launch_ui(s, UI_FULL_WSELF, Ur.as<double>(), Ui.as<double>(), rij.as<double>(), poff.as<int>(),
                               nullptr, pti.as<int>(), ptj.as<int>(), N, 1.0, -1, st);

@@ -21,12 +21,14 @@ __global__ __launch_bounds__(64) void k_dedr(SnapDev s, const double* __restrict
     const int p = blockIdx.x * 64 + threadIdx.x;
     const int np = npairs_dev ? *npairs_dev : npairs_host;
     if (p >= np) return;
+    const int ya = yatom[p];
+    if (ya < 0) return;
     const int tjp = tj[p];
     const double rc = (s.radelem[ti[p]] + s.radelem[tjp]) * s.rcutfac;
     PairGeom g;
     pair_geometry<true>(rij[3 * p], rij[3 * p + 1], rij[3 * p + 2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
     const size_t n = static_cast<size_t>(N);
-    const size_t yb = static_cast<size_t>(yatom[p]) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
+    const size_t yb = static_cast<size_t>(ya) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
     double d0 = 0.0, d1 = 0.0, d2 = 0.0;
     row_chain<J, 3, 0, J / 2>(g, s.rootpq, [&](auto Jc, auto MBc, auto& pr, auto& pi, auto& dpr, auto& dpi) {
         constexpr int JJ = decltype(Jc)::value, MB = decltype(MBc)::value;
@@ -72,6 +74,8 @@ __global__ __launch_bounds__(64 * NW, WPE) void k_dedr_split(SnapDev s, const do
     const int p = (blockIdx.x * NW + static_cast<int>(threadIdx.x >> 6)) * 21 + lane / 3, comp = lane % 3;
     const int np = npairs_dev ? *npairs_dev : npairs_host;
     if (lane >= 63 || p >= np) return;
+    const int ya = yatom[p];
+    if (ya < 0) return;
     const int tjp = tj[p];
     const double rc = (s.radelem[ti[p]] + s.radelem[tjp]) * s.rcutfac;
     PairGeom g;
@@ -83,7 +87,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void k_dedr_split(SnapDev s, const do
     g.dbr[0] = comp == 0 ? g.dbr[0] : (comp == 1 ? g.dbr[1] : g.dbr[2]);
     g.dbi[0] = comp == 0 ? g.dbi[0] : (comp == 1 ? g.dbi[1] : g.dbi[2]);
     const size_t n = static_cast<size_t>(N);
-    const size_t yb = static_cast<size_t>(yatom[p]) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
+    const size_t yb = static_cast<size_t>(ya) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
     const double dsu = g.dsfac * uk;
     double d = 0.0;
     row_chain<J, 1, 0, J / 2>(g, s.rootpq, [&](auto Jc, auto MBc, auto& pr, auto& pi, auto& dpr, auto& dpi) {
@@ -138,12 +142,14 @@ __global__ __launch_bounds__(64 * NW) void k_dedr_gen(SnapDev s, const double* _
     }
     const int p = (tile * NW + static_cast<int>(threadIdx.x >> 6)) * 64 + static_cast<int>(threadIdx.x & 63);
     if (p >= np) return;
+    const int ya = yatom[p];
+    if (ya < 0) return;
     const int tjp = tj[p];
     const double rc = (s.radelem[ti[p]] + s.radelem[tjp]) * s.rcutfac;
     PairGeom g;
     pair_geometry<true>(rij[3 * p], rij[3 * p + 1], rij[3 * p + 2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
     const size_t n = static_cast<size_t>(N);
-    const size_t yb = static_cast<size_t>(yatom[p]) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
+    const size_t yb = static_cast<size_t>(ya) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
     double f = 0.5 * Yr[yb], t0 = 0.0, t1 = 0.0, t2 = 0.0;
     // With PREFETCH, Y rows are loaded one emitted row ahead (rows come in the order (1,0) .. (J,0),
     // (2,1) .. (J,1), ...) so that their latency overlaps the recursion of the current row.
@@ -223,11 +229,12 @@ __global__ __launch_bounds__(64, 2) void k_dedr_atom(const double* __restrict__ 
                                                     const double* __restrict__ wjelem, double rcutfac, double rmin0,
                                                     double rfac0, int switchflag, const double* __restrict__ rij,
                                                     const int* __restrict__ ti, const int* __restrict__ tj,
-                                                    const int* __restrict__ poff, double* __restrict__ dedr) {
+                                                    const int* __restrict__ poff, const int* __restrict__ pend,
+                                                    double* __restrict__ dedr) {
     constexpr int HE = n_half_elems(J);
     const int atom = blockIdx.x;
     const int lane = threadIdx.x, comp = lane % 3, slot = lane / 3;
-    const int q0 = poff[atom], q1 = poff[atom + 1];
+    const int q0 = poff[atom], q1 = pend[atom];
     const double* __restrict__ y = yt + static_cast<size_t>(atom) * HE * 2;
     for (int qb = q0; qb < q1; qb += 21) {
         const int q = qb + slot;
@@ -264,7 +271,8 @@ __global__ __launch_bounds__(64, 2) void k_dedr_atom(const double* __restrict__ 
 }
 
 void launch_dedr_atom(const SnapDev& s, const double* Yr, const double* Yi, double* yt, const double* rij,
-                      const int* ti, const int* tj, const int* pair_off, double* dedr, int N, hipStream_t st) {
+                      const int* ti, const int* tj, const int* pair_off, const int* pair_end, double* dedr, int N,
+                      hipStream_t st) {
     if (N <= 0) return;
     int HE = 0;
     switch (s.J) {
@@ -280,7 +288,7 @@ void launch_dedr_atom(const SnapDev& s, const double* Yr, const double* Yi, doub
 #define DA_CASE(JV)                                                                                               \
     case JV:                                                                                                      \
         hipLaunchKernelGGL((k_dedr_atom<JV>), dim3(N), dim3(64), 0, st, s.rootpq, yt, s.radelem, s.wjelem, s.rcutfac, \
-                           s.rmin0, s.rfac0, s.switchflag, rij, ti, tj, pair_off, dedr);                          \
+                           s.rmin0, s.rfac0, s.switchflag, rij, ti, tj, pair_off, pair_end, dedr);                \
         return;
         DA_CASE(2)
         DA_CASE(4)

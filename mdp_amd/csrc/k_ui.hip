@@ -46,7 +46,7 @@ __device__ __forceinline__ double sub_sum(double v) {
 template <int J, int RLO, int RHI, int MODE, bool GEO = false, int SUB = 1>
 __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ Ur, double* __restrict__ Ui,
                                         const double* __restrict__ rij, const int* __restrict__ pair_off,
-                                        const int* __restrict__ perm, const int* __restrict__ ti,
+                                        const int* __restrict__ pair_end, const int* __restrict__ perm, const int* __restrict__ ti,
                                         const int* __restrict__ tj, int N, double wself, int elem_sel, int atom,
                                         const double* __restrict__ pgeo = nullptr, int sub = 0) {
     static_assert(SUB == 1 || (GEO && MODE == UI_HALF_WSELF), "lanes share an atom in the MD and fitting form only");
@@ -67,7 +67,7 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
     };
 
     // the next pair's data are loaded while the current pair's recursion runs
-    const int q0 = SUB == 1 || atom < N ? pair_off[atom] : 0, q1 = SUB == 1 || atom < N ? pair_off[atom + 1] : 0;
+    const int q0 = SUB == 1 || atom < N ? pair_off[atom] : 0, q1 = SUB == 1 || atom < N ? pair_end[atom] : 0;
     if constexpr (GEO) {
         double n[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         if (q0 + sub < q1)
@@ -162,7 +162,7 @@ constexpr int ui_ngroups() { return J == 8 ? 4 : (J == 6 ? 3 : 1); }
 template <int J, int MODE, bool GEO = false, int SUB = 1>
 __global__ __launch_bounds__(64) void k_ui(SnapDev s, double* __restrict__ Ur, double* __restrict__ Ui,
                                            const double* __restrict__ rij, const int* __restrict__ pair_off,
-                                           const int* __restrict__ perm, const int* __restrict__ ti,
+                                           const int* __restrict__ pair_end, const int* __restrict__ perm, const int* __restrict__ ti,
                                            const int* __restrict__ tj, int N, double wself, int elem_sel,
                                            const double* __restrict__ pgeo) {
     constexpr int NG = ui_ngroups<J>();
@@ -171,28 +171,28 @@ __global__ __launch_bounds__(64) void k_ui(SnapDev s, double* __restrict__ Ur, d
     const int atom = ablock * (64 / SUB) + static_cast<int>(threadIdx.x) / SUB, sub = threadIdx.x % SUB;
     if (SUB == 1 && atom >= N) return;
     if constexpr (J == 8) {
-        if (group == 0) ui_rows<8, 0, 0, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
-        else if (group == 1) ui_rows<8, 1, 1, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
-        else if (group == 2) ui_rows<8, 2, 2, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
-        else ui_rows<8, 3, 4, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        if (group == 0) ui_rows<8, 0, 0, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else if (group == 1) ui_rows<8, 1, 1, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else if (group == 2) ui_rows<8, 2, 2, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else ui_rows<8, 3, 4, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
     } else if constexpr (J == 6) {
-        if (group == 0) ui_rows<6, 0, 0, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
-        else if (group == 1) ui_rows<6, 1, 1, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
-        else ui_rows<6, 2, 3, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        if (group == 0) ui_rows<6, 0, 0, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else if (group == 1) ui_rows<6, 1, 1, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        else ui_rows<6, 2, 3, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
     } else {
-        ui_rows<J, 0, J / 2, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
+        ui_rows<J, 0, J / 2, MODE, GEO, SUB>(s, Ur, Ui, rij, pair_off, pair_end, perm, ti, tj, N, wself, elem_sel, atom, pgeo, sub);
     }
 }
 
 template <int J, int MODE, bool GEO = false, int SUB = 1>
-static void ui_groups(const SnapDev& s, double* Ur, double* Ui, const double* rij, const int* off, const int* perm,
-                      const int* ti, const int* tj, int N, double wself, int esel, hipStream_t st,
+static void ui_groups(const SnapDev& s, double* Ur, double* Ui, const double* rij, const int* off, const int* end,
+                      const int* perm, const int* ti, const int* tj, int N, double wself, int esel, hipStream_t st,
                       const double* pgeo = nullptr) {
     constexpr int NG = ui_ngroups<J>();
     constexpr int A = 64 / SUB;   // atoms per workgroup
     const int ablocks = ((N + A - 1) / A + 7) / 8 * 8;   // padded to whole XCD rounds; excess blocks return
-    hipLaunchKernelGGL((k_ui<J, MODE, GEO, SUB>), dim3(ablocks * NG), dim3(64), 0, st, s, Ur, Ui, rij, off, perm, ti, tj,
-                       N, wself, esel, pgeo);
+    hipLaunchKernelGGL((k_ui<J, MODE, GEO, SUB>), dim3(ablocks * NG), dim3(64), 0, st, s, Ur, Ui, rij, off, end, perm, ti,
+                       tj, N, wself, esel, pgeo);
 }
 
 void launch_ui(const SnapDev& s, UiMode mode, double* Ur, double* Ui, const double* rij, const int* pair_off,
@@ -201,11 +201,11 @@ void launch_ui(const SnapDev& s, UiMode mode, double* Ur, double* Ui, const doub
 #define UI_CASE(JV)                                                                                   \
     case JV:                                                                                          \
         if (mode == UI_ACCUMULATE)                                                                    \
-            ui_groups<JV, UI_ACCUMULATE>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, esel, st); \
+            ui_groups<JV, UI_ACCUMULATE>(s, Ur, Ui, rij, pair_off, pair_off + 1, perm, ti, tj, N, wself, esel, st); \
         else if (mode == UI_HALF_WSELF)                                                               \
-            ui_groups<JV, UI_HALF_WSELF>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, esel, st); \
+            ui_groups<JV, UI_HALF_WSELF>(s, Ur, Ui, rij, pair_off, pair_off + 1, perm, ti, tj, N, wself, esel, st); \
         else                                                                                          \
-            ui_groups<JV, UI_FULL_WSELF>(s, Ur, Ui, rij, pair_off, perm, ti, tj, N, wself, esel, st); \
+            ui_groups<JV, UI_FULL_WSELF>(s, Ur, Ui, rij, pair_off, pair_off + 1, perm, ti, tj, N, wself, esel, st); \
         break;
     switch (s.J) {
         UI_CASE(2)
@@ -243,43 +243,46 @@ void launch_pair_geo(const SnapDev& s, const double* rij, const int* ti, const i
     hipLaunchKernelGGL(k_pair_geo, dim3((cap + 255) / 256), dim3(256), 0, st, s, rij, ti, tj, np_dev, pgeo);
 }
 
-// compute_ui with the per-atom sums in LDS (half layout plus wself, from the pair geometry pgeo).  Lanes
-// are pairs: workgroup block b holds the atoms whose first pair lies in [b*UI_PB, (b+1)*UI_PB), so with at
-// most UI_MAXP pairs per atom a block has fewer than UI_PB + UI_MAXP <= 512 pairs, one per lane.  Each
-// lane runs the row-chain recursion of its pair; every finished half row, scaled by sfac w_j, goes to LDS;
-// then thread (ma, atom) adds the row entry of the atom's pairs in pair order and writes U, with wself added
-// to the diagonal last (upstream adds it first, cpuSnap.cpp:312-542; the sums agree to rounding, as those of
-// the per-atom kernel do).  The workgroups are persistent over the blocks; all lanes share the control flow
-// of the recursion.
-constexpr int UI_PB = 416, UI_MAXP = 96, UI_NL = 512;
+// compute_ui with the per-atom sums in LDS (half layout plus wself, from the pair geometry pgeo).  Lanes are pairs.
+// The pairs of `ab` (at most 64) consecutive atoms are contiguous; window b of such a block holds its atoms whose first pair lies in
+// [b*UI_PB, (b+1)*UI_PB) of the block, so with at most 96 pairs per atom (UI_NL - UI_PB) a window has at most UI_NL
+// pairs, one per lane.  Each lane runs the row-chain recursion of its pair; every finished half row, scaled by
+// sfac w_j, goes to LDS; then thread (ma, atom) adds the row entry of the atom's pairs in pair order and writes U, with
+// wself added to the diagonal last (upstream adds it first, cpuSnap.cpp:312-542; the sums agree to rounding, as those
+// of the per-atom kernel do).  The workgroups are persistent over the blocks; all lanes share the control flow of the
+// recursion.
+constexpr int UI_PB = 416, UI_NL = 512;
 
 template <int J>
 __global__ __launch_bounds__(UI_NL) void k_ui_lds(const double* __restrict__ rootpq, double* __restrict__ Ur,
                                                  double* __restrict__ Ui, const double* __restrict__ pgeo,
-                                                 const int* __restrict__ poff, int N, double wself) {
+                                                 const int* __restrict__ poff, const int* __restrict__ pend, int N,
+                                                 double wself, int ab) {
     constexpr int RW = J + 1;
     __shared__ double sr[UI_NL * RW], si[UI_NL * RW];
-    __shared__ int s_off[UI_NL + 1];   // pair offsets (relative to the block) of the block's atoms
+    __shared__ int s_off[64 + 1];   // pair offsets (relative to the window) of the window's atoms
     const int lane = threadIdx.x;
-    const int ptot = poff[N];
     const size_t n = static_cast<size_t>(N);
-    for (int b = blockIdx.x; static_cast<long>(b) * UI_PB <= ptot; b += gridDim.x) {
-        // atoms a0..a1-1: a0 (a1) is the first atom with poff[a] >= b*UI_PB (>= (b+1)*UI_PB), by binary search
-        auto lower = [&](long v) {
-            int lo = 0, hi = N;
+    const int blocks = (N + ab - 1) / ab;
+    for (int blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
+      const int f0 = ab * blk, f1 = min(f0 + ab, N), base = poff[f0], ptot = pend[f1 - 1] - base;
+      for (int b = 0; b * UI_PB <= ptot; ++b) {
+        // atoms a0..a1-1: a0 (a1) is the first atom whose pairs start at or behind b*UI_PB ((b+1)*UI_PB)
+        auto lower = [&](int v) {
+            int lo = f0, hi = f1;
             while (lo < hi) {
                 const int mid = lo + (hi - lo) / 2;
-                if (poff[mid] < v) lo = mid + 1;
+                if (poff[mid] - base < v) lo = mid + 1;
                 else hi = mid;
             }
             return lo;
         };
-        const int a0 = lower(static_cast<long>(b) * UI_PB), a1 = lower(static_cast<long>(b + 1) * UI_PB);
+        const int a0 = lower(b * UI_PB), a1 = lower((b + 1) * UI_PB);
         const int na = a1 - a0;
-        if (na <= 0) continue;
-        const int q0 = poff[a0], np = poff[a1] - q0;   // np < UI_PB + UI_MAXP <= UI_NL
-        __syncthreads();   // the previous block's readers are done with s_off and the row stage
-        for (int k = lane; k <= na; k += UI_NL) s_off[k] = poff[a0 + k] - q0;
+        if (na <= 0) continue;   // uniform
+        const int q0 = poff[a0], np = pend[a1 - 1] - q0;   // at most UI_NL
+        __syncthreads();   // the previous window's readers are done with s_off and the row stage
+        for (int k = lane; k <= na; k += UI_NL) s_off[k] = (k < na ? poff[a0 + k] : pend[a1 - 1]) - q0;
         PairGeom g;   // lanes past the block's pairs run the recursion on a zero pair; nothing reads them
         g.ar = g.ai = g.br = g.bi = 0.0;
         double sf = 0.0;
@@ -303,7 +306,7 @@ __global__ __launch_bounds__(UI_NL) void k_ui_lds(const double* __restrict__ roo
             constexpr int row = h_block(L) + (L + 1) * MB;
             for (int t = lane; t < na * (L + 1); t += UI_NL) {
                 const int ma = t / na, al = t - ma * na;   // consecutive threads: consecutive atoms
-                const int p1 = min(s_off[al + 1], UI_NL);   // the bound holds with <= UI_MAXP pairs per atom
+                const int p1 = min(s_off[al + 1], UI_NL);   // the bound holds with at most 96 pairs per atom
                 double ar = 0.0, ai = 0.0;
                 for (int p = s_off[al]; p < p1; ++p) {
                     ar += sr[p * RW + ma];
@@ -314,18 +317,19 @@ __global__ __launch_bounds__(UI_NL) void k_ui_lds(const double* __restrict__ roo
                 Ui[o] = ai;
             }
         });
+      }
     }
 }
 
-void launch_ui_geo_lds(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int N,
-                       double wself, int groups, hipStream_t st) {
+void launch_ui_geo_lds(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off,
+                       const int* pair_end, int N, double wself, int groups, int ab, hipStream_t st) {
     if (N <= 0) return;
     const int G = groups > 0 ? groups : 512;
     switch (s.J) {
-        case 2: hipLaunchKernelGGL((k_ui_lds<2>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, N, wself); break;
-        case 4: hipLaunchKernelGGL((k_ui_lds<4>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, N, wself); break;
-        case 6: hipLaunchKernelGGL((k_ui_lds<6>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, N, wself); break;
-        case 8: hipLaunchKernelGGL((k_ui_lds<8>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, N, wself); break;
+        case 2: hipLaunchKernelGGL((k_ui_lds<2>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, pair_end, N, wself, ab); break;
+        case 4: hipLaunchKernelGGL((k_ui_lds<4>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, pair_end, N, wself, ab); break;
+        case 6: hipLaunchKernelGGL((k_ui_lds<6>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, pair_end, N, wself, ab); break;
+        case 8: hipLaunchKernelGGL((k_ui_lds<8>), dim3(G), dim3(UI_NL), 0, st, s.rootpq, Ur, Ui, pgeo, pair_off, pair_end, N, wself, ab); break;
         default: break;
     }
 }
@@ -340,12 +344,12 @@ int ui_lanes_per_atom(int J, int N) {
     return waves <= 24 ? 16 : (waves <= 512 ? 4 : 1);
 }
 
-void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int N,
-                   double wself, hipStream_t st, int lanes) {
+void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off,
+                   const int* pair_end, int N, double wself, hipStream_t st, int lanes) {
     if (N <= 0) return;
     if (lanes == 0) lanes = ui_lanes_per_atom(s.J, N);
 #define UG(JV, SUBV)                                                                                                 \
-    ui_groups<JV, UI_HALF_WSELF, true, SUBV>(s, Ur, Ui, nullptr, pair_off, nullptr, nullptr, nullptr, N, wself, -1, st, \
+    ui_groups<JV, UI_HALF_WSELF, true, SUBV>(s, Ur, Ui, nullptr, pair_off, pair_end, nullptr, nullptr, nullptr, N, wself, -1, st, \
                                              pgeo)
 #define UG_CASE(JV)                                                        \
     case JV:                                                               \

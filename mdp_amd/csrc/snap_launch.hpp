@@ -41,17 +41,18 @@ void launch_ui(const SnapDev& s, UiMode mode, double* Ur, double* Ui, const doub
                hipStream_t st);
 // compute_ui on the half layout with wself (UI_HALF_WSELF) from per-pair geometry written by the MD
 // pair list: pgeo[5p..5p+4] = (a_r, a_i, b_r, b_i, sfac * w_j) of pair p, pairs of atom i in
-// [pair_off[i], pair_off[i+1]).  lanes: 1, 4 or 16 lanes share an atom's pairs (0: by ui_lanes_per_atom).
-void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int natoms,
-                   double wself, hipStream_t st, int lanes = 0);
+// [pair_off[i], pair_end[i]).  lanes: 1, 4 or 16 lanes share an atom's pairs (0: by ui_lanes_per_atom).
+void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off,
+                   const int* pair_end, int natoms, double wself, hipStream_t st, int lanes = 0);
 int ui_lanes_per_atom(int J, int natoms);
 // pgeo[5q..5q+4] = (a_r, a_i, b_r, b_i, sfac w_j) of every pair q < *np_dev (cap: the launch's pair capacity)
 void launch_pair_geo(const SnapDev& s, const double* rij, const int* ti, const int* tj, const int* np_dev, int cap,
                      double* pgeo, hipStream_t st);
-// The same result with the per-atom sums formed in LDS, one lane per pair (at most 96 pairs per atom);
+// The same result with the per-atom sums formed in LDS, one lane per pair (at most 96 pairs per atom, the pairs of
+// atoms ab k .. ab k + ab - 1 contiguous and in atom order, ab <= 64);
 // persistent over `groups` workgroups of 512 lanes (0: 512).
 void launch_ui_geo_lds(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off,
-                       int natoms, double wself, int groups, hipStream_t st);
+                       const int* pair_end, int natoms, double wself, int groups, int ab, hipStream_t st);
 
 // Y[half rows] of every atom (Y zeroed by the caller where untouched).  beta_t[triple] holds the
 // effective weight of each coupling triple (multiplicity, (j1+1)/(j+1) and 1/(j+1) factors folded
@@ -96,17 +97,19 @@ void launch_zi(const SnapDev& s, const double* Ur, const double* Ui, long off1, 
                int natoms, int bnorm, hipStream_t st);
 
 // dE/dr_ij per pair: 2 sum' d(sfac U_ij)/dr . Y(atom of the pair); pairs p in [0, *npairs) (device count)
-// or [0, npairs_host) when npairs_dev == nullptr.  yatom[p] = row of Y used (aii), ybase[p] optional
+// or [0, npairs_host) when npairs_dev == nullptr; a pair with yatom[p] < 0 is skipped (an empty slot of the MD pair
+// list).  yatom[p] = row of Y used (aii), ybase[p] optional
 // element offset (elements) for chemflag.  The full layout always runs the SU(2)-generator kernel; the
 // half layout runs the given variant (dedr_variants).
 void launch_dedr(const SnapDev& s, const double* Yr, const double* Yi, const double* rij, const int* yatom,
                  const int* ti, const int* tj, const long* ybase, double* dedr, int natoms, int npairs_host,
                  const int* npairs_dev, hipStream_t st, bool half_layout = false, int variant = 0);
-// dE/dr with one centre atom per wave (pairs sorted by centre atom, CSR offsets pair_off): Y (half
+// dE/dr with one centre atom per wave (pairs of an atom in [pair_off, pair_end)): Y (half
 // layout) is first copied atom-major into yt (2 * n_half_elems(J) * natoms doubles) so that each
 // wave reads its atom's Y through the scalar cache.
 void launch_dedr_atom(const SnapDev& s, const double* Yr, const double* Yi, double* yt, const double* rij,
-                      const int* ti, const int* tj, const int* pair_off, double* dedr, int natoms, hipStream_t st);
+                      const int* ti, const int* tj, const int* pair_off, const int* pair_end, double* dedr, int natoms,
+                      hipStream_t st);
 // Variants of the MD path's dE/dr (0: all three components per lane; 2, 3, 4: one component per lane
 // with at least that many waves per SIMD; 5: launch_dedr_atom; 6, 7: variant 2 with 2 or 4 waves per
 // workgroup on consecutive pair tiles; 8, 9: lane = pair, derivatives from U through the SU(2)

@@ -74,3 +74,68 @@ def test_small_box_lists_vs_bruteforce(oracle, cells):
         a = sorted(zip(nj[off[i]:off[i + 1]].tolist(), map(tuple, ns[off[i]:off[i + 1]].tolist())))
         b = sorted(zip(j2[o2[i]:o2[i + 1]].tolist(), map(tuple, s2[o2[i]:o2[i + 1]].tolist())))
         assert a == b, i
+
+
+@pytest.mark.parametrize("n,J,types,zbl", [(5, 4, 1, True), (250, 6, 2, False), (16000, 2, 1, False), (18522, 2, 2, False),
+                                           (18522, 2, 1, True)])
+def test_pair_list_blocks_vs_oracle(oracle, n, J, types, zbl):
+    """The pair list in blocks of 16 atoms (up to 16,384) and of 64, with gaps at the blocks' ends: pair count,
+    energies, forces and virials, also with two types and the ZBL term."""
+    from conftest import relerr
+    from mdp_amd import snapcpp
+    from mdp_amd.md import SnapMD
+    if n == 5:
+        x, box = lattice.crystal("bcc", 2, 3.316, 0.1, 3)
+        x = np.ascontiguousarray(x[:5])
+    else:
+        x, box = lattice.crystal("bcc", round((n / 2) ** (1 / 3)), 3.316, 0.1, 3) if n != 250 else _atoms(250, 9)
+    n = len(x)
+    ty = np.random.default_rng(2).integers(1, types + 1, n).astype(np.int32)
+    rad, wt = [0.5, 0.48][:types], [1.0, 0.9][:types]
+    param = [types, J, RCUTFAC, 0.99363, 0, 1, 1, 0, 0, 0, 0]
+    coeff = np.tile(_coeff(oracle, J, 4), types)
+    md = SnapMD(x, box, ty, J, coeff, rad, wt, [180.95] * types)
+    s = snapcpp.initsna(oracle, param, rad, wt, coeff)
+    B = np.diag(box)
+    p = snapcpp.pairs_from_box(x, ty, B[0], B[1], B[2], [1, 1, 1], s)
+    e, f, w = snapcpp.snappotential_pairs(oracle, s, p)
+    if zbl:
+        import zbl_oracle
+        md.set_zbl()
+        g, d, v = zbl_oracle.bind(oracle.cdll)
+        z = snapcpp.initsna(oracle, [1, 2, 4.8, 0.99363, 0, 1, 1, 0, 0, 0, 0], [0.5], [1.0])
+        q = snapcpp.pairs_from_box(x, np.ones(n, np.int32), B[0], B[1], B[2], [1, 1, 1], z)   # all pairs within 4.8 A
+        P, rij, ai = q["ijnum"], np.ascontiguousarray(q["rij"].ravel()), np.ascontiguousarray(q["ai"], np.int32)
+        u, ux, ez, fz, wz = np.zeros(P), np.zeros(3 * P), np.zeros(n), np.zeros(3 * n), np.zeros(6 * n)
+        g(u, ux, rij, zbl_oracle.TA_MU, P)
+        d(ez, fz, u, ux, ai, P, 3)
+        v(wz, ux, rij, -0.5, ai, 3, n, P)
+        e, f, w = e + ez, f - fz.reshape(n, 3), w + wz.reshape(6, n).T
+    md.compute()
+    st = md.state()
+    assert md.stats()["pairs"] == p["ijnum"]
+    assert relerr(st["eatom"], e) < 1e-10
+    assert relerr(st["f"], f) < 1e-10
+    assert relerr(st["vatom"], w) < 1e-10
+
+
+@pytest.mark.parametrize("n", [128, 9826])
+@pytest.mark.parametrize("nvt", [False, True])
+def test_steps_one_by_one_and_in_a_run(oracle, n, nvt):
+    """Twelve steps in one run, where a step's first half goes with the end of the step before, against twelve runs of
+    one step, where it is a launch of its own: the same arithmetic, so to rounding of the last place along the
+    trajectory.  9,826 atoms are above the one-workgroup thermostat."""
+    x, box = lattice.crystal("bcc", round((n / 2) ** (1 / 3)), 3.316, 0.05, 8)
+    v = lattice.maxwell_boltzmann(len(x), 180.95, 300.0, seed=4)
+    out = []
+    for chunks in ([12], [1] * 12):
+        md = _engine(x, box, 2, _coeff(oracle, 2, 3), v=v)
+        if nvt:
+            md.set_nvt(300.0, 500.0, 0.05, endstep=50, mtchain=4, nc_tchain=2)
+        md.compute()
+        for c in chunks:
+            md.run(c)
+        st = md.state()
+        out.append([st[k] for k in ("x", "v", "f", "eatom", "vatom")] + ([np.concatenate([np.ravel(a) for a in md.nvt_state().values()])] if nvt else []))
+    for a, b in zip(*out):
+        assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
