@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <numeric>
 #include <vector>
@@ -243,7 +244,11 @@ void cpuSnapComputeUi(double* Utotr, double* Utoti, double* rootpqarray, double*
         int* d_tj = put(4, tj, ijnum, st);
         int* d_off = put(5, off.data(), off.size(), st);
         int* d_perm = perm.empty() ? nullptr : put(6, perm.data(), perm.size(), st);
-        if (!chemflag) {
+        if (!chemflag && perm.empty()) {   // pairs sorted by centre atom: their geometry once, then lanes sharing atoms
+            double* d_geo = dev<double>(7, 5 * static_cast<size_t>(ijnum));
+            launch_pair_geo(s, d_rij, d_ti, d_tj, nullptr, ijnum, d_geo, st);
+            launch_ui_acc_geo(s, d_ur, d_ui, d_geo, d_off, inum, st);
+        } else if (!chemflag) {
             launch_ui(s, UI_ACCUMULATE, d_ur, d_ui, d_rij, d_off, d_perm, d_ti, d_tj, inum, 0.0, -1, st);
         } else {
             for (int e = 0; e < nelem; ++e) {
@@ -278,9 +283,33 @@ void cpuAddWself2Ui(double* Utotr, double* Utoti, double wself, int* idxu_block,
 }
 
 namespace {
+// Whether a caller's Clebsch-Gordan table is the library's own (to rounding): the LDS-staged kernels carry the
+// coefficients of one direction as compile-time constants.  Any other table goes through the general kernels.
+bool own_cg(const double* cg, const SnapIndex& ix) {
+    for (int k = 0; k < ix.idxcg_max; ++k)
+        if (!(std::abs(cg[k] - ix.cglist[k]) <= 1e-14)) return false;
+    return true;
+}
+
+// The LDS-staged kernels read the half rows of U only: what they serve is a U whose other rows are the mirror images that
+// AddWself2Ui writes.  An array a caller filled otherwise goes through the general kernels, which read all of it.
+bool own_mirror(const SnapDev& s, const double* d_ur, const double* d_ui, int inum, hipStream_t st) {
+    int* d = dev<int>(39, 1);
+    int differs = 1;
+    MDP_HIP(hipMemsetAsync(d, 0, sizeof(int), st));
+    launch_mirror_differs(s, d_ur, d_ui, d, inum, st);
+    get(&differs, d, 1, st);
+    MDP_HIP(hipStreamSynchronize(st));
+    return !differs;
+}
+
 // blist for all element triples (layout ii + N*jjb + N*idxb_max*jelem), before bzero
 void all_triples_b(const SnapDev& s, const double* d_ur, const double* d_ui, double* d_b, int nelem, int inum, int bnorm,
-                   hipStream_t st) {
+                   bool cg_own, hipStream_t st) {
+    if (nelem == 1 && cg_own && own_mirror(s, d_ur, d_ui, inum, st)) {
+        launch_b_full(s, d_ur, d_ui, d_b, inum, bnorm, st);
+        return;
+    }
     const long nu = static_cast<long>(inum) * s.idxu_max;
     for (int e1 = 0; e1 < nelem; ++e1)
         for (int e2 = 0; e2 < nelem; ++e2)
@@ -314,7 +343,7 @@ void cpuSnapComputeEi(double* eatom, double* Utotr, double* Utoti, double* cglis
         int* d_t = put(5, type, inum, st);
         double* d_e = put_arg(6, eatom, eext, st);
         double* d_b = dev<double>(7, static_cast<size_t>(inum) * idxb_max * ne * ne * ne);
-        all_triples_b(s, d_ur, d_ui, d_b, ne, inum, bnorm_flag, st);
+        all_triples_b(s, d_ur, d_ui, d_b, ne, inum, bnorm_flag, own_cg(cglist, index_for(twojmax)), st);
         if (bzero_flag) launch_bzero(s, d_b, d_bz, d_il, d_t, wselfall_flag, chemflag, ne, inum, 0, st);
         launch_ei_from_b(s, d_e, d_b, d_c, d_il, d_t, chemflag, ne, ncoeffall, inum, st);
         get_arg(eatom, d_e, eext, st);
@@ -338,7 +367,7 @@ void cpuSnapComputeBi(double* blist, double* Utotr, double* Utoti, double* cglis
         double* d_ui = put(1, Utoti, nu, st);
         double* d_bz = put(2, bzero, twojmax + 1, st);
         double* d_b = dev<double>(3, nb);
-        all_triples_b(s, d_ur, d_ui, d_b, ne, inum, bnorm_flag, st);
+        all_triples_b(s, d_ur, d_ui, d_b, ne, inum, bnorm_flag, own_cg(cglist, index_for(twojmax)), st);
         if (bzero_flag) launch_bzero(s, d_b, d_bz, nullptr, nullptr, wselfall_flag, 0, ne, inum, 0, st);
         get(blist, d_b, nb, st);
         finish(st);
@@ -365,7 +394,18 @@ void cpuSnapComputeYi(double* ylist_r, double* ylist_i, double* Utotr, double* U
         double* d_yi = out_arg(3, ylist_i, nu);
         MDP_HIP(hipMemsetAsync(d_yr, 0, sizeof(double) * nu, st));
         MDP_HIP(hipMemsetAsync(d_yi, 0, sizeof(double) * nu, st));
-        if (ne == 1 && !chemflag) {
+        // one element block for every atom: the LDS-staged kernels when coupling table and U are as the library makes them
+        bool one = ne == 1;
+        for (int i = 0; one && chemflag && i < inum; ++i) one = map[type[i]] == 0;
+        if (one && own_cg(cglist, ix) && own_mirror(s, d_ur, d_ui, inum, st)) {
+            std::vector<double> bt = y_beta_table(ix, beta, 0, 0, 0, 1, 0, ncoeffall, bnorm_flag);
+            std::vector<int> order((twojmax / 2 + 1) * (twojmax + 1));
+            yi_row_order(twojmax, order.data());
+            double* d_bt = put(4, bt.data(), bt.size(), st);
+            int* d_ord = put(5, order.data(), order.size(), st);
+            launch_yi_full(s, d_ur, d_ui, d_bt, d_yr, d_yi, d_ord, inum, st);
+            MDP_HIP(hipStreamSynchronize(st));
+        } else if (ne == 1 && !chemflag) {
             std::vector<double> bt = y_beta_table(ix, beta, 0, 0, 0, 1, 0, ncoeffall, bnorm_flag);
             double* d_bt = put(4, bt.data(), bt.size(), st);
             launch_yi(s, d_ur, d_ui, d_bt, d_yr, d_yi, nullptr, inum, true, st);
@@ -696,7 +736,7 @@ void cpuSnapTallyBispectrumVirial(double* bv, double* bispectrum, double* dbdr, 
             double* d_rij = put_arg(3, rij, 3 * static_cast<size_t>(ijnum), st);
             int* d_aii = put(4, aii, ijnum, st);
             int* d_ti = put(5, ti, ijnum, st);
-            launch_tally_bv(d_bv, d_b, d_dbdr, d_rij, d_aii, d_ti, inum, ijnum, ncoeff, nperdim, quadraticflag, st);
+            launch_tally_bv(d_bv, d_b, d_dbdr, d_rij, d_aii, d_ti, inum, ijnum, ncoeff, nperdim, ntype, quadraticflag, st);
         }
         get_arg(bv, d_bv, nbv, st);
         finish(st);

@@ -80,7 +80,9 @@ void launch_bi(const SnapDev& s, const double* Ur, const double* Ui, long off1, 
 #undef BI_CASE
 }
 
-// Z of one coupling triple (blockIdx.y), all rows mb and columns ma, into Z[jjz*N + atom]
+// Z of one row mb (blockIdx.z) of one coupling triple (blockIdx.y), all columns ma, into Z[jjz*N + atom].  A row per
+// wave: with all rows of a triple on one wave the heaviest triple's chain set the time of a small system (54 atoms,
+// twojmax 8: 133 us; 106 so).
 template <int J>
 __global__ __launch_bounds__(64) void k_zi(SnapDev s, const double* __restrict__ Ur, const double* __restrict__ Ui,
                                            long off1, long off2, double* __restrict__ Zr, double* __restrict__ Zi,
@@ -99,7 +101,8 @@ __global__ __launch_bounds__(64) void k_zi(SnapDev s, const double* __restrict__
                     if (t == triple_id(J, J1, J2, JO)) {
                         const int zb = s.idxz_block[JO + J2 * (J + 1) + J1 * (J + 1) * (J + 1)];
                         const double scale = bnorm ? 1.0 / (JO + 1) : 1.0;
-                        for (int mb = 0; 2 * mb <= JO; ++mb) {
+                        const int mb = blockIdx.z;
+                        if (2 * mb <= JO) {
                             double zr[JO + 1], zi[JO + 1];
 #pragma unroll
                             for (int m = 0; m <= JO; ++m) { zr[m] = 0.0; zi[m] = 0.0; }
@@ -127,7 +130,7 @@ void launch_zi(const SnapDev& s, const double* Ur, const double* Ui, long off1, 
         case 8: nt = n_triples(8); break;
         default: return;
     }
-    dim3 grid((N + 63) / 64, nt);
+    dim3 grid((N + 63) / 64, nt, s.J / 2 + 1);
 #define ZI_CASE(JV) \
     case JV: hipLaunchKernelGGL((k_zi<JV>), grid, dim3(64), 0, st, s, Ur, Ui, off1, off2, Zr, Zi, N, bnorm); break;
     switch (s.J) {

@@ -40,7 +40,7 @@ __device__ __forceinline__ double sub_sum(double v) {
 // GEO: the pair's Cayley-Klein parameters and weighted switching factor come precomputed from
 // pgeo[5q..5q+4] = (a_r, a_i, b_r, b_i, sfac * w_j) (the MD pair list writes them once per step with the
 // same pair_geometry), instead of being derived here from r_ij in every row group.
-// SUB > 1 (with GEO, UI_HALF_WSELF): SUB adjacent lanes share an atom and take every SUB-th of its pairs, so that a
+// SUB > 1 (with GEO): SUB adjacent lanes share an atom and take every SUB-th of its pairs, so that a
 // small system puts SUB times as many waves on the chip and each walks a SUB-th of the serial chain of pairs; the
 // partial sums are added across the lanes at the end and lane k % SUB stores element k.
 template <int J, int RLO, int RHI, int MODE, bool GEO = false, int SUB = 1>
@@ -49,7 +49,7 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
                                         const int* __restrict__ pair_end, const int* __restrict__ perm, const int* __restrict__ ti,
                                         const int* __restrict__ tj, int N, double wself, int elem_sel, int atom,
                                         const double* __restrict__ pgeo = nullptr, int sub = 0) {
-    static_assert(SUB == 1 || (GEO && MODE == UI_HALF_WSELF), "lanes share an atom in the MD and fitting form only");
+    static_assert(SUB == 1 || (GEO && MODE != UI_FULL_WSELF), "lanes share an atom only where pgeo gives the pairs");
     constexpr int NE = rows_elems(J, RLO, RHI);
     double accr[NE], acci[NE];
 #pragma unroll
@@ -128,6 +128,7 @@ __device__ __forceinline__ void ui_rows(const SnapDev& s, double* __restrict__ U
             for (int ma = 0; ma <= JJ; ++ma) {
                 const size_t o = static_cast<size_t>(row + ma) * n + atom;
                 if constexpr (MODE == UI_ACCUMULATE) {
+                    if (SUB > 1 && sub != (base + ma) % SUB) continue;
                     Ur[o] += accr[base + ma];
                     Ui[o] += acci[base + ma];
                 } else if constexpr (MODE == UI_HALF_WSELF) {
@@ -221,9 +222,10 @@ void launch_ui(const SnapDev& s, UiMode mode, double* Ur, double* Ui, const doub
 // pairs of a list whose length is on the device (np_dev): one lane per pair.
 __global__ __launch_bounds__(256) void k_pair_geo(SnapDev s, const double* __restrict__ rij,
                                                   const int* __restrict__ ti, const int* __restrict__ tj,
-                                                  const int* __restrict__ np_dev, double* __restrict__ pgeo) {
+                                                  const int* __restrict__ np_dev, int cap,
+                                                  double* __restrict__ pgeo) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= *np_dev) return;
+    if (q >= (np_dev ? *np_dev : cap)) return;
     const int tjq = tj[q];
     PairGeom g;
     pair_geometry<false>(rij[3 * static_cast<size_t>(q)], rij[3 * static_cast<size_t>(q) + 1],
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(256) void k_pair_geo(SnapDev s, const double* __res
 void launch_pair_geo(const SnapDev& s, const double* rij, const int* ti, const int* tj, const int* np_dev, int cap,
                      double* pgeo, hipStream_t st) {
     if (cap <= 0) return;
-    hipLaunchKernelGGL(k_pair_geo, dim3((cap + 255) / 256), dim3(256), 0, st, s, rij, ti, tj, np_dev, pgeo);
+    hipLaunchKernelGGL(k_pair_geo, dim3((cap + 255) / 256), dim3(256), 0, st, s, rij, ti, tj, np_dev, cap, pgeo);
 }
 
 // compute_ui with the per-atom sums in LDS (half layout plus wself, from the pair geometry pgeo).  Lanes are pairs.
@@ -369,6 +371,33 @@ void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo,
     }
 #undef UG_CASE
 #undef UG
+}
+
+void launch_ui_acc_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int N,
+                       hipStream_t st) {
+    if (N <= 0) return;
+    const int lanes = ui_lanes_per_atom(s.J, N);
+#define UA(JV, SUBV)                                                                                                  \
+    ui_groups<JV, UI_ACCUMULATE, true, SUBV>(s, Ur, Ui, nullptr, pair_off, pair_off + 1, nullptr, nullptr, nullptr, N, \
+                                             0.0, -1, st, pgeo)
+#define UA_CASE(JV)         \
+    case JV:                \
+        if (lanes == 16)    \
+            UA(JV, 16);     \
+        else if (lanes == 4) \
+            UA(JV, 4);      \
+        else                \
+            UA(JV, 1);      \
+        break;
+    switch (s.J) {
+        UA_CASE(2)
+        UA_CASE(4)
+        UA_CASE(6)
+        UA_CASE(8)
+        default: break;
+    }
+#undef UA_CASE
+#undef UA
 }
 
 }  // namespace mdp

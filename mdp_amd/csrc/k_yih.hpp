@@ -203,12 +203,12 @@ __device__ __forceinline__ void y_couplings_shared_a(int mb, int malim, const do
 // complex-interleaved LDS layout; SYM: the swap symmetry of the (J1, J1) couplings; UNI: 1 makes the
 // shared-row loop's row index wave-uniform explicitly (140 instead of 166 VGPRs at twojmax 8, the row tests
 // become scalar branches), 2 also the output row's (j, mb), which costs spills.
-template <int J, int JO, bool PA = false, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0>
+template <int J, int JO, bool PA = false, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0, bool FULL = false>
 __device__ __forceinline__ void y_row_lds(const double* __restrict__ cg, int row, int mb, int atom, bool live, int N,
                                           const double* __restrict__ lr, const double* __restrict__ li, int lane,
                                           const double* __restrict__ beta_t, double* __restrict__ Yr,
                                           double* __restrict__ Yi, double* __restrict__ epart) {
-    const int malim = (2 * mb == JO) ? mb : JO;
+    const int malim = (!FULL && 2 * mb == JO) ? mb : JO;
     const size_t n = static_cast<size_t>(N);
     double yr[JO + 1], yi[JO + 1];
 #pragma unroll
@@ -231,13 +231,14 @@ __device__ __forceinline__ void y_row_lds(const double* __restrict__ cg, int row
     }
     if (!live) return;
     const int hrow = h_block(JO) + (JO + 1) * mb;
-    const size_t o = static_cast<size_t>(hrow) * n + atom;
+    const size_t o = static_cast<size_t>(FULL ? u_block(JO) + (JO + 1) * mb : hrow) * n + atom;
     double e = 0.0;
 #pragma unroll
     for (int ma = 0; ma <= JO; ++ma) {
         if (ma <= malim) {
             Yr[o + ma * n] = yr[ma];
             Yi[o + ma * n] = yi[ma];
+            if constexpr (FULL) continue;
             const double w = (2 * mb < JO || ma < mb) ? 1.0 : 0.5;
             if constexpr (CX) {
                 const double2 u = reinterpret_cast<const double2*>(lr)[(hrow + ma) * 64 + lane];
@@ -247,12 +248,22 @@ __device__ __forceinline__ void y_row_lds(const double* __restrict__ cg, int row
             }
         }
     }
-    if constexpr (!PA) epart[static_cast<size_t>(row) * n + atom] = e;
+    if constexpr (!PA && !FULL) epart[static_cast<size_t>(row) * n + atom] = e;
+}
+
+// FULL: U and Y in the upstream layout (element (j, mb, ma) at u_block(j) + (j + 1) mb + ma) instead of the half
+// layout; of U the half rows are read, of Y they are written, the middle row of even layers to its end.  The half rows
+// of a layer come first in either layout.
+template <int J>
+__device__ __forceinline__ int full_element(int e) {
+    int j = 0;
+    while (e >= h_block(j + 1)) ++j;
+    return u_block(j) + e - h_block(j);
 }
 
 // The coefficient tables (cg, beta_t, order) are separate read-only, non-aliased kernel arguments so
 // that their wave-uniform loads go through the scalar cache into SGPRs.
-template <int J, int W, bool PA = false, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0>
+template <int J, int W, bool PA = false, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0, bool FULL = false>
 __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ cg, const double* __restrict__ Ur,
                                                     const double* __restrict__ Ui, const double* __restrict__ beta_t,
                                                     double* __restrict__ Yr, double* __restrict__ Yi,
@@ -269,8 +280,9 @@ __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ c
     const size_t n = static_cast<size_t>(N);
     if (threadIdx.x == 0) next_row = 0;
     for (int e = wave; e < HE; e += W) {
-        const double ur = live ? Ur[static_cast<size_t>(e) * n + atom] : 0.0;
-        const double ui = live ? Ui[static_cast<size_t>(e) * n + atom] : 0.0;
+        const size_t g = static_cast<size_t>(FULL ? full_element<J>(e) : e) * n + atom;
+        const double ur = live ? Ur[g] : 0.0;
+        const double ui = live ? Ui[g] : 0.0;
         if constexpr (CX) {
             reinterpret_cast<double2*>(lbuf)[e * 64 + lane] = make_double2(ur, ui);
         } else {
@@ -291,7 +303,7 @@ __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ c
         static_for<0, J + 1>([&](auto JOc) {
             constexpr int JO = decltype(JOc)::value;
             if (jo == JO)
-                y_row_lds<J, JO, PA, SA, CX, SYM, UNI>(cg, row, mb, atom, live, N, lr, li, lane, beta_t, Yr, Yi,
+                y_row_lds<J, JO, PA, SA, CX, SYM, UNI, FULL>(cg, row, mb, atom, live, N, lr, li, lane, beta_t, Yr, Yi,
                                                       epart);
         });
     }
@@ -310,7 +322,7 @@ constexpr int yi_rows_lds() {   // doubles: the staged U, or the partial rows an
     return 2 * n_half_elems(J) * 64 > (2 * (J + 1) + 1) * W * 64 ? 2 * n_half_elems(J) * 64 : (2 * (J + 1) + 1) * W * 64;
 }
 
-template <int J, int W>
+template <int J, int W, bool FULL = false>
 __global__ __launch_bounds__(64 * W) void k_yi_rows(const double* __restrict__ cg, const double* __restrict__ Ur,
                                                     const double* __restrict__ Ui, const double* __restrict__ beta_t,
                                                     double* __restrict__ Yr, double* __restrict__ Yi,
@@ -325,17 +337,18 @@ __global__ __launch_bounds__(64 * W) void k_yi_rows(const double* __restrict__ c
     const bool live = atom < N;
     const size_t n = static_cast<size_t>(N);
     double2* const lc = reinterpret_cast<double2*>(lbuf);
-    for (int e = wave; e < HE; e += W)
-        lc[e * 64 + lane] = live ? make_double2(Ur[static_cast<size_t>(e) * n + atom], Ui[static_cast<size_t>(e) * n + atom])
-                                 : make_double2(0.0, 0.0);
+    for (int e = wave; e < HE; e += W) {
+        const size_t g = static_cast<size_t>(FULL ? full_element<J>(e) : e) * n + atom;
+        lc[e * 64 + lane] = live ? make_double2(Ur[g], Ui[g]) : make_double2(0.0, 0.0);
+    }
     __syncthreads();
     const int jo = half_row_j(row), mb = half_row_mb(row);
     static_for<0, J + 1>([&](auto JOc) {
         constexpr int JO = decltype(JOc)::value;
         if (jo == JO) {   // uniform over the workgroup
             constexpr int PER = (JO + W) / W;   // elements of the row that a wave finishes: ma = wave + W h
-            const int malim = (2 * mb == JO) ? mb : JO;
-            const int hrow = h_block(JO) + (JO + 1) * mb;
+            const int malim = (!FULL && 2 * mb == JO) ? mb : JO;
+            const int hrow = h_block(JO) + (JO + 1) * mb, orow = FULL ? u_block(JO) + (JO + 1) * mb : hrow;
             double yr[JO + 1], yi[JO + 1];
 #pragma unroll
             for (int m = 0; m <= JO; ++m) { yr[m] = 0.0; yi[m] = 0.0; }
@@ -360,13 +373,14 @@ __global__ __launch_bounds__(64 * W) void k_yi_rows(const double* __restrict__ c
                         y.y += p.y;
                     }
                     if (live) {
-                        Yr[static_cast<size_t>(hrow + ma) * n + atom] = y.x;
-                        Yi[static_cast<size_t>(hrow + ma) * n + atom] = y.y;
+                        Yr[static_cast<size_t>(orow + ma) * n + atom] = y.x;
+                        Yi[static_cast<size_t>(orow + ma) * n + atom] = y.y;
                     }
                     const double wt = (2 * mb < JO || ma < mb) ? 1.0 : 0.5;
                     e += wt * (u[h].x * y.x + u[h].y * y.y);
                 }
             }
+            if constexpr (FULL) return;   // no energy partials
             double* const es = lbuf + 2 * (J + 1) * W * 64;
             es[wave * 64 + lane] = e;
             __syncthreads();
@@ -380,35 +394,37 @@ __global__ __launch_bounds__(64 * W) void k_yi_rows(const double* __restrict__ c
     });
 }
 
-template <int J, int W>
+template <int J, int W, bool FULL = false>
 void launch_yi_rows(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
                     double* epart, const int* order, int N, hipStream_t st) {
     const int blocks = ((N + 63) / 64 + 7) / 8 * 8;   // whole XCD rounds; workgroups past the last block return
-    hipLaunchKernelGGL((k_yi_rows<J, W>), dim3(blocks * n_half_rows(J)), dim3(64 * W), 0, st, s.cg, Ur, Ui, beta_t, Yr, Yi,
+    hipLaunchKernelGGL((k_yi_rows<J, W, FULL>), dim3(blocks * n_half_rows(J)), dim3(64 * W), 0, st, s.cg, Ur, Ui, beta_t, Yr, Yi,
                        epart, order, N);
 }
 
 // B of every bispectrum triple (j >= j1) from the half U of 64 atoms staged in LDS, as k_yi_half stages
 // it: B = 2 sum' U*(j).Z(j1,j2,j) (cpuSnap.cpp:1899-2072 semantics, no bzero subtraction), Z rows from
 // z_row_lds, the middle column of even layers weighted 1/2.  Waves take whole triples from a shared
-// counter; blist[jjb * N + atom].
-template <int J, int W, bool CX = true>
+// counter; blist[jjb * N + atom].  `groups` workgroups share a block's triples (every groups-th each, the last and
+// heaviest first), so that a few blocks still reach many CUs.
+template <int J, int W, bool CX = true, bool FULL = false>
 __global__ __launch_bounds__(64 * W) void k_b_half(const double* __restrict__ cg, const double* __restrict__ Ur,
                                                    const double* __restrict__ Ui, double* __restrict__ blist, int N,
-                                                   int bnorm) {
+                                                   int bnorm, int groups) {
     constexpr int HE = n_half_elems(J), NB = n_bisp(J);
     __shared__ double lbuf[2 * HE * 64];   // lr | li, or (re, im) pairs under CX
     double* const lr = lbuf;
     double* const li = CX ? nullptr : lbuf + HE * 64;
     __shared__ int next_task;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int atom = blockIdx.x * 64 + lane;
+    const int atom = static_cast<int>(blockIdx.x) / groups * 64 + lane, group = static_cast<int>(blockIdx.x) % groups;
     const bool live = atom < N;
     const size_t n = static_cast<size_t>(N);
     if (threadIdx.x == 0) next_task = 0;
     for (int e = wave; e < HE; e += W) {
-        const double ur = live ? Ur[static_cast<size_t>(e) * n + atom] : 0.0;
-        const double ui = live ? Ui[static_cast<size_t>(e) * n + atom] : 0.0;
+        const size_t g = static_cast<size_t>(FULL ? full_element<J>(e) : e) * n + atom;
+        const double ur = live ? Ur[g] : 0.0;
+        const double ui = live ? Ui[g] : 0.0;
         if constexpr (CX) {
             reinterpret_cast<double2*>(lbuf)[e * 64 + lane] = make_double2(ur, ui);
         } else {
@@ -420,8 +436,8 @@ __global__ __launch_bounds__(64 * W) void k_b_half(const double* __restrict__ cg
     for (;;) {
         int t = 0;
         if (lane == 0) t = atomicAdd(&next_task, 1);
-        t = __builtin_amdgcn_readfirstlane(__shfl(t, 0));
-        if (t >= NB) break;
+        t = NB - 1 - group - groups * __builtin_amdgcn_readfirstlane(__shfl(t, 0));
+        if (t < 0) break;
         static_for<0, J + 1>([&](auto J1c) {
             constexpr int J1 = decltype(J1c)::value;
             static_for<0, J1 + 1>([&](auto J2c) {

@@ -41,8 +41,8 @@ bool launch_b_half(const SnapDev& s, const double* Ur, const double* Ui, double*
     if (N <= 0) return true;
     const dim3 grid((N + 63) / 64), block(64 * 4);
     switch (s.J) {
-        case 2: hipLaunchKernelGGL((k_b_half<2, 4>), grid, block, 0, st, s.cg, Ur, Ui, blist, N, bnorm); return true;
-        case 4: hipLaunchKernelGGL((k_b_half<4, 4>), grid, block, 0, st, s.cg, Ur, Ui, blist, N, bnorm); return true;
+        case 2: hipLaunchKernelGGL((k_b_half<2, 4>), grid, block, 0, st, s.cg, Ur, Ui, blist, N, bnorm, 1); return true;
+        case 4: hipLaunchKernelGGL((k_b_half<4, 4>), grid, block, 0, st, s.cg, Ur, Ui, blist, N, bnorm, 1); return true;
         default: return false;
     }
 }

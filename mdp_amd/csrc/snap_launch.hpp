@@ -45,7 +45,11 @@ void launch_ui(const SnapDev& s, UiMode mode, double* Ur, double* Ui, const doub
 void launch_ui_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off,
                    const int* pair_end, int natoms, double wself, hipStream_t st, int lanes = 0);
 int ui_lanes_per_atom(int J, int natoms);
-// pgeo[5q..5q+4] = (a_r, a_i, b_r, b_i, sfac w_j) of every pair q < *np_dev (cap: the launch's pair capacity)
+// cpuSnapComputeUi's accumulation (UI_ACCUMULATE) from the pair geometry, one element, pairs sorted by centre atom
+void launch_ui_acc_geo(const SnapDev& s, double* Ur, double* Ui, const double* pgeo, const int* pair_off, int natoms,
+                       hipStream_t st);
+// pgeo[5q..5q+4] = (a_r, a_i, b_r, b_i, sfac w_j) of every pair q < *np_dev (cap: the launch's pair capacity; all of
+// them when np_dev is null)
 void launch_pair_geo(const SnapDev& s, const double* rij, const int* ti, const int* tj, const int* np_dev, int cap,
                      double* pgeo, hipStream_t st);
 // The same result with the per-atom sums formed in LDS, one lane per pair (at most 96 pairs per atom, the pairs of
@@ -85,6 +89,15 @@ void yi_row_order(int J, int* out);
 bool launch_yi_half_pa(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_pa, double* Yr,
                        double* Yi, const int* order, int N, hipStream_t st);
 bool launch_b_half(const SnapDev& s, const double* Ur, const double* Ui, double* blist, int N, int bnorm,
+                   hipStream_t st);
+
+// Y and B of one element block from a full-layout U, through the LDS-staged kernels of the MD path: the half rows of Y
+// (every ma, also behind the middle of an even layer; Y zeroed by the caller elsewhere) and every B before bzero.
+// The ma-direction Clebsch-Gordan coefficients are compile-time constants: for callers whose table is the library's.
+// order = yi_row_order(J).
+void launch_yi_full(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
+                    const int* order, int N, hipStream_t st);
+void launch_b_full(const SnapDev& s, const double* Ur, const double* Ui, double* blist, int N, int bnorm,
                    hipStream_t st);
 
 // B of the idxb triples: blist[ii + N*jjb] = 2 sum' U*(j).Z(j1,j2,j)  (before bzero; Z/(j+1) if bnorm).
@@ -193,7 +206,7 @@ void launch_tally_bd(double* db, const double* b, const double* dbdr, const int*
                      const int* aj, const int* ti, int inum, int ijnum, int ncoeff, int nperdim, int quadratic,
                      hipStream_t st);
 void launch_tally_bv(double* bv, const double* b, const double* dbdr, const double* rij, const int* aii,
-                     const int* ti, int inum, int ijnum, int ncoeff, int nperdim, int quadratic, hipStream_t st);
+                     const int* ti, int inum, int ijnum, int ncoeff, int nperdim, int ntype, int quadratic, hipStream_t st);
 
 // fatom[3*ai] += dE, fatom[3*aj] -= dE, vatom[6*ai + (xx,yy,zz,xy,xz,yz)] += -r (x) dE  (atomic)
 void launch_tally_force_atomic(double* fatom, double* vatom, const double* dedr, const double* rij, const int* ai,
@@ -243,6 +256,8 @@ void launch_tally_virial_full(double* vatom, const double* fij, const double* ri
 // AddWself2Ui on device (wself on the diagonal, mirror of rows 2mb < j)
 void launch_add_wself(const SnapDev& s, double* Ur, double* Ui, double wself, const int* type, int wselfall,
                       int chemflag, int nelem, int inum, hipStream_t st);
+// *differs = 1 where U (one element) is not its own mirror image, as AddWself2Ui leaves it
+void launch_mirror_differs(const SnapDev& s, const double* Ur, const double* Ui, int* differs, int N, hipStream_t st);
 
 // generic compute_yi accumulate for element blocks: Y[e3] += sum beta_t(e1,e2,e3,ielem) Z(e1,e2) over
 // the atoms whose element (map[type[ii]]) equals isel (all atoms if isel < 0); per_atom: beta_t[triple*N + atom]
