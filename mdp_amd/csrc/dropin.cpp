@@ -775,6 +775,28 @@ bool fetch_args(F&& f) {
     });
     return ok;
 }
+// max, min and order of device-resident index arrays, in one read-back (see launch_index_range)
+struct IndexRange {
+    int max, neg_min, drop;
+};
+template <size_t K>
+void index_ranges(const int* const (&a)[K], int n, IndexRange (&r)[K], hipStream_t st) {
+    int* d = dev<int>(38, 3 * K);
+    MDP_HIP(hipMemsetAsync(d, 0x80, sizeof(int) * 3 * K, st));
+    for (size_t k = 0; k < K; ++k) launch_index_range(a[k], n, d + 3 * k, st);
+    get(reinterpret_cast<int*>(r), d, 3 * K, st);
+    MDP_HIP(hipStreamSynchronize(st));
+}
+// the library's tables of J with the caller's device-resident numeric tables in their place
+SnapDev device_tables(int J, const double* rootpq, const double* radelem, const double* wjelem, const int* map,
+                      hipStream_t st) {
+    SnapDev s = tables(J, nullptr, nullptr, nullptr, nullptr, nullptr, 1, st);
+    if (rootpq) s.rootpq = rootpq;
+    if (radelem) s.radelem = radelem;
+    if (wjelem) s.wjelem = wjelem;
+    if (map) s.map = map;
+    return s;
+}
 int max_type(const std::vector<int>& a, size_t n) { return std::max(1, max_of(a.data(), static_cast<long>(n), 1)); }
 }  // namespace
 
@@ -785,6 +807,38 @@ void mdp_hipSnapComputeUi(double* Stotr, double* Stoti, double* rootpqarray, dou
                           double* radelem, double rmin0, double rfac0, double rcutfac, int* idxu_block, int* map, int* ai,
                           int* ti, int* tj, int twojmax, int idxu_max, int inum, int ijnum, int switchflag, int chemflag) {
     (void)idxu_block;
+    // one element and pairs in the order of their centre atoms: everything stays on the device
+    bool done = false, sorted = true;
+    if (!fetch_args([&] {
+            if (chemflag) return;
+            if (inum <= 0) {
+                done = true;
+                return;
+            }
+            hipStream_t st = library_stream();
+            SnapDev s = device_tables(twojmax, rootpqarray, radelem, wjelem, map, st);
+            if (idxu_max != s.idxu_max) throw Error("idxu_max does not match twojmax");
+            s.rcutfac = rcutfac;
+            s.rfac0 = rfac0;
+            s.rmin0 = rmin0;
+            s.switchflag = switchflag;
+            if (ijnum > 0) {
+                const int* const arr[1] = {ai};
+                IndexRange r[1];
+                index_ranges(arr, ijnum, r, st);
+                if (r[0].neg_min > 0 || r[0].max >= inum) throw Error("pair centre index out of range [0, inum)");
+                sorted = r[0].drop <= 0;
+                if (!sorted) return;
+                int* d_off = dev<int>(5, static_cast<size_t>(inum) + 1);
+                double* d_geo = dev<double>(7, 5 * static_cast<size_t>(ijnum));
+                launch_csr_of_sorted(ai, ijnum, d_off, inum, st);
+                launch_pair_geo(s, rij, ti, tj, nullptr, ijnum, d_geo, st);
+                launch_ui_acc_geo(s, Stotr, Stoti, d_geo, d_off, inum, st);
+                finish(st);
+            }
+            done = true;
+        }) || done)
+        return;
     std::vector<int> h_ai, h_ti, h_tj, h_map;
     std::vector<double> h_rp, h_wj, h_rad;
     if (!fetch_args([&] {
@@ -808,6 +862,17 @@ void mdp_hipSnapComputeUi(double* Stotr, double* Stoti, double* rootpqarray, dou
 void mdp_hipAddWself2Ui(double* ulisttot_r, double* ulisttot_i, double wself, int* idxu_block, int* type, int* map,
                         int* ai, int wselfall_flag, int chemflag, int idxu_max, int nelements, int twojmax, int inum) {
     (void)ai;
+    if (!chemflag) {   // types and elements are not read
+        fetch_args([&] {
+            if (inum <= 0) return;
+            hipStream_t st = library_stream();
+            SnapDev s = device_tables(twojmax, nullptr, nullptr, nullptr, map, st);
+            if (idxu_max != s.idxu_max) throw Error("idxu_max does not match twojmax");
+            launch_add_wself(s, ulisttot_r, ulisttot_i, wself, type, wselfall_flag, 0, nelements, inum, st);
+            finish(st);
+        });
+        return;
+    }
     std::vector<int> h_type, h_map;
     if (!fetch_args([&] {
             h_type = fetch(type, static_cast<size_t>(std::max(inum, 0)));
@@ -826,25 +891,22 @@ void mdp_hipSnapComputeEi(double* eatom, double* ulisttot_r, double* ulisttot_i,
                           double* coeffelem, int* ilist, int* map, int* type, int* idxb, int* idxcg_block,
                           int* idxu_block, int twojmax, int idxb_max, int idxu_max, int nelements, int ncoeffall,
                           int bnorm_flag, int bzero_flag, int wselfall_flag, int quadraticflag, int inum) {
-    (void)quadraticflag;
-    std::vector<int> h_il, h_type, h_map;
-    std::vector<double> h_cg, h_bz, h_c;
-    if (!fetch_args([&] {
-            const size_t n = static_cast<size_t>(std::max(inum, 0));
-            h_il = fetch(ilist, n);
-            h_type = fetch(type, n);
-            const int nt = max_type(h_type, n);
-            h_map = fetch(map, nt + 1);
-            const int rows = max_of(h_map.data() + 1, nt, 0) + 1;
-            h_cg = fetch(cglist, static_cast<size_t>(index_for(twojmax).idxcg_max));
-            h_bz = fetch(bzero, twojmax + 1);
-            h_c = fetch(coeffelem, static_cast<size_t>(ncoeffall) * rows);
-        }))
-        return;
-    DevIo io;
-    cpuSnapComputeEi(eatom, ulisttot_r, ulisttot_i, h_cg.data(), h_bz.data(), h_c.data(), h_il.data(), h_map.data(),
-                     h_type.data(), idxb, idxcg_block, idxu_block, twojmax, idxb_max, idxu_max, nelements, ncoeffall,
-                     bnorm_flag, bzero_flag, wselfall_flag, 1, inum);
+    (void)quadraticflag; (void)idxb; (void)idxcg_block; (void)idxu_block;
+    std::vector<double> h_cg;
+    if (!fetch_args([&] { h_cg = fetch(cglist, static_cast<size_t>(index_for(twojmax).idxcg_max)); })) return;
+    guarded([&] {
+        if (inum <= 0) return;
+        hipStream_t st = library_stream();
+        SnapDev s = tables(twojmax, nullptr, h_cg.data(), nullptr, nullptr, nullptr, 1, st);
+        s.map = map;
+        if (idxu_max != s.idxu_max || idxb_max != s.idxb_max) throw Error("table sizes do not match twojmax");
+        const int ne = nelements;
+        double* d_b = dev<double>(7, static_cast<size_t>(inum) * idxb_max * ne * ne * ne);
+        all_triples_b(s, ulisttot_r, ulisttot_i, d_b, ne, inum, bnorm_flag, own_cg(h_cg.data(), index_for(twojmax)), st);
+        if (bzero_flag) launch_bzero(s, d_b, bzero, ilist, type, wselfall_flag, 1, ne, inum, 0, st);
+        launch_ei_from_b(s, eatom, d_b, coeffelem, ilist, type, 1, ne, ncoeffall, inum, st);
+        finish(st);
+    });
 }
 
 // SnapComputeYi backend 3, coefficient form (mdpcore.h:3221-3244; src/C++/Core/cpuSnap4.cpp:697-796):
@@ -945,6 +1007,28 @@ void mdp_hipSnapComputeFi(double* fatom, double* vatom, double* ylist_r, double*
                           int* idxu_block, int* map, int* aii, int* ai, int* aj, int* ti, int* tj, int twojmax,
                           int idxu_max, int inum, int anum, int ijnum, int switchflag, int chemflag) {
     (void)idxu_block;
+    if (!chemflag) {   // one element block of Y: everything stays on the device
+        fetch_args([&] {
+            if (ijnum <= 0) return;
+            hipStream_t st = library_stream();
+            const int* const arr[2] = {ai, aj};
+            IndexRange r[2];
+            index_ranges(arr, ijnum, r, st);
+            if (r[0].max >= anum || r[1].max >= anum)
+                throw Error("SnapComputeFi: a pair atom index is not below anum");
+            SnapDev s = device_tables(twojmax, rootpqarray, radelem, wjelem, map, st);
+            if (idxu_max != s.idxu_max) throw Error("idxu_max does not match twojmax");
+            s.rcutfac = rcutfac;
+            s.rfac0 = rfac0;
+            s.rmin0 = rmin0;
+            s.switchflag = switchflag;
+            double* d_de = dev<double>(9, 3 * static_cast<size_t>(ijnum));
+            launch_dedr(s, ylist_r, ylist_i, rij, aii, ti, tj, nullptr, d_de, inum, ijnum, nullptr, st);
+            launch_tally_force_atomic_soa(fatom, vatom, d_de, rij, ai, aj, ijnum, anum, st);
+            finish(st);
+        });
+        return;
+    }
     std::vector<int> h_aii, h_ai, h_aj, h_ti, h_tj, h_map;
     std::vector<double> h_rp, h_wj, h_rad;
     if (!fetch_args([&] {

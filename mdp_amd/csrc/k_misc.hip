@@ -4,6 +4,8 @@
 // performance-critical force path lives in k_ui/k_yi/k_dedr and the MD engine.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "snap_device.hpp"
 #include "snap_launch.hpp"
 
@@ -108,6 +110,63 @@ void exclusive_scan(const int* in, int* out, int n, int* tmp, hipStream_t st) {
     if (nb > 0) hipLaunchKernelGGL(k_scan_block, dim3(nb), dim3(SCAN_BLOCK), 0, st, in, out, tmp, n);
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, st, tmp, nb, out + n);
     if (nb > 0) hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(SCAN_BLOCK), 0, st, out, tmp, n);
+}
+
+// ================================================================================================
+// checks of a caller's device-resident pair arrays
+// ================================================================================================
+
+// out[0] = max, out[1] = max of -value, out[2] = 1 when a value is smaller than the one before it (out cleared to a
+// value below all of them).  One pass on the device instead of a read-back and three host loops (315,000 pairs: 0.6 ms).
+__global__ __launch_bounds__(256) void k_index_range(const int* __restrict__ a, int n, int* __restrict__ out) {
+    int hi = -2147483647, lo = -2147483647, drop = 0;
+    for (int p = blockIdx.x * 256 + threadIdx.x; p < n; p += 256 * gridDim.x) {
+        const int v = a[p];
+        hi = max(hi, v);
+        lo = max(lo, v == -2147483647 - 1 ? 2147483647 : -v);
+        drop |= p > 0 && v < a[p - 1];
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o /= 2) {
+        hi = max(hi, __shfl_xor(hi, o));
+        lo = max(lo, __shfl_xor(lo, o));
+        drop |= __shfl_xor(drop, o);
+    }
+    __shared__ int red[4][3];
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6][0] = hi;
+        red[threadIdx.x >> 6][1] = lo;
+        red[threadIdx.x >> 6][2] = drop;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        const int k = threadIdx.x;
+        const int v = max(max(red[0][k], red[1][k]), max(red[2][k], red[3][k]));
+        if (k < 2 || v) atomicMax(out + k, v);
+    }
+}
+
+void launch_index_range(const int* a, int n, int* out, hipStream_t st) {
+    if (n <= 0) return;
+    // at most 128 workgroups, one atomic per word each: 2,048 waves' atomics on the same words took 57 us
+    hipLaunchKernelGGL(k_index_range, dim3(std::min(128, static_cast<int>(nblk(n, 256)))), dim3(256), 0, st, a, n, out);
+}
+
+// off[i] = first position p of the ascending array a[0..n) with a[p] >= i, for i = 0 .. m (all values in [0, m))
+__global__ void k_csr_of_sorted(const int* __restrict__ a, int n, int* __restrict__ off, int m) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i > m) return;
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        if (a[mid] < i) lo = mid + 1;
+        else hi = mid;
+    }
+    off[i] = lo;
+}
+
+void launch_csr_of_sorted(const int* a, int n, int* off, int m, hipStream_t st) {
+    hipLaunchKernelGGL(k_csr_of_sorted, dim3(nblk(m + 1, 256)), dim3(256), 0, st, a, n, off, m);
 }
 
 // ================================================================================================
