@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/mdpsnap.h"
+#include "host_copy.hpp"
 #include "runtime.hpp"
 
 using namespace mdp;
@@ -22,20 +23,22 @@ namespace {
 // Per-argument device buffers, reused across calls (guarded by the library mutex).
 DevBuf g_slot[40];
 DevTables g_tab;
+HostCopies g_copies;   // between the caller's host arrays and the slots
 
 template <class T>
 T* dev(int slot, size_t n) {
     return static_cast<T*>(g_slot[slot].ensure(sizeof(T) * std::max<size_t>(n, 1)));
 }
 template <class T>
-T* put(int slot, const T* h, size_t n, hipStream_t st) {
+T* put(int slot, const T* h, size_t n, hipStream_t st, bool get_follows = false) {
     T* d = dev<T>(slot, n);
-    if (n) MDP_HIP(hipMemcpyAsync(d, h, sizeof(T) * n, hipMemcpyHostToDevice, st));
+    g_copies.put(d, h, sizeof(T) * n, st, get_follows);
     return d;
 }
+// h holds the values after finish()
 template <class T>
 void get(T* h, const T* d, size_t n, hipStream_t st) {
-    if (n) MDP_HIP(hipMemcpyAsync(h, d, sizeof(T) * n, hipMemcpyDeviceToHost, st));
+    g_copies.get(h, d, sizeof(T) * n, st);
 }
 
 // Argument I/O of the shared bodies below.  The cpuSnap.h entry points pass host arrays, staged through
@@ -51,6 +54,10 @@ T* put_arg(int slot, const T* p, size_t n, hipStream_t st) {
     return g_devio ? const_cast<T*>(p) : put(slot, p, n, st);
 }
 template <class T>
+T* inout_arg(int slot, T* p, size_t n, hipStream_t st) {
+    return g_devio ? p : put(slot, p, n, st, true);
+}
+template <class T>
 T* out_arg(int slot, T* p, size_t n) {
     return g_devio ? p : dev<T>(slot, n);
 }
@@ -60,7 +67,7 @@ void get_arg(T* h, const T* d, size_t n, hipStream_t st) {
 }
 void finish(hipStream_t st) {
     MDP_HIP(hipGetLastError());
-    MDP_HIP(hipStreamSynchronize(st));
+    g_copies.finish(st);
 }
 
 int max_of(const int* a, long n, int floor_v = -1) {
@@ -100,6 +107,10 @@ void guarded(F&& f) {
         f();
     } catch (const std::exception& e) {
         set_error(e.what());
+        try {
+            g_copies.abandon(library_stream());
+        } catch (const std::exception&) {   // no stream: nothing was copied
+        }
     }
 }
 
@@ -179,7 +190,7 @@ void cpuNeighPairList(int* pairnum, int* pairlist, double* x, double* rcutsq, in
         exclusive_scan(d_cnt, d_off, inum, d_tmp, st);
         int total = 0;
         get(&total, d_off + inum, 1, st);
-        MDP_HIP(hipStreamSynchronize(st));
+        finish(st);
         int* d_pl = dev<int>(10, total);
         launch_pair_fill(d_pl, d_off, d_x, d_rc, d_il, d_nl, d_nn, d_at, d_al, inum, dim, ntypes, st);
         get(pairnum, d_cnt, inum, st);
@@ -237,8 +248,8 @@ void cpuSnapComputeUi(double* Utotr, double* Utoti, double* rootpqarray, double*
         std::vector<int> off, perm;
         pairs_by_atom(aii, ijnum, inum, off, perm);
         const size_t nu = static_cast<size_t>(inum) * idxu_max * nelem;
-        double* d_ur = put_arg(0, Utotr, nu, st);
-        double* d_ui = put_arg(1, Utoti, nu, st);
+        double* d_ur = inout_arg(0, Utotr, nu, st);
+        double* d_ui = inout_arg(1, Utoti, nu, st);
         double* d_rij = put_arg(2, rij, 3 * static_cast<size_t>(ijnum), st);
         int* d_ti = put(3, ti, ijnum, st);
         int* d_tj = put(4, tj, ijnum, st);
@@ -272,8 +283,8 @@ void cpuAddWself2Ui(double* Utotr, double* Utoti, double wself, int* idxu_block,
         SnapDev s = tables(twojmax, nullptr, nullptr, nullptr, nullptr, map, ntypes, st);
         if (idxu_max != s.idxu_max) throw Error("idxu_max does not match twojmax");
         const size_t nu = static_cast<size_t>(inum) * idxu_max * nelements;
-        double* d_ur = put_arg(0, Utotr, nu, st);
-        double* d_ui = put_arg(1, Utoti, nu, st);
+        double* d_ur = inout_arg(0, Utotr, nu, st);
+        double* d_ui = inout_arg(1, Utoti, nu, st);
         int* d_t = put(2, type, inum, st);
         launch_add_wself(s, d_ur, d_ui, wself, d_t, wselfall_flag, chemflag, nelements, inum, st);
         get_arg(Utotr, d_ur, nu, st);
@@ -299,7 +310,7 @@ bool own_mirror(const SnapDev& s, const double* d_ur, const double* d_ui, int in
     MDP_HIP(hipMemsetAsync(d, 0, sizeof(int), st));
     launch_mirror_differs(s, d_ur, d_ui, d, inum, st);
     get(&differs, d, 1, st);
-    MDP_HIP(hipStreamSynchronize(st));
+    finish(st);
     return !differs;
 }
 
@@ -341,7 +352,7 @@ void cpuSnapComputeEi(double* eatom, double* Utotr, double* Utoti, double* cglis
         double* d_c = put(3, coeffelem, static_cast<size_t>(ncoeffall) * ncoef_rows, st);
         int* d_il = put(4, ilist, inum, st);
         int* d_t = put(5, type, inum, st);
-        double* d_e = put_arg(6, eatom, eext, st);
+        double* d_e = inout_arg(6, eatom, eext, st);
         double* d_b = dev<double>(7, static_cast<size_t>(inum) * idxb_max * ne * ne * ne);
         all_triples_b(s, d_ur, d_ui, d_b, ne, inum, bnorm_flag, own_cg(cglist, index_for(twojmax)), st);
         if (bzero_flag) launch_bzero(s, d_b, d_bz, d_il, d_t, wselfall_flag, chemflag, ne, inum, 0, st);
@@ -404,31 +415,27 @@ void cpuSnapComputeYi(double* ylist_r, double* ylist_i, double* Utotr, double* U
             double* d_bt = put(4, bt.data(), bt.size(), st);
             int* d_ord = put(5, order.data(), order.size(), st);
             launch_yi_full(s, d_ur, d_ui, d_bt, d_yr, d_yi, d_ord, inum, st);
-            MDP_HIP(hipStreamSynchronize(st));
         } else if (ne == 1 && !chemflag) {
             std::vector<double> bt = y_beta_table(ix, beta, 0, 0, 0, 1, 0, ncoeffall, bnorm_flag);
             double* d_bt = put(4, bt.data(), bt.size(), st);
             launch_yi(s, d_ur, d_ui, d_bt, d_yr, d_yi, nullptr, inum, true, st);
-            MDP_HIP(hipStreamSynchronize(st));
         } else {
             std::vector<int> ae(inum);
             for (int i = 0; i < inum; ++i) ae[i] = chemflag ? map[type[i]] : 0;
             int* d_ae = put(5, ae.data(), ae.size(), st);
             const int nie = chemflag ? max_of(ae.data(), inum, 0) + 1 : 1;
             const long nu1 = static_cast<long>(inum) * idxu_max;
-            std::vector<std::vector<double>> keep;
             int slot = 6;
             for (int ie = 0; ie < nie; ++ie)
                 for (int e1 = 0; e1 < ne; ++e1)
                     for (int e2 = 0; e2 < ne; ++e2)
                         for (int e3 = 0; e3 < ne; ++e3) {
-                            keep.push_back(y_beta_table(ix, beta, e1, e2, e3, ne, ie, ncoeffall, bnorm_flag));
+                            const std::vector<double> bt = y_beta_table(ix, beta, e1, e2, e3, ne, ie, ncoeffall, bnorm_flag);
                             if (slot >= 40) throw Error("too many element combinations for the staging slots");
-                            double* d_bt = put(slot++, keep.back().data(), keep.back().size(), st);
+                            double* d_bt = put(slot++, bt.data(), bt.size(), st);
                             launch_yi_acc(s, d_ur, d_ui, nu1 * e1, nu1 * e2, nu1 * e3, d_bt, d_yr, d_yi, d_ae,
                                           chemflag ? ie : -1, inum, st);
                         }
-            MDP_HIP(hipStreamSynchronize(st));
         }
         get_arg(ylist_r, d_yr, nu, st);
         get_arg(ylist_i, d_yi, nu, st);
@@ -470,8 +477,8 @@ void cpuSnapComputeFi(double* fatom, double* vatom, double* ylist_r, double* yli
         int* d_tj = put(7, tj, ijnum, st);
         long* d_yb = chemflag ? put(8, yb.data(), yb.size(), st) : nullptr;
         double* d_de = dev<double>(9, 3 * static_cast<size_t>(ijnum));
-        double* d_f = put_arg(10, fatom, 3 * static_cast<size_t>(fext), st);
-        double* d_v = put_arg(11, vatom, 6 * static_cast<size_t>(vext), st);
+        double* d_f = inout_arg(10, fatom, 3 * static_cast<size_t>(fext), st);
+        double* d_v = inout_arg(11, vatom, 6 * static_cast<size_t>(vext), st);
         launch_dedr(s, d_yr, d_yi, d_rij, d_aii, d_ti, d_tj, d_yb, d_de, inum, ijnum, nullptr, st);
         if (g_vsoa >= 0)
             launch_tally_force_atomic_soa(d_f, d_v, d_de, d_rij, d_ai, d_aj, ijnum, g_vsoa, st);
@@ -499,21 +506,29 @@ void uij_common(double* Sr, double* Si, double* dr[3], double* di[3], double* ro
     const size_t n = static_cast<size_t>(idxu_max) * ijnum;
     double* d_sr = out_arg(0, Sr, n);
     double* d_si = out_arg(1, Si, n);
-    double* ddr[3];
-    double* ddi[3];
-    for (int k = 0; k < 3; ++k) {   // upstream leaves some derivative rows untouched: stage them
-        ddr[k] = put_arg(2 + k, dr[k], n, st);
-        ddi[k] = put_arg(5 + k, di[k], n, st);
+    // Upstream leaves some derivative rows untouched: device arrays keep them in place; for host arrays the rows that are
+    // written lie one after another on the device and go to their places on the way back.
+    const size_t nw = static_cast<size_t>(du_block(twojmax + 1)) * ijnum;
+    double* packed = g_devio ? nullptr : dev<double>(2, 6 * nw);
+    double *ddr[3], *ddi[3];
+    for (int k = 0; k < 3; ++k) {
+        ddr[k] = g_devio ? dr[k] : packed + 2 * k * nw;
+        ddi[k] = g_devio ? di[k] : packed + (2 * k + 1) * nw;
     }
     double* d_rij = put_arg(8, rij, 3 * static_cast<size_t>(ijnum), st);
     int* d_ti = put(9, ti, ijnum, st);
     int* d_tj = put(10, tj, ijnum, st);
-    launch_uij(s, d_sr, d_si, ddr, ddi, d_rij, d_ti, d_tj, ijnum, st);
+    launch_uij(s, d_sr, d_si, ddr, ddi, !g_devio, d_rij, d_ti, d_tj, ijnum, st);
     get_arg(Sr, d_sr, n, st);
     get_arg(Si, d_si, n, st);
-    for (int k = 0; k < 3; ++k) {
-        get_arg(dr[k], ddr[k], n, st);
-        get_arg(di[k], ddi[k], n, st);
+    if (!g_devio) {
+        std::vector<HostCopies::Part> parts;
+        const size_t row = sizeof(double) * static_cast<size_t>(ijnum);
+        for (int a = 0; a < 6; ++a)
+            for (int j = 0; j <= twojmax; ++j)
+                parts.push_back({(a % 2 ? di : dr)[a / 2] + static_cast<size_t>(index_for(twojmax).idxu_block[j]) * ijnum,
+                                 sizeof(double) * a * nw + row * du_block(j), row * (du_block(j + 1) - du_block(j))});
+        g_copies.get_parts(parts, packed, sizeof(double) * 6 * nw, st);
     }
     finish(st);
 }
@@ -584,8 +599,8 @@ void cpuAddUarraytot(double* Stotr, double* Stoti, double* Sr, double* Si, int* 
         if (count_u(J) != idxu_max) throw Error("idxu_max is not a U index-space size");
         SnapDev s = tables(J, nullptr, nullptr, nullptr, nullptr, chemflag ? map : nullptr, ntypes, st);
         const size_t nu = static_cast<size_t>(inum) * idxu_max * nelem, np = static_cast<size_t>(ijnum) * idxu_max;
-        double* d_tr = put_arg(0, Stotr, nu, st);
-        double* d_ti = put_arg(1, Stoti, nu, st);
+        double* d_tr = inout_arg(0, Stotr, nu, st);
+        double* d_ti = inout_arg(1, Stoti, nu, st);
         double* d_sr = put_arg(2, Sr, np, st);
         double* d_si = put_arg(3, Si, np, st);
         int* d_ai = put(4, ai, ijnum, st);
@@ -756,7 +771,8 @@ namespace {
 template <class T>
 std::vector<T> fetch(const T* d, size_t n) {
     std::vector<T> h(std::max<size_t>(n, 1));
-    if (n) MDP_HIP(hipMemcpy(h.data(), d, sizeof(T) * n, hipMemcpyDeviceToHost));
+    get(h.data(), d, n, library_stream());
+    finish(library_stream());
     return h;
 }
 // device-I/O scope for one backend-3 call
@@ -785,7 +801,7 @@ void index_ranges(const int* const (&a)[K], int n, IndexRange (&r)[K], hipStream
     MDP_HIP(hipMemsetAsync(d, 0x80, sizeof(int) * 3 * K, st));
     for (size_t k = 0; k < K; ++k) launch_index_range(a[k], n, d + 3 * k, st);
     get(reinterpret_cast<int*>(r), d, 3 * K, st);
-    MDP_HIP(hipStreamSynchronize(st));
+    finish(st);
 }
 // the library's tables of J with the caller's device-resident numeric tables in their place
 SnapDev device_tables(int J, const double* rootpq, const double* radelem, const double* wjelem, const int* map,
@@ -919,11 +935,12 @@ void mdp_hipSnapComputeYi(double* ylist_r, double* ylist_i, double* ulisttot_r, 
     std::vector<double> h_cg, h_c;
     if (!fetch_args([&] {
             const size_t n = static_cast<size_t>(std::max(inum, 0));
+            h_cg.resize(static_cast<size_t>(index_for(twojmax).idxcg_max));
+            get(h_cg.data(), cglist, h_cg.size(), library_stream());   // with the next one
             h_type = fetch(type, n);
             const int nt = max_type(h_type, n);
             h_map = fetch(map, nt + 1);
             const int rows = max_of(h_map.data() + 1, nt, 0) + 1;
-            h_cg = fetch(cglist, static_cast<size_t>(index_for(twojmax).idxcg_max));
             h_c = fetch(betalist, static_cast<size_t>(ncoeffall) * rows);
         }))
         return;

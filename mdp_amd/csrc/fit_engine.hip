@@ -18,6 +18,7 @@
 
 #include "fit_launch.hpp"
 #include "mdpsnap.h"
+#include "host_copy.hpp"
 #include "runtime.hpp"
 #include "snap_launch.hpp"
 
@@ -272,8 +273,9 @@ struct mdp_fit {
 
     void set_positions(const double* xh) {
         check_positions(xh, "mdp_fit_set_positions");
-        MDP_HIP(hipMemcpyAsync(x.p, xh, sizeof(double) * 3 * N, hipMemcpyHostToDevice, st));
-        MDP_HIP(hipStreamSynchronize(st));
+        EngineCopies c(st);
+        c.put(x.p, xh, sizeof(double) * 3 * N);
+        c.finish();
     }
 
     void ensure_pairs(long need) {
@@ -663,12 +665,10 @@ int mdp_fit_layout(mdp_fit* h, long* atom_off, long* pair_off) {
 int mdp_fit_get(mdp_fit* h, double* blist, double* dblist) {
     return api([&] {
         const int ib = h->tab.idx.idxb_max;
-        if (blist)
-            MDP_HIP(hipMemcpy(blist, h->blist.p, sizeof(double) * static_cast<size_t>(h->N) * ib,
-                              hipMemcpyDeviceToHost));
-        if (dblist)
-            MDP_HIP(hipMemcpy(dblist, h->dblist.p, sizeof(double) * 3 * static_cast<size_t>(h->npairs) * ib,
-                              hipMemcpyDeviceToHost));
+        EngineCopies c(h->st);
+        if (blist) c.get(blist, h->blist.p, sizeof(double) * static_cast<size_t>(h->N) * ib);
+        if (dblist) c.get(dblist, h->dblist.p, sizeof(double) * 3 * static_cast<size_t>(h->npairs) * ib);
+        c.finish();
     });
 }
 
@@ -703,11 +703,11 @@ int mdp_fit_descriptors(mdp_fit* h, double* bi, double* bd, double* bv) {
         if (!h) throw Error("mdp_fit_descriptors: null handle");
         h->lsq_tallies();
         const size_t kt = static_cast<size_t>(h->ntypes) * h->tab.idx.idxb_max;
-        if (bi) MDP_HIP(hipMemcpyAsync(bi, h->l_bi.p, sizeof(double) * h->C * kt, hipMemcpyDeviceToHost, h->st));
-        if (bd)
-            MDP_HIP(hipMemcpyAsync(bd, h->l_bd.p, sizeof(double) * 3 * h->N * kt, hipMemcpyDeviceToHost, h->st));
-        if (bv) MDP_HIP(hipMemcpyAsync(bv, h->l_bv.p, sizeof(double) * 6 * h->C * kt, hipMemcpyDeviceToHost, h->st));
-        MDP_HIP(hipStreamSynchronize(h->st));
+        EngineCopies c(h->st);
+        if (bi) c.get(bi, h->l_bi.p, sizeof(double) * h->C * kt);
+        if (bd) c.get(bd, h->l_bd.p, sizeof(double) * 3 * h->N * kt);
+        if (bv) c.get(bv, h->l_bv.p, sizeof(double) * 6 * h->C * kt);
+        c.finish();
     });
 }
 

@@ -177,12 +177,13 @@ void launch_csr_of_sorted(const int* a, int n, int* off, int m, hipStream_t st) 
 // of one derivative in registers, every finished row (j, mb) written as it comes, with its mirror image where upstream
 // writes one.  Component 0 also writes U.  What upstream leaves unwritten (the derivative rows 2 mb > j of even
 // layers, and those behind (j + 1)/2 of odd ones) is left alone; the derivative row mb = (j + 1)/2 of an odd layer holds
-// the bare dU, as upstream leaves it.  (One lane per pair with all rows, its recursion through global memory: 737 us
+// the bare dU, as upstream leaves it.  `packed`: the derivative rows that are written lie one after another (du_block).  (One lane per pair with all rows, its recursion through global memory: 737 us
 // for 1,080 pairs at twojmax 8; 13 so.)
 template <int J>
 __global__ __launch_bounds__(64) void k_uij(SnapDev s, double* __restrict__ Sr, double* __restrict__ Si,
                                             double* __restrict__ dr0, double* __restrict__ dr1, double* __restrict__ dr2,
                                             double* __restrict__ di0, double* __restrict__ di1, double* __restrict__ di2,
+                                            bool packed,
                                             const double* __restrict__ rij, const int* __restrict__ ti,
                                             const int* __restrict__ tj, int ijnum) {
     const int ij = blockIdx.x * 64 + threadIdx.x, comp = blockIdx.z;
@@ -205,6 +206,7 @@ __global__ __launch_bounds__(64) void k_uij(SnapDev s, double* __restrict__ Sr, 
         row_chain<J, 1, R, R>(g, s.rootpq, [&](auto Jc, auto, auto& pr, auto& pi, auto& dpr, auto& dpi) {
             constexpr int JJ = decltype(Jc)::value;
             constexpr int lo = u_block(JJ) + (JJ + 1) * R, hi = u_block(JJ) + (JJ + 1) * (JJ - R);
+            const int shift = packed ? u_block(JJ) - du_block(JJ) : 0;
 #pragma unroll
             for (int ma = 0; ma <= JJ; ++ma) {
                 const size_t o = ij + P * (lo + ma), m = ij + P * (hi + JJ - ma);
@@ -217,11 +219,12 @@ __global__ __launch_bounds__(64) void k_uij(SnapDev s, double* __restrict__ Sr, 
                         Si[m] = g.sfac * (even ? -pi[ma] : pi[ma]);
                     }
                 }
-                dR[o] = dsu * pr[ma] + g.sfac * dpr[0][ma];
-                dI[o] = dsu * pi[ma] + g.sfac * dpi[0][ma];
+                const size_t od = o - P * shift, md = m - P * shift;
+                dR[od] = dsu * pr[ma] + g.sfac * dpr[0][ma];
+                dI[od] = dsu * pi[ma] + g.sfac * dpi[0][ma];
                 if constexpr (JJ == 2 * R + 1) {
-                    dR[m] = even ? dpr[0][ma] : -dpr[0][ma];
-                    dI[m] = even ? -dpi[0][ma] : dpi[0][ma];
+                    dR[md] = even ? dpr[0][ma] : -dpr[0][ma];
+                    dI[md] = even ? -dpi[0][ma] : dpi[0][ma];
                 }
             }
         });
@@ -229,14 +232,14 @@ __global__ __launch_bounds__(64) void k_uij(SnapDev s, double* __restrict__ Sr, 
 }
 
 void launch_uij(const SnapDev& s, double* Sr, double* Si, double* const dSr[3], double* const dSi[3],
-                const double* rij, const int* ti, const int* tj, int ijnum, hipStream_t st) {
+                bool packed, const double* rij, const int* ti, const int* tj, int ijnum, hipStream_t st) {
     if (ijnum <= 0) return;
     const dim3 grid(nblk(ijnum, 64), s.J / 2 + 1, 3);
     switch (s.J) {
 #define UIJ_CASE(JV)                                                                                              \
     case JV:                                                                                                      \
         hipLaunchKernelGGL(k_uij<JV>, grid, dim3(64), 0, st, s, Sr, Si, dSr[0], dSr[1], dSr[2], dSi[0], dSi[1], dSi[2], \
-                           rij, ti, tj, ijnum);                                                                   \
+                           packed, rij, ti, tj, ijnum);                                                           \
         break;
         UIJ_CASE(2)
         UIJ_CASE(4)

@@ -29,6 +29,7 @@
 
 #include "../../include/mdpsnap.h"
 #include "mlp_launch.hpp"
+#include "host_copy.hpp"
 #include "runtime.hpp"
 #include "snap_device.hpp"
 #include "zbl.hpp"
@@ -1682,9 +1683,10 @@ struct mdp_md {
         for (long k = 0; k < 3L * N; ++k)
             if (!std::isfinite(xh[k]) || (vh && !std::isfinite(vh[k])))
                 throw Error("mdp_md_set_state: non-finite position or velocity");
-        MDP_HIP(hipMemcpyAsync(x.p, xh, sizeof(double) * 3 * N, hipMemcpyHostToDevice, st));
-        if (vh) MDP_HIP(hipMemcpyAsync(v.p, vh, sizeof(double) * 3 * N, hipMemcpyHostToDevice, st));
-        MDP_HIP(hipStreamSynchronize(st));
+        EngineCopies c(st);
+        c.put(x.p, xh, sizeof(double) * 3 * N);
+        if (vh) c.put(v.p, vh, sizeof(double) * 3 * N);
+        c.finish();
         forces_current = false;
     }
 
@@ -1862,12 +1864,13 @@ int mdp_md_run(mdp_md* md, int nsteps) {
 int mdp_md_get(mdp_md* md, double* x, double* v, double* f, double* eatom, double* vatom) {
     return api([&] {
         const size_t n = md->N;
-        MDP_HIP(hipStreamSynchronize(md->st));
-        if (x) MDP_HIP(hipMemcpy(x, md->x.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost));
-        if (v) MDP_HIP(hipMemcpy(v, md->v.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost));
-        if (f) MDP_HIP(hipMemcpy(f, md->f.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost));
-        if (eatom) MDP_HIP(hipMemcpy(eatom, md->eatom.p, sizeof(double) * n, hipMemcpyDeviceToHost));
-        if (vatom) MDP_HIP(hipMemcpy(vatom, md->vir.p, sizeof(double) * 6 * n, hipMemcpyDeviceToHost));
+        EngineCopies c(md->st);
+        if (x) c.get(x, md->x.p, sizeof(double) * 3 * n);
+        if (v) c.get(v, md->v.p, sizeof(double) * 3 * n);
+        if (f) c.get(f, md->f.p, sizeof(double) * 3 * n);
+        if (eatom) c.get(eatom, md->eatom.p, sizeof(double) * n);
+        if (vatom) c.get(vatom, md->vir.p, sizeof(double) * 6 * n);
+        c.finish();
     });
 }
 

@@ -2,6 +2,7 @@
 #include "runtime.hpp"
 
 #include <algorithm>
+#include <cstring>
 
 namespace mdp {
 
@@ -30,42 +31,50 @@ std::mutex& library_mutex() {
 
 void DevTables::upload(const SnapIndex& ix, const double* rootpq_h, const double* cg_h, const double* radelem_h,
                        const double* wjelem_h, const int* map_h, int ntypes, hipStream_t st) {
-    idx = ix;
-    auto put = [&](DevBuf& b, const void* h, size_t bytes) {
-        b.ensure(bytes);
-        if (h && bytes) MDP_HIP(hipMemcpyAsync(b.p, h, bytes, hipMemcpyHostToDevice, st));
+    std::vector<char> h;
+    auto put = [&](const void* p, size_t bytes) {   // a null table is zeros
+        const size_t o = h.size();
+        h.resize(o + (bytes + 63) / 64 * 64, 0);
+        if (p && bytes) std::memcpy(h.data() + o, p, bytes);
+        return o;
     };
     const int jd = ix.J + 1;
-    put(rootpq, rootpq_h ? rootpq_h : ix.rootpq.data(), sizeof(double) * (ix.J + 2) * (ix.J + 2));
-    put(cg, cg_h ? cg_h : ix.cglist.data(), sizeof(double) * ix.idxcg_max);
-    std::vector<double> zeros(ntypes + 1, 0.0);
-    std::vector<int> izeros(ntypes + 1, 0);
-    put(radelem, radelem_h ? radelem_h : zeros.data(), sizeof(double) * (ntypes + 1));
-    put(wjelem, wjelem_h ? wjelem_h : zeros.data(), sizeof(double) * (ntypes + 1));
-    put(map, map_h ? map_h : izeros.data(), sizeof(int) * (ntypes + 1));
-    put(idxz, ix.idxz.data(), sizeof(int) * ix.idxz.size());
-    put(idxb, ix.idxb.data(), sizeof(int) * ix.idxb.size());
-    put(idxu_block, ix.idxu_block.data(), sizeof(int) * jd);
-    put(idxz_block, ix.idxz_block.data(), sizeof(int) * jd * jd * jd);
-    put(idxb_block, ix.idxb_block.data(), sizeof(int) * jd * jd * jd);
-    put(idxcg_block, ix.idxcg_block.data(), sizeof(int) * jd * jd * jd);
+    const size_t rootpq = put(rootpq_h ? rootpq_h : ix.rootpq.data(), sizeof(double) * (ix.J + 2) * (ix.J + 2));
+    const size_t cg = put(cg_h ? cg_h : ix.cglist.data(), sizeof(double) * ix.idxcg_max);
+    const size_t radelem = put(radelem_h, sizeof(double) * (ntypes + 1));
+    const size_t wjelem = put(wjelem_h, sizeof(double) * (ntypes + 1));
+    const size_t map = put(map_h, sizeof(int) * (ntypes + 1));
+    const size_t idxz = put(ix.idxz.data(), sizeof(int) * ix.idxz.size());
+    const size_t idxb = put(ix.idxb.data(), sizeof(int) * ix.idxb.size());
+    const size_t idxu_block = put(ix.idxu_block.data(), sizeof(int) * jd);
+    const size_t idxz_block = put(ix.idxz_block.data(), sizeof(int) * jd * jd * jd);
+    const size_t idxb_block = put(ix.idxb_block.data(), sizeof(int) * jd * jd * jd);
+    const size_t idxcg_block = put(ix.idxcg_block.data(), sizeof(int) * jd * jd * jd);
+    if (idx.J != ix.J || h != content) {
+        content.clear();
+        idx = ix;
+        buf.ensure(h.size());
+        MDP_HIP(hipMemcpyAsync(buf.p, h.data(), h.size(), hipMemcpyHostToDevice, st));
+        MDP_HIP(hipStreamSynchronize(st));
+        content.swap(h);
+    }
+    char* const d = buf.as<char>();
     view.J = ix.J;
     view.idxu_max = ix.idxu_max;
     view.idxz_max = ix.idxz_max;
     view.idxb_max = ix.idxb_max;
     view.idxcg_max = ix.idxcg_max;
-    view.rootpq = rootpq.as<double>();
-    view.cg = cg.as<double>();
-    view.radelem = radelem.as<double>();
-    view.wjelem = wjelem.as<double>();
-    view.map = map.as<int>();
-    view.idxz = idxz.as<int>();
-    view.idxb = idxb.as<int>();
-    view.idxu_block = idxu_block.as<int>();
-    view.idxz_block = idxz_block.as<int>();
-    view.idxb_block = idxb_block.as<int>();
-    view.idxcg_block = idxcg_block.as<int>();
-    MDP_HIP(hipStreamSynchronize(st));   // host staging vectors above go out of scope
+    view.rootpq = reinterpret_cast<double*>(d + rootpq);
+    view.cg = reinterpret_cast<double*>(d + cg);
+    view.radelem = reinterpret_cast<double*>(d + radelem);
+    view.wjelem = reinterpret_cast<double*>(d + wjelem);
+    view.map = reinterpret_cast<int*>(d + map);
+    view.idxz = reinterpret_cast<int*>(d + idxz);
+    view.idxb = reinterpret_cast<int*>(d + idxb);
+    view.idxu_block = reinterpret_cast<int*>(d + idxu_block);
+    view.idxz_block = reinterpret_cast<int*>(d + idxz_block);
+    view.idxb_block = reinterpret_cast<int*>(d + idxb_block);
+    view.idxcg_block = reinterpret_cast<int*>(d + idxcg_block);
 }
 
 std::vector<double> y_beta_table(const SnapIndex& ix, const double* beta, int e1, int e2, int e3, int ne, int ielem,

@@ -59,8 +59,10 @@ struct DevBuf {
 // Device copy of the SNAP tables for one parameter set.
 struct DevTables {
     SnapIndex idx;
-    DevBuf rootpq, cg, radelem, wjelem, map, idxz, idxb, idxu_block, idxz_block, idxb_block, idxcg_block;
-    SnapDev view;   // pointers into the buffers above
+    DevBuf buf;                  // all tables, one after another
+    std::vector<char> content;   // what buf holds; empty: nothing yet
+    SnapDev view;                // pointers into buf
+    // Copies the tables to the device, in one piece, unless they are there byte for byte.
     void upload(const SnapIndex& ix, const double* rootpq_h, const double* cg_h, const double* radelem_h,
                 const double* wjelem_h, const int* map_h, int ntypes, hipStream_t st);
 };

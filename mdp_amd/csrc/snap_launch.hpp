@@ -163,10 +163,17 @@ namespace mdp {
 
 // ---- descriptor path, tallies and pair arrays (generic kernels) ------------------------------
 
+// the derivative rows of layer j that the per-pair recursion writes: the half rows and, of odd layers, the next one
+__host__ __device__ constexpr int du_block(int j) {
+    int b = 0;
+    for (int l = 0; l < j; ++l) b += (l + 1) * (l % 2 ? (l + 1) / 2 + 1 : l / 2 + 1);
+    return b;
+}
 // cpuComputeSij / cpuComputeUij: per-pair U and d(sfac U)/dr; dS[k] are the x/y/z derivative arrays
-// (each [idxu_max*ijnum] at ij + ijnum*jju).
+// (each [idxu_max*ijnum] at ij + ijnum*jju; packed: only the rows that are
+// written, at ij + ijnum*(du_block(j) + (j + 1) mb + ma)).
 void launch_uij(const SnapDev& s, double* Sr, double* Si, double* const dSr[3], double* const dSi[3],
-                const double* rij, const int* ti, const int* tj, int ijnum, hipStream_t st);
+                bool packed, const double* rij, const int* ti, const int* tj, int ijnum, hipStream_t st);
 
 // Stot = wself on the diagonal of the own-element block (element read through type[ai[ii]]).
 void launch_zero_utot(const SnapDev& s, double* Sr, double* Si, double wself, const int* type, const int* ai,

@@ -107,7 +107,7 @@ def test_a_callers_u_is_read_whole(gpu, oracle, J):
     assert relerr(a["Yi"], own["Yi"]) > 1e-6
 
 
-@pytest.mark.parametrize("J,P", [(2, 1), (4, 63), (6, 65), (8, 129)])
+@pytest.mark.parametrize("J,P", [(2, 1), (4, 63), (6, 65), (8, 129), (2, 200001)])
 def test_uij_rows(gpu, oracle, J, P):
     """U and dU of every pair; the derivative rows that are not written keep what they held."""
     p = _pairs(5, P, 1, 11 + P)
