@@ -664,10 +664,13 @@ def main():
         f"({100 * achieved / FP64_PEAK_TFLOPS:.1f}% of FP64 peak); whole step "
         f"{step_flops / (elapsed / a.steps) / 1e12:.2f} TFLOP/s")
     # The algorithmic count is the upstream compute_yi's.  compute_yi variants 115 and 116 skip the terms that
-    # the swap symmetry of the (j1, j1) couplings makes redundant, so the FP64 work they execute is smaller.
+    # the swap symmetry of the (j1, j1) couplings makes redundant, and 308 also forms a product of two U elements
+    # once for all layers it couples to, so the FP64 work they execute is smaller.
     executed = None
-    if dom == "compute_yi" and int(md.tuning().get("chosen", {}).get("compute_yi_waves", 0)) in (115, 116):
-        executed = fl["yi_md_sym"] * n
+    count = {115: "yi_md_sym", 116: "yi_md_sym", 308: "yi_md_class"}
+    variant = int(md.tuning().get("chosen", {}).get("compute_yi_waves", 0))
+    if dom == "compute_yi" and variant in count:
+        executed = fl[count[variant]] * n
         log(f"  compute_yi executes {executed / per_launch[dom]:.3f} of the algorithmic flops: "
             f"{executed / (ms_avg * 1e-3) / 1e12:.2f} TFLOP/s executed")
 

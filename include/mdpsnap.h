@@ -201,7 +201,7 @@ const char *mdp_md_timer_name(int k);
 int mdp_md_num_timers(void);
 
 /* Launch variants chosen by the engine's autotuner after the first force evaluation, as a JSON object
- * with the measured ms per launch of every variant (set MDP_AUTOTUNE=0 to keep the defaults). */
+ * with the measured ms per launch of those timed (set MDP_AUTOTUNE=0 to keep the defaults). */
 int mdp_md_tuning(mdp_md *md, char *buf, int len);
 
 /* Mean number of pairs per force evaluation since timing was last switched (mdp_md_set_timing). */

@@ -82,7 +82,7 @@ void launch_bi(const SnapDev& s, const double* Ur, const double* Ui, long off1, 
 
 // Z of one row mb (blockIdx.z) of one coupling triple (blockIdx.y), all columns ma, into Z[jjz*N + atom].  A row per
 // wave: with all rows of a triple on one wave the heaviest triple's chain set the time of a small system (54 atoms,
-// twojmax 8: 133 us; 106 so).
+// twojmax 8: 133 us; 19 so, with the triple's number a constant).
 template <int J>
 __global__ __launch_bounds__(64) void k_zi(SnapDev s, const double* __restrict__ Ur, const double* __restrict__ Ui,
                                            long off1, long off2, double* __restrict__ Zr, double* __restrict__ Zi,
@@ -98,7 +98,8 @@ __global__ __launch_bounds__(64) void k_zi(SnapDev s, const double* __restrict__
             static_for<0, J + 1>([&](auto JOc) {
                 constexpr int JO = decltype(JOc)::value;
                 if constexpr (coupled(J1, J2, JO)) {
-                    if (t == triple_id(J, J1, J2, JO)) {
+                    constexpr int TRIPLE = triple_id(J, J1, J2, JO);
+                    if (t == TRIPLE) {
                         const int zb = s.idxz_block[JO + J2 * (J + 1) + J1 * (J + 1) * (J + 1)];
                         const double scale = bnorm ? 1.0 / (JO + 1) : 1.0;
                         const int mb = blockIdx.z;

@@ -298,7 +298,8 @@ __global__ __launch_bounds__(64) void k_fit_zb(const double* __restrict__ cg, co
             static_for<0, J + 1>([&](auto JOc) {
                 constexpr int JO = decltype(JOc)::value;
                 if constexpr (coupled(J1, J2, JO)) {
-                    if (t == triple_id(J, J1, J2, JO)) {
+                    constexpr int TRIPLE = triple_id(J, J1, J2, JO);
+                    if (t == TRIPLE) {
                         constexpr int ZB = z_block(J, J1, J2, JO);
                         const double scale = bnorm ? 1.0 / (JO + 1) : 1.0;
                         double bsum = 0.0;

@@ -28,7 +28,13 @@ void launch_yi_rows_8(const SnapDev&, const double*, const double*, const double
 void launch_yi_rows_small(const SnapDev&, const double*, const double*, const double*, double*, double*, double*,
                           const int*, int, hipStream_t);
 
-constexpr int YI_ROWS = 208;   // variant id of k_yi_rows
+void launch_yi_class_8(const SnapDev&, const double*, const double*, const double*, double*, double*, double*, int,
+                       hipStream_t);
+void launch_yi_class_small(const SnapDev&, const double*, const double*, const double*, double*, double*, double*, int,
+                           hipStream_t);
+
+constexpr int YI_ROWS = 208;    // variant id of k_yi_rows
+constexpr int YI_CLASS = 308;   // variant id of k_yi_class
 
 void yi_row_order(int J, int* out) {
     auto cgn = [](int m, int j1, int j2, int j) {
@@ -54,16 +60,27 @@ void yi_row_order(int J, int* out) {
     for (size_t k = 0; k < cost.size(); ++k) out[k] = cost[k].second;
 }
 
+// A workgroup per output row where a workgroup per 64 atoms would leave most CUs idle, then the classes; at twojmax 6, where
+// the classes' longest wave is as long as a block of rows, these in between.  us, per row (208) / rows of a block (8; 116 at
+// twojmax 8) / classes (308): twojmax 4, 1,024 atoms 5.4 / 9.9 / 8.3, 4,394 atoms 9.7 / 10.2 / 8.4, 16,000 atoms
+// 23 / 12.7 / 10.5; twojmax 6, 4,394 atoms 26 / 38 / 40, 8,192 atoms 44 / 41 / 44, 16,000 atoms 87 / 53 / 53, 31,250 atoms
+// - / 92 / 77; twojmax 8, 1,024 atoms 30 / 127 / 92, 4,394 atoms 108 / 144 / 98, 128,000 atoms - / 1,277 / 941.
+int yi_default_variant(int J, int N) {
+    if (N <= 64 * (J == 8 ? 60 : (J == 6 ? 112 : 50))) return YI_ROWS;
+    return J == 6 && N <= 64 * 250 ? 8 : YI_CLASS;
+}
+
 int yi_half_variants(int J, int* ids) {
     if (J == 8) {   // waves per workgroup; 112: 12 waves, the larger layer's U rows shared across couplings;
                     // 113: the same with (re, im) adjacent in LDS; 115: 113 with the swap symmetry of the
                     // (j1, j1) couplings; 116: 115 with the row index made wave-uniform explicitly;
-                    // 208: a workgroup per output row (k_yi_rows)
+                    // 208: a workgroup per output row (k_yi_rows); 308: a wave per class of rows (k_yi_class)
         ids[0] = 8; ids[1] = 12; ids[2] = 4; ids[3] = 112; ids[4] = 113; ids[5] = 115; ids[6] = 116; ids[7] = YI_ROWS;
-        return 8;
+        ids[8] = YI_CLASS;
+        return 9;
     }
-    ids[0] = 8; ids[1] = YI_ROWS;
-    return 2;
+    ids[0] = 8; ids[1] = YI_ROWS; ids[2] = YI_CLASS;
+    return 3;
 }
 
 void launch_yi_half(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
@@ -74,6 +91,13 @@ void launch_yi_half(const SnapDev& s, const double* Ur, const double* Ui, const 
             launch_yi_rows_8(s, Ur, Ui, beta_t, Yr, Yi, epart, order, N, st);
         else
             launch_yi_rows_small(s, Ur, Ui, beta_t, Yr, Yi, epart, order, N, st);
+        return;
+    }
+    if (waves == YI_CLASS) {
+        if (s.J == 8)
+            launch_yi_class_8(s, Ur, Ui, beta_t, Yr, Yi, epart, N, st);
+        else
+            launch_yi_class_small(s, Ur, Ui, beta_t, Yr, Yi, epart, N, st);
         return;
     }
     switch (s.J) {

@@ -30,8 +30,9 @@ template <int J1, bool CX = false>
 __device__ __forceinline__ void lds_row(int mb1, const double* __restrict__ lr, const double* __restrict__ li,
                                         int lane, double (&ar)[J1 + 1], double (&ai)[J1 + 1]) {
     const double2* __restrict__ lc = reinterpret_cast<const double2*>(lr);
+    constexpr int HB = h_block(J1);
     if (2 * mb1 <= J1) {
-        const int b = (h_block(J1) + (J1 + 1) * mb1) * 64 + lane;
+        const int b = (HB + (J1 + 1) * mb1) * 64 + lane;
 #pragma unroll
         for (int m = 0; m <= J1; ++m) {
             if constexpr (CX) {
@@ -44,7 +45,7 @@ __device__ __forceinline__ void lds_row(int mb1, const double* __restrict__ lr, 
             }
         }
     } else {
-        const int b = (h_block(J1) + (J1 + 1) * (J1 - mb1)) * 64 + lane;
+        const int b = (HB + (J1 + 1) * (J1 - mb1)) * 64 + lane;
         const double sm = (mb1 & 1) ? -1.0 : 1.0;
 #pragma unroll
         for (int m = 0; m <= J1; ++m) {
@@ -181,8 +182,8 @@ __device__ __forceinline__ void y_couplings_shared_a(int mb, int malim, const do
                     const int mb2 = mb + (J1 + J2 - JO) / 2 - mb1;
                     constexpr bool SAME = SYM && (J1 == J2);
                     if (mb2 >= 0 && mb2 <= J2 && (!SAME || mb2 >= mb1)) {
-                        constexpr int T = triple_id(J, J1, J2, JO);
-                        double cb = cg[cg_block(J, J1, J2, JO) + mb1 * (J2 + 1) + mb2] * beta_t[T];
+                        constexpr int T = triple_id(J, J1, J2, JO), CGB = cg_block(J, J1, J2, JO);
+                        double cb = cg[CGB + mb1 * (J2 + 1) + mb2] * beta_t[T];
                         if (SAME && mb2 == mb1) {
                             z_terms_same_row<J1, JO>(malim, ar, ai, cb, yr, yi);
                         } else {
@@ -198,22 +199,21 @@ __device__ __forceinline__ void y_couplings_shared_a(int mb, int malim, const do
     });
 }
 
-// PA: per-atom weights beta_t[triple * N + atom] (the learned surrogate's dE/dB) and no energy partials;
-// otherwise wave-uniform weights beta_t[triple].  SA: couplings through y_couplings_shared_a; CX: the
+// SA: couplings through y_couplings_shared_a; CX: the
 // complex-interleaved LDS layout; SYM: the swap symmetry of the (J1, J1) couplings; UNI: 1 makes the
 // shared-row loop's row index wave-uniform explicitly (140 instead of 166 VGPRs at twojmax 8, the row tests
 // become scalar branches), 2 also the output row's (j, mb), which costs spills.
-template <int J, int JO, bool PA = false, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0, bool FULL = false>
+template <int J, int JO, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0>
 __device__ __forceinline__ void y_row_lds(const double* __restrict__ cg, int row, int mb, int atom, bool live, int N,
                                           const double* __restrict__ lr, const double* __restrict__ li, int lane,
                                           const double* __restrict__ beta_t, double* __restrict__ Yr,
                                           double* __restrict__ Yi, double* __restrict__ epart) {
-    const int malim = (!FULL && 2 * mb == JO) ? mb : JO;
+    const int malim = (2 * mb == JO) ? mb : JO;
     const size_t n = static_cast<size_t>(N);
     double yr[JO + 1], yi[JO + 1];
 #pragma unroll
     for (int m = 0; m <= JO; ++m) { yr[m] = 0.0; yi[m] = 0.0; }
-    if constexpr (SA && !PA) {
+    if constexpr (SA) {
         y_couplings_shared_a<J, JO, CX, SYM, UNI>(mb, malim, lr, li, lane, cg, beta_t, yr, yi);
     } else {
         static_for<0, J + 1>([&](auto J1c) {
@@ -222,23 +222,21 @@ __device__ __forceinline__ void y_row_lds(const double* __restrict__ cg, int row
                 constexpr int J2 = decltype(J2c)::value;
                 if constexpr (coupled(J1, J2, JO)) {
                     constexpr int T = triple_id(J, J1, J2, JO);
-                    const double beta =
-                        PA ? (live ? beta_t[static_cast<size_t>(T) * n + atom] : 0.0) : beta_t[T];
-                    z_row_lds<J, J1, J2, JO, CX, SYM>(mb, malim, lr, li, lane, cg, beta, yr, yi);
+                    z_row_lds<J, J1, J2, JO, CX, SYM>(mb, malim, lr, li, lane, cg, beta_t[T], yr, yi);
                 }
             });
         });
     }
     if (!live) return;
-    const int hrow = h_block(JO) + (JO + 1) * mb;
-    const size_t o = static_cast<size_t>(FULL ? u_block(JO) + (JO + 1) * mb : hrow) * n + atom;
+    constexpr int HB = h_block(JO);
+    const int hrow = HB + (JO + 1) * mb;
+    const size_t o = static_cast<size_t>(hrow) * n + atom;
     double e = 0.0;
 #pragma unroll
     for (int ma = 0; ma <= JO; ++ma) {
         if (ma <= malim) {
             Yr[o + ma * n] = yr[ma];
             Yi[o + ma * n] = yi[ma];
-            if constexpr (FULL) continue;
             const double w = (2 * mb < JO || ma < mb) ? 1.0 : 0.5;
             if constexpr (CX) {
                 const double2 u = reinterpret_cast<const double2*>(lr)[(hrow + ma) * 64 + lane];
@@ -248,7 +246,7 @@ __device__ __forceinline__ void y_row_lds(const double* __restrict__ cg, int row
             }
         }
     }
-    if constexpr (!PA && !FULL) epart[static_cast<size_t>(row) * n + atom] = e;
+    epart[static_cast<size_t>(row) * n + atom] = e;
 }
 
 // FULL: U and Y in the upstream layout (element (j, mb, ma) at u_block(j) + (j + 1) mb + ma) instead of the half
@@ -263,7 +261,7 @@ __device__ __forceinline__ int full_element(int e) {
 
 // The coefficient tables (cg, beta_t, order) are separate read-only, non-aliased kernel arguments so
 // that their wave-uniform loads go through the scalar cache into SGPRs.
-template <int J, int W, bool PA = false, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0, bool FULL = false>
+template <int J, int W, bool SA = false, bool CX = false, bool SYM = false, int UNI = 0>
 __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ cg, const double* __restrict__ Ur,
                                                     const double* __restrict__ Ui, const double* __restrict__ beta_t,
                                                     double* __restrict__ Yr, double* __restrict__ Yi,
@@ -280,7 +278,7 @@ __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ c
     const size_t n = static_cast<size_t>(N);
     if (threadIdx.x == 0) next_row = 0;
     for (int e = wave; e < HE; e += W) {
-        const size_t g = static_cast<size_t>(FULL ? full_element<J>(e) : e) * n + atom;
+        const size_t g = static_cast<size_t>(e) * n + atom;
         const double ur = live ? Ur[g] : 0.0;
         const double ui = live ? Ui[g] : 0.0;
         if constexpr (CX) {
@@ -303,8 +301,7 @@ __global__ __launch_bounds__(64 * W) void k_yi_half(const double* __restrict__ c
         static_for<0, J + 1>([&](auto JOc) {
             constexpr int JO = decltype(JOc)::value;
             if (jo == JO)
-                y_row_lds<J, JO, PA, SA, CX, SYM, UNI, FULL>(cg, row, mb, atom, live, N, lr, li, lane, beta_t, Yr, Yi,
-                                                      epart);
+                y_row_lds<J, JO, SA, CX, SYM, UNI>(cg, row, mb, atom, live, N, lr, li, lane, beta_t, Yr, Yi, epart);
         });
     }
 }
@@ -348,7 +345,8 @@ __global__ __launch_bounds__(64 * W) void k_yi_rows(const double* __restrict__ c
         if (jo == JO) {   // uniform over the workgroup
             constexpr int PER = (JO + W) / W;   // elements of the row that a wave finishes: ma = wave + W h
             const int malim = (!FULL && 2 * mb == JO) ? mb : JO;
-            const int hrow = h_block(JO) + (JO + 1) * mb, orow = FULL ? u_block(JO) + (JO + 1) * mb : hrow;
+            constexpr int HB = h_block(JO), OB = FULL ? u_block(JO) : HB;
+            const int hrow = HB + (JO + 1) * mb, orow = OB + (JO + 1) * mb;
             double yr[JO + 1], yi[JO + 1];
 #pragma unroll
             for (int m = 0; m <= JO; ++m) { yr[m] = 0.0; yi[m] = 0.0; }
@@ -455,7 +453,8 @@ __global__ __launch_bounds__(64 * W) void k_b_half(const double* __restrict__ cg
                                 for (int m = 0; m <= JO; ++m) { zr[m] = 0.0; zi[m] = 0.0; }
                                 z_row_lds<J, J1, J2, JO, CX, true>(mb, malim, lr, li, lane, cg,
                                                                    bnorm ? 1.0 / (JO + 1) : 1.0, zr, zi);
-                                const int hrow = h_block(JO) + (JO + 1) * mb;
+                                constexpr int HB = h_block(JO);
+                                const int hrow = HB + (JO + 1) * mb;
 #pragma unroll
                                 for (int ma = 0; ma <= JO; ++ma)
                                     if (ma <= malim) {

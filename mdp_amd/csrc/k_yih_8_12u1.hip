@@ -5,7 +5,7 @@ namespace mdp {
 
 void launch_yi_half_8_12u1(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr,
                           double* Yi, double* epart, const int* order, int N, hipStream_t st) {
-    hipLaunchKernelGGL((k_yi_half<8, 12, false, true, true, true, 1>), dim3((N + 63) / 64), dim3(64 * 12), 0, st, s.cg, Ur, Ui, beta_t, Yr, Yi,
+    hipLaunchKernelGGL((k_yi_half<8, 12, true, true, true, 1>), dim3((N + 63) / 64), dim3(64 * 12), 0, st, s.cg, Ur, Ui, beta_t, Yr, Yi,
                        epart, order, N);
 }
 

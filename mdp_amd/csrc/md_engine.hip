@@ -988,7 +988,7 @@ struct mdp_md {
     int sur_nin = 0, sur_ntrip = 0, audit_every = 0;
     double audit_tol = 0.0;
     DevTables tab_s;
-    DevBuf sUr, sUi, sB, sE, sG, sBeta, sYr, sYi, sParams, sPacked, sAff, sJjb, sFac, sRowOrder, fP, vP, eP, ssq;
+    DevBuf sUr, sUi, sB, sE, sG, sBeta, sYr, sYi, sParams, sPacked, sAff, sJjb, sFac, fP, vP, eP, ssq;
     long audits = 0, fallbacks = 0;
     double rmse_last = 0, rmse_max = 0, rmse_sum = 0;
     // autotuned launch variants (see autotune())
@@ -1102,10 +1102,7 @@ struct mdp_md {
             }
         }
         nrows = n_half_rows(J);
-        // until (or without) the autotuner: a workgroup per output row where a workgroup per 64 atoms would leave
-        // most CUs idle (us, per row / per block: twojmax 8, 4,394 atoms 106 / 132, 8,192 atoms 184 / 144; twojmax 6,
-        // 8,192 atoms 56 / 72, 16,000 atoms 105 / 82)
-        yi_waves = N <= 64 * (J == 8 ? 80 : 128) ? 208 : (J == 8 ? 116 : 8);
+        yi_waves = yi_default_variant(J, N);   // until (or without) the autotuner
         const int lanes = ui_lanes_per_atom(J, N);
         ui_variant = lanes > 1 ? lanes : 0;
         // 256 lanes per cell while they shorten the serial scan (us with 128 / 256: 2,000 atoms 12 / 8, 31,250 atoms
@@ -1381,9 +1378,6 @@ struct mdp_md {
         put(sParams, params, sizeof(float) * MLP_NPARAM);
         put(sAff, a.data(), sizeof(double) * 34);
         put(sJjb, jjb.data(), sizeof(int) * jjb.size());
-        std::vector<int> sorder((js / 2 + 1) * (js / 2 + 1));   // half-U rows (j, mb), 2mb <= j <= js
-        yi_row_order(js, sorder.data());
-        put(sRowOrder, sorder.data(), sizeof(int) * sorder.size());
         put(sFac, fac.data(), sizeof(double) * fac.size());
         sPacked.ensure(sizeof(unsigned short) * MLP_NPACK);
         launch_mlp_pack(sParams.as<float>(), sPacked.as<unsigned short>(), st);
@@ -1424,7 +1418,7 @@ struct mdp_md {
             launch_beta_peratom(sG.as<double>(), sJjb.as<int>(), sFac.as<double>(), sur_ntrip, N, sBeta.as<double>(),
                                 st);
             launch_yi_half_pa(s4, sUr.as<double>(), sUi.as<double>(), sBeta.as<double>(), sYr.as<double>(),
-                              sYi.as<double>(), sRowOrder.as<int>(), N, st);
+                              sYi.as<double>(), N, st);
             launch_dedr(s4, sYr.as<double>(), sYi.as<double>(), prij.as<double>(), pi.as<int>(), pti.as<int>(),
                         ptj.as<int>(), nullptr, dedr.as<double>(), N, pair_slots, pair_base.as<int>() + pair_blocks(), st,
                         true, 10);
@@ -1533,11 +1527,11 @@ struct mdp_md {
             ids[0] = v;
             nv = 1;
         } else {
-            // a workgroup per output row (208) up to one block of 64 atoms per CU; at twojmax 8 the others but 116 are
-            // its predecessors
+            // a workgroup per output row (208) up to one block of 64 atoms per CU; at twojmax 8 all but the classes (308)
+            // are their predecessors
             const bool few = N <= 64 * 256;
             nv = static_cast<int>(std::remove_if(ids, ids + nv, [&](int v) {
-                return v == 208 ? !few : (J == 8 && v != 116);
+                return v == 208 ? !few : (J == 8 && v != 308);
             }) - ids);
         }
         best = 1e30;

@@ -80,14 +80,15 @@ void launch_yi_half(const SnapDev& s, const double* Uhr, const double* Uhi, cons
                     double* Yhi, double* epart, const int* row_order, int natoms, hipStream_t st, int waves = 8);
 // waves-per-workgroup variants available for twojmax J (ids = waves); returns their number
 int yi_half_variants(int J, int* ids);
+int yi_default_variant(int J, int N);   // by the number of atoms
 // row ids of the half domain sorted by decreasing compute_yi work
 void yi_row_order(int J, int* out);
 // The learned surrogate's twojmax 2 / 4 descriptor path on the half layout (rows 2mb <= j, [e][N]): Y
-// with per-atom weights beta_pa[triple * N + atom] (no energy partials; order = yi_row_order(J)), and
+// with per-atom weights beta_pa[triple * N + atom] (no energy partials), and
 // every B (bispectrum triples j >= j1, blist[jjb * N + atom], no bzero subtraction).  Both stage the
 // half U of 64 atoms in LDS.  Return false for other twojmax.
 bool launch_yi_half_pa(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_pa, double* Yr,
-                       double* Yi, const int* order, int N, hipStream_t st);
+                       double* Yi, int N, hipStream_t st);
 bool launch_b_half(const SnapDev& s, const double* Ur, const double* Ui, double* blist, int N, int bnorm,
                    hipStream_t st);
 

@@ -26,13 +26,14 @@ __device__ __forceinline__ void y_row(const SnapDev& s, int row, int mb, int ato
         static_for<0, J1 + 1>([&](auto J2c) {
             constexpr int J2 = decltype(J2c)::value;
             if constexpr (coupled(J1, J2, JO)) {
-                const double beta = PER_ATOM ? beta_t[static_cast<size_t>(triple_id(J, J1, J2, JO)) * n + atom]
-                                             : beta_t[triple_id(J, J1, J2, JO)];
+                constexpr int T = triple_id(J, J1, J2, JO);
+                const double beta = PER_ATOM ? beta_t[static_cast<size_t>(T) * n + atom] : beta_t[T];
                 z_row<J, J1, J2, JO>(mb, malim, U1r, U1i, U2r, U2i, n, atom, s.cg, beta, yr, yi);
             }
         });
     });
-    const size_t o = static_cast<size_t>(u_block(JO) + (JO + 1) * mb) * n + atom;
+    constexpr int UB = u_block(JO);
+    const size_t o = static_cast<size_t>(UB + (JO + 1) * mb) * n + atom;
     double e = 0.0;
 #pragma unroll
     for (int ma = 0; ma <= JO; ++ma) {

@@ -15,7 +15,7 @@ __device__ __forceinline__ void z_row(int mb, int malim, const double* __restric
                                       const double* __restrict__ U2r, const double* __restrict__ U2i, size_t n, int atom,
                                       const double* __restrict__ cg, double scale, double (&zr)[JO + 1],
                                       double (&zi)[JO + 1]) {
-    constexpr int CGB = cg_block(J, J1, J2, JO);
+    constexpr int CGB = cg_block(J, J1, J2, JO), UB1 = u_block(J1), UB2 = u_block(J2);
     const double* __restrict__ c = cg + CGB;
     const int mb1min = max(0, (2 * mb - JO - J2 + J1) / 2);
     const int mb2max = (2 * mb - JO - (2 * mb1min - J1) + J2) / 2;
@@ -23,8 +23,8 @@ __device__ __forceinline__ void z_row(int mb, int malim, const double* __restric
     for (int ib = 0; ib < nb; ++ib) {
         const int mb1 = mb1min + ib, mb2 = mb2max - ib;
         const double cb = c[mb1 * (J2 + 1) + mb2] * scale;
-        const size_t o1 = static_cast<size_t>(u_block(J1) + (J1 + 1) * mb1) * n + atom;
-        const size_t o2 = static_cast<size_t>(u_block(J2) + (J2 + 1) * mb2) * n + atom;
+        const size_t o1 = static_cast<size_t>(UB1 + (J1 + 1) * mb1) * n + atom;
+        const size_t o2 = static_cast<size_t>(UB2 + (J2 + 1) * mb2) * n + atom;
         double ar[J1 + 1], ai[J1 + 1], br[J2 + 1], bi[J2 + 1];
 #pragma unroll
         for (int m = 0; m <= J1; ++m) { ar[m] = U1r[o1 + m * n]; ai[m] = U1i[o1 + m * n]; }

@@ -17,6 +17,9 @@ enumerated from the loop bounds of the index spaces -- the denominators of the r
 * ``yi_md_sym`` per atom: what compute_yi executes when the (j1, j1) couplings take each unordered pair
                       of U rows once (the swap symmetry of their two factors): for those couplings only the
                       row pairs mb1 < mb2 (whole) and mb1 = mb2 (the terms m1 <= m2) are computed.
+* ``yi_md_class`` per atom: what compute_yi executes when a product of two U elements is formed once for all layers
+                      it couples to: 6 per product (row pairs and terms as in yi_md_sym), 4 per product and layer (2 for
+                      the first of a sum) and 4 per column and layer for the row weight, plus 4 per entry for U.Y.
 * ``ei``   per atom : the upstream fused energy (cpuSnap.cpp:544-719): Z over the half domain of each
                       bispectrum triple (10*na*nb + 4*nb) + 4 for the U.Z product + 2 for beta*B.
 * ``zb``   per atom : every Z entry (cpuSnap.cpp:1899-1969: 10*na*nb + 4*nb per idxz entry) plus B of
@@ -47,6 +50,28 @@ def _row_updates(J, derivs):
         for j in range(max(1, 2 * mb), J + 1):
             tot += first + mid * (j - 1) + last
     return tot
+
+
+def _yi_class_flops(J):
+    total = 0
+    for k in range(J + 1):   # output rows (j, mb) with j - 2 mb = k
+        total += sum(4 * ((j // 2 if k == 0 else j) + 1) for j in range(k, J + 1, 2))
+        for j1 in range(J + 1):
+            for j2 in range((j1 + k) % 2, j1 + 1, 2):
+                c = (j1 + j2 - k) // 2   # mb1 + mb2
+                for mb1 in range(max(0, c - j2), min(j1, c) + 1):
+                    if j1 == j2 and mb1 > c - mb1:
+                        continue
+                    for t in range(j1 + j2 + 1):   # m1 + m2
+                        m2 = abs(2 * t - j1 - j2)
+                        layers = len(range(max(k, j1 - j2, m2), min(J, j1 + j2) + 1, 2))
+                        if layers == 0 or (k == 0 and 2 * t > j1 + j2):
+                            continue
+                        n = min(j1, t) - max(0, t - j2) + 1
+                        if j1 == j2 and 2 * mb1 == c:
+                            n = (n + 1) // 2
+                        total += 6 * n + layers * (4 * n - 2 + 4)
+    return total
 
 
 @lru_cache(maxsize=None)
@@ -95,8 +120,8 @@ def snap_flops(J):
         if j >= j1:
             ei += 2
     dbdr = _row_updates(J, True) + 3 * (4 * elems + 2 * terms)
-    return dict(ui=ui, dedr=dedr, dedr_gen=dedr_gen, yi=yi, yi_md=yi_md, yi_md_sym=yi_md_sym, ei=ei, zb=zb,
-                dbdr=dbdr)
+    return dict(ui=ui, dedr=dedr, dedr_gen=dedr_gen, yi=yi, yi_md=yi_md, yi_md_sym=yi_md_sym,
+                yi_md_class=_yi_class_flops(J), ei=ei, zb=zb, dbdr=dbdr)
 
 
 def dedr_key(variant):

@@ -31,6 +31,16 @@ def test_yi_row_workgroups_vs_oracle(oracle, monkeypatch, J, n):
     assert md.tuning()["chosen"]["compute_yi_waves"] == 208
 
 
+@pytest.mark.parametrize("n", [1, 63, 65, 250])
+@pytest.mark.parametrize("J", [2, 4, 6, 8])
+def test_yi_classes_vs_oracle(oracle, monkeypatch, J, n):
+    """compute_yi with the output rows of one j - 2 mb on a wave (variant 308)."""
+    monkeypatch.setenv("MDP_YI_VARIANT", "308")
+    x, box = _atoms(n, 7 + n + J)
+    md = _first_step_vs_oracle(oracle, x, box, J, 3)
+    assert md.tuning()["chosen"]["compute_yi_waves"] == 308
+
+
 @pytest.mark.parametrize("variant", ["4", "16"])
 @pytest.mark.parametrize("J,n", [(2, 1), (4, 63), (6, 65), (8, 17), (8, 250)])
 def test_ui_lanes_per_atom_vs_oracle(oracle, monkeypatch, J, n, variant):
