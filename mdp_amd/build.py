@@ -19,8 +19,14 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libmdpsnap.so")
 HEADER = os.path.join(ROOT, "include", "mdpsnap.h")
 
-SOURCES = ["k_fit.hip", "k_fit_mfma.hip", "k_fitlsq.hip", "k_fit_zb.hip", "k_yih_8_8.hip", "k_yih_8_12.hip", "k_yih_8_4.hip", "k_yih_8_12s.hip", "k_yih_8_12c.hip", "k_yih_8_12y.hip", "k_yih_8_12u1.hip", "k_yih_rows_8.hip", "k_yih_rows.hip", "k_yih_small.hip", "k_yih_full_8.hip", "k_yih_full_b.hip", "k_yih_full.hip", "k_yic_8.hip", "k_yic.hip", "k_yi.hip", "k_yia.hip", "k_yih.hip", "k_dedr.hip", "k_bz.hip", "k_ui.hip", "k_misc.hip", "md_engine.hip", "fit_engine.hip", "k_mlp.hip", "k_sur.hip", "surrogate_api.cpp", "dropin.cpp", "velocity.cpp",
-           "runtime.cpp", "host_copy.cpp", "snap_tables.cpp", "pairpot.hip", "cellsort.hip", "app_input.cpp"]
+# the slowest to compile first
+SOURCES = ["k_fit.hip", "k_yih_full_8.hip", "k_yic_8.hip", "k_fit_zb.hip", "k_yi.hip", "k_yia.hip", "k_bz.hip",
+           "k_dedr.hip", "k_fit_mfma.hip", "k_fitlsq.hip", "k_yih_8_8.hip", "k_yih_8_12.hip", "k_yih_8_4.hip",
+           "k_yih_8_12s.hip", "k_yih_8_12c.hip", "k_yih_8_12y.hip", "k_yih_8_12u1.hip", "k_yih_rows_8.hip",
+           "k_yih_rows.hip", "k_yih_small.hip", "k_yih_full_b.hip", "k_yih_full.hip", "k_yic.hip", "k_yih.hip",
+           "k_ui.hip", "k_misc.hip", "md_engine.hip", "fit_engine.hip", "k_mlp.hip", "k_sur.hip",
+           "surrogate_api.cpp", "dropin.cpp", "velocity.cpp", "runtime.cpp", "host_copy.cpp", "snap_tables.cpp",
+           "pairpot.hip", "cellsort.hip", "app_input.cpp"]
 
 ARCH = os.environ.get("MDP_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",
