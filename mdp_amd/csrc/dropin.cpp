@@ -66,7 +66,12 @@ void get_arg(T* h, const T* d, size_t n, hipStream_t st) {
     if (!g_devio) get(h, d, n, st);
 }
 void finish(hipStream_t st) {
-    MDP_HIP(hipGetLastError());
+    try {
+        MDP_HIP(hipGetLastError());
+    } catch (...) {   // nothing writes to what the gets were to fill once a caller that owns it unwinds
+        g_copies.abandon(st);
+        throw;
+    }
     g_copies.finish(st);
 }
 

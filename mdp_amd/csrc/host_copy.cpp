@@ -193,11 +193,23 @@ void HostCopies::get(void* dst, const void* src, size_t bytes, hipStream_t st) {
 }
 
 void HostCopies::get_parts(const std::vector<Part>& parts, const void* src, size_t bytes, hipStream_t st) {
+    const size_t before = pending.size();
+    try {
+        // while the device works on what was asked of it before
+        for (const Part& t : parts)
+            if (t.bytes >= SHARED) copy_threads().post(moving, t.dst, nullptr, t.bytes);
+        issue(parts, src, bytes, st);
+    } catch (...) {   // the caller may free what the threads make pages of as it unwinds
+        copy_threads().wait(moving);
+        if (pending.size() > before) pending.erase(pending.begin() + static_cast<long>(before), pending.end());
+        throw;
+    }
+}
+
+// the copies of get_parts into the pinned chunks, and what is to be moved on from there
+void HostCopies::issue(const std::vector<Part>& parts, const void* src, size_t bytes, hipStream_t st) {
     hipEvent_t* ev;
     size_t k = 0;
-    // while the device works on what was asked of it before
-    for (const Part& t : parts)
-        if (t.bytes >= SHARED) copy_threads().post(moving, t.dst, nullptr, t.bytes);
     for (size_t o = 0; o < bytes; o += PIECE) {
         const size_t n = std::min(PIECE, bytes - o);
         char* p = take(n, st, &ev);

@@ -29,7 +29,7 @@ public:
     };
     // dst is written by the next finish() on the same stream
     void get(void* dst, const void* src, size_t bytes, hipStream_t st);
-    // the parts (ascending, disjoint) of src[0..bytes)
+    // the parts (ascending, disjoint) of src[0..bytes).  Where it throws, nothing writes to this call's parts any more
     void get_parts(const std::vector<Part>& parts, const void* src, size_t bytes, hipStream_t st);
     // waits for the stream and for every byte of the gets
     void finish(hipStream_t st);
@@ -56,6 +56,7 @@ private:
     Group moving;    // what the threads still do for the gets
     size_t at = 0;   // first free byte over all chunks
     char* take(size_t bytes, hipStream_t st, hipEvent_t** ev);
+    void issue(const std::vector<Part>& parts, const void* src, size_t bytes, hipStream_t st);
 };
 
 // Copies of the engines' own calls: a process-wide set behind a lock, held for the lifetime of this object.  Every copy

@@ -1,0 +1,178 @@
+// The copies between host arrays and the device (mdp_amd/csrc/host_copy.cpp) on the CPU: the few HIP calls they make
+// are played here.  A stream is a queue of copies that run when it, or an event behind them, is waited for, so a chunk
+// that is filled again too early, or a byte that is handed on too early, shows as wrong data.
+//   host_copies_cpu bytes | unwind
+#include <sys/mman.h>
+#include <unistd.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <random>
+#include <string>
+#include <vector>
+
+#include "../mdp_amd/csrc/host_copy.hpp"
+#include "../mdp_amd/csrc/runtime.hpp"
+
+namespace {
+
+struct Stream {
+    int device = 0;
+    std::vector<std::function<void()>> queue;
+    size_t done = 0;
+    void run(size_t upto) {
+        for (; done < upto; ++done) queue[done]();
+    }
+};
+struct Event {
+    int device;
+    Stream* stream = nullptr;
+    size_t upto = 0;
+};
+thread_local int current_device = 0;
+bool refuse_copies = false;
+
+Stream* of(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
+hipStream_t handle(Stream& s) { return reinterpret_cast<hipStream_t>(&s); }
+
+}  // namespace
+
+extern "C" {
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void* p) {
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
+    if (refuse_copies) return hipErrorUnknown;
+    of(st)->queue.push_back([=] { std::memcpy(d, s, n); });
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t st) {
+    of(st)->run(of(st)->queue.size());
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(new Event{current_device});
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+    delete reinterpret_cast<Event*>(e);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
+    Event* v = reinterpret_cast<Event*>(e);
+    if (v->device != of(st)->device) return hipErrorInvalidHandle;
+    v->stream = of(st);
+    v->upto = of(st)->queue.size();
+    return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+    Event* v = reinterpret_cast<Event*>(e);
+    v->stream->run(v->upto);
+    return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "an error of the test"; }
+}
+
+namespace {
+
+void expect(bool ok, const std::string& what) {
+    if (ok) return;
+    std::printf("FAILED: %s\n", what.c_str());
+    std::exit(1);
+}
+
+// Every size on both sides of the limits: shared among threads or not (192 KB), one piece or more (2 MB), one batch of
+// pieces or more (16 MB), all chunks in use (32 MB); several copies before a finish; parts with gaps between them.
+void bytes() {
+    std::mt19937_64 rng(1);
+    mdp::HostCopies c;
+    Stream st;
+    const size_t KB = 1 << 10, MB = 1 << 20;
+    const std::vector<std::vector<size_t>> groups = {
+        {1, 63, 64, 65}, {192 * KB - 1, 192 * KB, 5}, {2 * MB - 1, 2 * MB, 2 * MB + 1}, {16 * MB - 3, 16 * MB + 3},
+        {30 * MB, 3 * MB, 7}, {32 * MB, 64}, {40 * MB + 5, 2 * MB + 11, 192 * KB, 100}};
+    for (const auto& sizes : groups) {
+        std::vector<std::vector<unsigned char>> src, dev, back, kept;
+        for (size_t n : sizes) {
+            src.emplace_back(n);
+            for (size_t i = 0; i < n; i += 8) {
+                const unsigned long long r = rng();
+                std::memcpy(&src.back()[i], &r, std::min<size_t>(8, n - i));
+            }
+            dev.emplace_back(n, 0);
+            back.emplace_back(n, 0xAA);
+        }
+        kept = src;
+        for (size_t k = 0; k < sizes.size(); ++k) {
+            c.put(dev[k].data(), src[k].data(), sizes[k], handle(st), k % 2);
+            std::memset(src[k].data(), 0x55, sizes[k]);   // the call has read it
+        }
+        for (size_t k = 0; k < sizes.size(); ++k) {
+            if (k % 2 && sizes[k] > 10) {   // in three parts, a byte left out between them
+                const size_t a = sizes[k] / 3, b = sizes[k] / 2;
+                unsigned char* d = back[k].data();
+                c.get_parts({{d, 0, a}, {d + a + 1, a + 1, b - a - 1}, {d + b + 1, b + 1, sizes[k] - b - 1}}, dev[k].data(),
+                            sizes[k], handle(st));
+                kept[k][a] = kept[k][b] = 0xAA;
+            } else {
+                c.get(back[k].data(), dev[k].data(), sizes[k], handle(st));
+            }
+        }
+        c.finish(handle(st));
+        for (size_t k = 0; k < sizes.size(); ++k)
+            expect(back[k] == kept[k], "bytes of " + std::to_string(sizes[k]) + " as they were");
+        std::printf("%zu copies from %zu bytes on: ok\n", sizes.size(), sizes[0]);
+    }
+}
+
+size_t resident(void* p, size_t n) {
+    std::vector<unsigned char> v(n / 4096);
+    expect(mincore(p, n, v.data()) == 0, "mincore");
+    size_t k = 0;
+    for (unsigned char b : v) k += b & 1;
+    return k;
+}
+
+// A copy that fails leaves nothing behind that still writes to its destination: the caller may free it as it unwinds.
+void unwind() {
+    const size_t n = size_t(512) << 20;
+    void* p = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+    expect(p != MAP_FAILED, "mmap");
+    madvise(p, n, MADV_NOHUGEPAGE);
+    mdp::HostCopies c;
+    Stream st;
+    std::vector<char> src(1 << 20);
+    refuse_copies = true;
+    bool thrown = false;
+    try {
+        c.get(p, src.data(), n, handle(st));
+    } catch (const mdp::Error&) {
+        thrown = true;
+    }
+    const size_t at_throw = resident(p, n);
+    usleep(300000);
+    const size_t later = resident(p, n);
+    std::printf("pages when the call failed %zu, 0.3 s later %zu\n", at_throw, later);
+    expect(thrown, "the failed copy is reported");
+    expect(at_throw == later, "no page of the destination is written after the call has failed");
+    refuse_copies = false;
+    c.finish(handle(st));   // and nothing of it is left to be delivered
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "bytes")
+        bytes();
+    else if (what == "unwind")
+        unwind();
+    else
+        return 2;
+    std::printf("ok\n");
+    return 0;
+}
