@@ -263,25 +263,47 @@ void HostCopies::abandon(hipStream_t st) noexcept {
 }
 
 namespace {
-std::mutex& engine_mutex() {
-    static std::mutex m;
-    return m;
-}
-HostCopies& engine_copies() {
-    static HostCopies c;
-    return c;
+// The sets that no engine's copies use at the moment.  Four of them (of at most 32 MB of pinned memory each) are kept for
+// the next copies, more are given back: as many engines as a program runs on different threads copy without allocating.
+struct IdleSets {
+    static constexpr size_t KEPT = 4;
+    std::mutex m;
+    std::vector<std::unique_ptr<HostCopies>> sets;
+    IdleSets() { sets.reserve(KEPT); }
+};
+IdleSets& idle_sets() {
+    static IdleSets s;
+    return s;
 }
 }  // namespace
 
-EngineCopies::EngineCopies(hipStream_t s) : st(s) { engine_mutex().lock(); }
-EngineCopies::~EngineCopies() {
-    if (open) engine_copies().abandon(st);
-    engine_mutex().unlock();
+EngineCopies::EngineCopies(hipStream_t s) : st(s) {
+    IdleSets& idle = idle_sets();
+    {
+        std::lock_guard<std::mutex> lk(idle.m);
+        if (!idle.sets.empty()) {
+            set = std::move(idle.sets.back());
+            idle.sets.pop_back();
+        }
+    }
+    if (!set) set = std::make_unique<HostCopies>();
 }
-void EngineCopies::put(void* dst, const void* src, size_t bytes) { engine_copies().put(dst, src, bytes, st); }
-void EngineCopies::get(void* dst, const void* src, size_t bytes) { engine_copies().get(dst, src, bytes, st); }
+EngineCopies::~EngineCopies() {
+    if (open) set->abandon(st);
+    IdleSets& idle = idle_sets();
+    std::lock_guard<std::mutex> lk(idle.m);
+    if (idle.sets.size() < IdleSets::KEPT) idle.sets.push_back(std::move(set));
+}
+void EngineCopies::put(void* dst, const void* src, size_t bytes) {
+    open = true;
+    set->put(dst, src, bytes, st);
+}
+void EngineCopies::get(void* dst, const void* src, size_t bytes) {
+    open = true;
+    set->get(dst, src, bytes, st);
+}
 void EngineCopies::finish() {
-    engine_copies().finish(st);
+    set->finish(st);
     open = false;
 }
 

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <memory>
 #include <vector>
 
 namespace mdp {
@@ -59,19 +60,22 @@ private:
     void issue(const std::vector<Part>& parts, const void* src, size_t bytes, hipStream_t st);
 };
 
-// Copies of the engines' own calls: a process-wide set behind a lock, held for the lifetime of this object.  Every copy
-// is complete after finish().
+// Copies of the engines' own calls, through a set of chunks that nobody else uses while this object lives: engines on
+// different threads don't wait for one another's streams.  Every copy is complete after finish().
 class EngineCopies {
 public:
     explicit EngineCopies(hipStream_t st);
     ~EngineCopies();
+    EngineCopies(const EngineCopies&) = delete;
+    EngineCopies& operator=(const EngineCopies&) = delete;
     void put(void* dst, const void* src, size_t bytes);
     void get(void* dst, const void* src, size_t bytes);
     void finish();
 
 private:
     hipStream_t st;
-    bool open = true;
+    std::unique_ptr<HostCopies> set;
+    bool open = false;   // something was asked for since the last finish()
 };
 
 }  // namespace mdp

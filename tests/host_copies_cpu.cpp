@@ -1,16 +1,20 @@
 // The copies between host arrays and the device (mdp_amd/csrc/host_copy.cpp) on the CPU: the few HIP calls they make
 // are played here.  A stream is a queue of copies that run when it, or an event behind them, is waited for, so a chunk
 // that is filled again too early, or a byte that is handed on too early, shows as wrong data.
-//   host_copies_cpu bytes | unwind
+//   host_copies_cpu bytes | unwind | two_engines
 #include <sys/mman.h>
 #include <unistd.h>
 
+#include <chrono>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <mutex>
 #include <random>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../mdp_amd/csrc/host_copy.hpp"
@@ -22,7 +26,9 @@ struct Stream {
     int device = 0;
     std::vector<std::function<void()>> queue;
     size_t done = 0;
+    std::function<void()> work;   // what the stream is busy with before its copies
     void run(size_t upto) {
+        if (work) work();
         for (; done < upto; ++done) queue[done]();
     }
 };
@@ -163,6 +169,44 @@ void unwind() {
     c.finish(handle(st));   // and nothing of it is left to be delivered
 }
 
+// An engine whose stream is busy keeps no other engine's copies waiting.  The first engine's stream is done only when the
+// second one has its bytes, or after 10 s.
+void two_engines() {
+    std::mutex m;
+    std::condition_variable cv;
+    bool waiting = false, second_done = false, in_time = false;
+    Stream busy, idle;
+    busy.work = [&] {
+        std::unique_lock<std::mutex> lk(m);
+        waiting = true;
+        cv.notify_all();
+        in_time = cv.wait_for(lk, std::chrono::seconds(10), [&] { return second_done; });
+    };
+    std::vector<char> a(100, 1), b(100, 2), got_a(100), got_b(100);
+    std::thread first([&] {
+        mdp::EngineCopies c(handle(busy));
+        c.get(got_a.data(), a.data(), a.size());
+        c.finish();
+    });
+    {
+        std::unique_lock<std::mutex> lk(m);
+        cv.wait(lk, [&] { return waiting; });
+    }
+    {
+        mdp::EngineCopies c(handle(idle));
+        c.get(got_b.data(), b.data(), b.size());
+        c.finish();
+    }
+    {
+        std::lock_guard<std::mutex> lk(m);
+        second_done = true;
+        cv.notify_all();
+    }
+    first.join();
+    expect(got_a == a && got_b == b, "bytes as they were");
+    expect(in_time, "the second engine's copies do not wait for the first engine's stream");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -171,6 +215,8 @@ int main(int argc, char** argv) {
         bytes();
     else if (what == "unwind")
         unwind();
+    else if (what == "two_engines")
+        two_engines();
     else
         return 2;
     std::printf("ok\n");
