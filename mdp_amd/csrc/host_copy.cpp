@@ -9,6 +9,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <deque>
+#include <map>
 #include <mutex>
 #include <thread>
 
@@ -126,6 +127,32 @@ CopyThreads& copy_threads() {
     return *o.t;
 }
 
+int device_of(hipStream_t st) {
+    hipDevice_t d = 0;
+    MDP_HIP(hipStreamGetDevice(st, &d));
+    return d;
+}
+
+// The stream's device as the current one: pinned memory and events belong to the device that is current when they are made,
+// and an event can only be recorded on that device's streams.
+class OnDeviceOf {
+public:
+    explicit OnDeviceOf(hipStream_t st) {
+        const int device = device_of(st);
+        MDP_HIP(hipGetDevice(&before));
+        if (before == device)
+            before = -1;
+        else
+            MDP_HIP(hipSetDevice(device));
+    }
+    ~OnDeviceOf() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+
+private:
+    int before = -1;
+};
+
 // below this a thread's wake-up costs more than its share of the copy
 constexpr size_t SHARED = size_t(192) << 10;
 
@@ -147,6 +174,7 @@ char* HostCopies::take(size_t bytes, hipStream_t st, hipEvent_t** ev) {
     const size_t k = at / CHUNK, o = at % CHUNK;
     if (k >= chunks.size()) {
         Chunk c;
+        const OnDeviceOf on(st);
         MDP_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.p), CHUNK, hipHostMallocDefault));
         chunks.push_back(c);
     }
@@ -216,7 +244,10 @@ void HostCopies::issue(const std::vector<Part>& parts, const void* src, size_t b
         MDP_HIP(hipMemcpyAsync(p, static_cast<const char*>(src) + o, n, hipMemcpyDeviceToHost, st));
         Pending q{p, nullptr, {}};
         if (n >= SHARED) {   // its bytes are moved on while the next piece is under way
-            if (!*ev) MDP_HIP(hipEventCreateWithFlags(ev, hipEventDisableTiming));
+            if (!*ev) {
+                const OnDeviceOf on(st);
+                MDP_HIP(hipEventCreateWithFlags(ev, hipEventDisableTiming));
+            }
             MDP_HIP(hipEventRecord(*ev, st));
             q.ready = *ev;
         }
@@ -263,13 +294,13 @@ void HostCopies::abandon(hipStream_t st) noexcept {
 }
 
 namespace {
-// The sets that no engine's copies use at the moment.  Four of them (of at most 32 MB of pinned memory each) are kept for
-// the next copies, more are given back: as many engines as a program runs on different threads copy without allocating.
+// The sets that no engine's copies use at the moment, by device.  Four of a device (of at most 32 MB of pinned memory each)
+// are kept for the next copies, more are given back: as many engines as a program runs on different threads copy without
+// allocating.
 struct IdleSets {
     static constexpr size_t KEPT = 4;
     std::mutex m;
-    std::vector<std::unique_ptr<HostCopies>> sets;
-    IdleSets() { sets.reserve(KEPT); }
+    std::map<int, std::vector<std::unique_ptr<HostCopies>>> of_device;
 };
 IdleSets& idle_sets() {
     static IdleSets s;
@@ -277,13 +308,15 @@ IdleSets& idle_sets() {
 }
 }  // namespace
 
-EngineCopies::EngineCopies(hipStream_t s) : st(s) {
+EngineCopies::EngineCopies(hipStream_t s) : st(s), device(device_of(s)) {
     IdleSets& idle = idle_sets();
     {
         std::lock_guard<std::mutex> lk(idle.m);
-        if (!idle.sets.empty()) {
-            set = std::move(idle.sets.back());
-            idle.sets.pop_back();
+        auto& sets = idle.of_device[device];
+        sets.reserve(IdleSets::KEPT);
+        if (!sets.empty()) {
+            set = std::move(sets.back());
+            sets.pop_back();
         }
     }
     if (!set) set = std::make_unique<HostCopies>();
@@ -292,7 +325,8 @@ EngineCopies::~EngineCopies() {
     if (open) set->abandon(st);
     IdleSets& idle = idle_sets();
     std::lock_guard<std::mutex> lk(idle.m);
-    if (idle.sets.size() < IdleSets::KEPT) idle.sets.push_back(std::move(set));
+    auto& sets = idle.of_device[device];
+    if (sets.size() < IdleSets::KEPT) sets.push_back(std::move(set));
 }
 void EngineCopies::put(void* dst, const void* src, size_t bytes) {
     open = true;

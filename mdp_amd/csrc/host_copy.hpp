@@ -13,7 +13,7 @@
 
 namespace mdp {
 
-// One set of pinned chunks.  Not thread-safe: its owner serialises the use.
+// One set of pinned chunks, for streams of one device.  Not thread-safe: its owner serialises the use.
 class HostCopies {
 public:
     HostCopies() = default;
@@ -74,6 +74,7 @@ public:
 
 private:
     hipStream_t st;
+    int device;   // of the stream: what the set belongs to
     std::unique_ptr<HostCopies> set;
     bool open = false;   // something was asked for since the last finish()
 };

@@ -1,7 +1,7 @@
 // The copies between host arrays and the device (mdp_amd/csrc/host_copy.cpp) on the CPU: the few HIP calls they make
 // are played here.  A stream is a queue of copies that run when it, or an event behind them, is waited for, so a chunk
 // that is filled again too early, or a byte that is handed on too early, shows as wrong data.
-//   host_copies_cpu bytes | unwind | two_engines
+//   host_copies_cpu bytes | unwind | two_engines | two_devices
 #include <sys/mman.h>
 #include <unistd.h>
 
@@ -11,8 +11,10 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <mutex>
 #include <random>
+#include <set>
 #include <string>
 #include <thread>
 #include <vector>
@@ -38,6 +40,21 @@ struct Event {
     size_t upto = 0;
 };
 thread_local int current_device = 0;
+struct Pinned {
+    size_t bytes;
+    int device;
+    std::set<int> used_by;
+};
+std::mutex pinned_lock;
+std::map<char*, Pinned> pinned_blocks;
+void used(const void* p, int device) {
+    std::lock_guard<std::mutex> lk(pinned_lock);
+    char* q = static_cast<char*>(const_cast<void*>(p));
+    auto b = pinned_blocks.upper_bound(q);
+    if (b == pinned_blocks.begin()) return;
+    --b;
+    if (q < b->first + b->second.bytes) b->second.used_by.insert(device);
+}
 bool refuse_copies = false;
 
 Stream* of(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
@@ -46,13 +63,22 @@ hipStream_t handle(Stream& s) { return reinterpret_cast<hipStream_t>(&s); }
 }  // namespace
 
 extern "C" {
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    std::lock_guard<std::mutex> lk(pinned_lock);
+    if (!(*p = std::malloc(n))) return hipErrorOutOfMemory;
+    pinned_blocks[static_cast<char*>(*p)] = Pinned{n, current_device, {}};
+    return hipSuccess;
+}
 hipError_t hipHostFree(void* p) {
+    std::lock_guard<std::mutex> lk(pinned_lock);
+    pinned_blocks.erase(static_cast<char*>(p));
     std::free(p);
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
     if (refuse_copies) return hipErrorUnknown;
+    used(d, of(st)->device);
+    used(s, of(st)->device);
     of(st)->queue.push_back([=] { std::memcpy(d, s, n); });
     return hipSuccess;
 }
@@ -78,6 +104,18 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
 hipError_t hipEventSynchronize(hipEvent_t e) {
     Event* v = reinterpret_cast<Event*>(e);
     v->stream->run(v->upto);
+    return hipSuccess;
+}
+hipError_t hipStreamGetDevice(hipStream_t st, hipDevice_t* device) {
+    *device = of(st)->device;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* device) {
+    *device = current_device;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int device) {
+    current_device = device;
     return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t) { return "an error of the test"; }
@@ -207,6 +245,26 @@ void two_engines() {
     expect(in_time, "the second engine's copies do not wait for the first engine's stream");
 }
 
+// Engines on two devices of one process, one after another and in turn, whichever device is the current one: an event
+// can only be recorded on a stream of the device it was made on, and pinned memory belongs to the device that allocated it.
+void two_devices() {
+    const size_t n = size_t(3) << 20;   // two pieces, each with an event
+    for (int k = 0; k < 8; ++k) {
+        Stream st;
+        st.device = k / 2 % 2;
+        current_device = k % 2;
+        std::vector<char> src(n, static_cast<char>(k)), back(n, 99);
+        mdp::EngineCopies c(handle(st));
+        c.get(back.data(), src.data(), n);
+        c.finish();
+        expect(back == src, "bytes as they were");
+        expect(current_device == k % 2, "the current device is left as it was");
+    }
+    for (const auto& b : pinned_blocks)
+        for (int d : b.second.used_by)
+            expect(d == b.second.device, "pinned memory is used by the device it was allocated for");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -217,6 +275,8 @@ int main(int argc, char** argv) {
         unwind();
     else if (what == "two_engines")
         two_engines();
+    else if (what == "two_devices")
+        two_devices();
     else
         return 2;
     std::printf("ok\n");

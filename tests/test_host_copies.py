@@ -1,5 +1,6 @@
 """The pinned-chunk copies (mdp_amd/csrc/host_copy.cpp) on the CPU, against played HIP calls (host_copies_cpu.cpp): every
-size around the limits they are cut at, byte for byte; what has to hold when a call fails and when several engines copy at once.
+size around the limits they are cut at, byte for byte; what has to hold when a call fails and when several engines, on one device
+or two, copy at once.
 """
 import os
 import subprocess
@@ -20,7 +21,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("what", ["bytes", "unwind", "two_engines"])
+@pytest.mark.parametrize("what", ["bytes", "unwind", "two_engines", "two_devices"])
 def test_host_copies(program, what):
     r = subprocess.run([program, what], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     print(r.stdout)
