@@ -464,9 +464,19 @@ void cpuSnapComputeFi(double* fatom, double* vatom, double* ylist_r, double* yli
         s.rfac0 = rfac0;
         s.rmin0 = rmin0;
         s.switchflag = switchflag;
+        int top_a = -1, top_b = -1, top_c = -1, atom = 0, centre = 0;   // largest of each; negative where an index is
+        for (int p = 0; p < ijnum; ++p) {
+            top_a = std::max(top_a, ai[p]);
+            top_b = std::max(top_b, aj[p]);
+            top_c = std::max(top_c, aii[p]);
+            atom |= ai[p] | aj[p];
+            centre |= aii[p];
+        }
+        if (centre < 0 || top_c >= inum) throw Error("SnapComputeFi: pair centre index out of range [0, inum)");
+        if (atom < 0) throw Error("SnapComputeFi: negative pair atom index");
         const size_t nu = static_cast<size_t>(inum) * idxu_max * nelem;
-        const int fext = std::max(max_of(ai, ijnum), max_of(aj, ijnum)) + 1;
-        const int vext = max_of(ai, ijnum) + 1;
+        const int fext = std::max(top_a, top_b) + 1;
+        const int vext = top_a + 1;
         std::vector<long> yb;
         if (chemflag) {
             yb.resize(ijnum);
@@ -804,7 +814,10 @@ template <size_t K>
 void index_ranges(const int* const (&a)[K], int n, IndexRange (&r)[K], hipStream_t st) {
     int* d = dev<int>(38, 3 * K);
     MDP_HIP(hipMemsetAsync(d, 0x80, sizeof(int) * 3 * K, st));
-    for (size_t k = 0; k < K; ++k) launch_index_range(a[k], n, d + 3 * k, st);
+    IndexArrays arrays = {};
+    static_assert(K <= sizeof(arrays.a) / sizeof(arrays.a[0]), "one launch takes them all");
+    std::copy(a, a + K, arrays.a);
+    launch_index_range(arrays, K, n, d, st);
     get(reinterpret_cast<int*>(r), d, 3 * K, st);
     finish(st);
 }
@@ -1033,11 +1046,14 @@ void mdp_hipSnapComputeFi(double* fatom, double* vatom, double* ylist_r, double*
         fetch_args([&] {
             if (ijnum <= 0) return;
             hipStream_t st = library_stream();
-            const int* const arr[2] = {ai, aj};
-            IndexRange r[2];
+            const int* const arr[3] = {ai, aj, aii};
+            IndexRange r[3];
             index_ranges(arr, ijnum, r, st);
             if (r[0].max >= anum || r[1].max >= anum)
                 throw Error("SnapComputeFi: a pair atom index is not below anum");
+            if (r[0].neg_min > 0 || r[1].neg_min > 0) throw Error("SnapComputeFi: negative pair atom index");
+            if (r[2].neg_min > 0 || r[2].max >= inum)
+                throw Error("SnapComputeFi: pair centre index out of range [0, inum)");
             SnapDev s = device_tables(twojmax, rootpqarray, radelem, wjelem, map, st);
             if (idxu_max != s.idxu_max) throw Error("idxu_max does not match twojmax");
             s.rcutfac = rcutfac;

@@ -116,9 +116,12 @@ void exclusive_scan(const int* in, int* out, int n, int* tmp, hipStream_t st) {
 // checks of a caller's device-resident pair arrays
 // ================================================================================================
 
-// out[0] = max, out[1] = max of -value, out[2] = 1 when a value is smaller than the one before it (out cleared to a
-// value below all of them).  One pass on the device instead of a read-back and three host loops (315,000 pairs: 0.6 ms).
-__global__ __launch_bounds__(256) void k_index_range(const int* __restrict__ a, int n, int* __restrict__ out) {
+// Of array b (blockIdx.y): out[3b] = max, out[3b + 1] = max of -value, out[3b + 2] = 1 when a value is smaller than the one
+// before it (out cleared to a value below all of them).  One pass on the device instead of a read-back and three host loops
+// (315,000 pairs: 0.6 ms).
+__global__ __launch_bounds__(256) void k_index_range(IndexArrays arrays, int n, int* __restrict__ out) {
+    const int* __restrict__ a = arrays.a[blockIdx.y];
+    out += 3 * blockIdx.y;
     int hi = -2147483647, lo = -2147483647, drop = 0;
     for (int p = blockIdx.x * 256 + threadIdx.x; p < n; p += 256 * gridDim.x) {
         const int v = a[p];
@@ -146,10 +149,10 @@ __global__ __launch_bounds__(256) void k_index_range(const int* __restrict__ a, 
     }
 }
 
-void launch_index_range(const int* a, int n, int* out, hipStream_t st) {
-    if (n <= 0) return;
+void launch_index_range(const IndexArrays& a, int count, int n, int* out, hipStream_t st) {
+    if (n <= 0 || count <= 0) return;
     // at most 128 workgroups, one atomic per word each: 2,048 waves' atomics on the same words took 57 us
-    hipLaunchKernelGGL(k_index_range, dim3(std::min(128, static_cast<int>(nblk(n, 256)))), dim3(256), 0, st, a, n, out);
+    hipLaunchKernelGGL(k_index_range, dim3(std::min(128, nblk(n, 256)), count), dim3(256), 0, st, a, n, out);
 }
 
 // off[i] = first position p of the ascending array a[0..n) with a[p] >= i, for i = 0 .. m (all values in [0, m))

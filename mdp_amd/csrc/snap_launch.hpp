@@ -264,8 +264,12 @@ void launch_tally_virial_full(double* vatom, const double* fij, const double* ri
 // AddWself2Ui on device (wself on the diagonal, mirror of rows 2mb < j)
 void launch_add_wself(const SnapDev& s, double* Ur, double* Ui, double wself, const int* type, int wselfall,
                       int chemflag, int nelem, int inum, hipStream_t st);
-// out[0..2] = max, max of -value, and 1 when not ascending, of a[0..n); out cleared to a value below all of them
-void launch_index_range(const int* a, int n, int* out, hipStream_t st);
+// out[3b .. 3b + 2] = max, max of -value, and 1 when not ascending, of a[b][0..n), b < count <= 3; out cleared to a value
+// below all of them
+struct IndexArrays {
+    const int* a[3];
+};
+void launch_index_range(const IndexArrays& a, int count, int n, int* out, hipStream_t st);
 // CSR offsets off[0..m] of the ascending array a[0..n) with values in [0, m)
 void launch_csr_of_sorted(const int* a, int n, int* off, int m, hipStream_t st);
 // *differs = 1 where U (one element) is not its own mirror image, as AddWself2Ui leaves it

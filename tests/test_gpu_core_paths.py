@@ -123,3 +123,31 @@ def test_forces_on_atoms_out_of_range_are_refused(gpu):
         *a("map", "ai", "ai", "aj", "ti", "tj"), 4, s.idxu_max, 20, 20, 300, 1, 0)
     assert "not below anum" in mdp_amd.last_error()
     assert np.all(d["f"].numpy() == 0.75) and np.all(d["v"].numpy() == 0.75)
+
+
+@pytest.mark.parametrize("route", ["device", "device, elements", "host"])
+@pytest.mark.parametrize("array,value", [("ai", -1), ("aj", -2147483648), ("aii", -1), ("aii", 20)])
+def test_negative_and_centre_indices_of_forces_are_refused(gpu, route, array, value):
+    """20 atoms; the device arrays also through the element-mapped route, and the host arrays.  Nothing is written."""
+    import mdp_amd
+    from mdp_amd.devarray import DevArray
+    s, p = _sna(gpu, 4), _pairs(20, 300, 1, 1)
+    q = dict(aii=p["ai"].copy(), ai=p["ai"].copy(), aj=p["aj"].copy(), ti=p["ti"], tj=p["tj"])
+    q[array][150] = value
+    y, f, v = np.ones(20 * s.idxu_max), np.full(60, 0.75), np.full(120, 0.75)
+    print(route, array, value, flush=True)
+    if route == "host":
+        gpu.cpuSnapComputeFi(f, v, y, y, s.rootpqarray, p["rij"], s.wjelem, s.radelem, s.rmin0, s.rfac0, s.rcutfac, s.map,
+                             q["aii"], q["ai"], q["aj"], q["ti"], q["tj"], 4, s.idxu_max, 20, 20, 300, 1, 0)
+        message = mdp_amd.last_error()
+    else:
+        d = {k: DevArray.from_numpy(a) for k, a in dict(q, rp=s.rootpqarray, rij=p["rij"], wj=s.wjelem, rad=s.radelem,
+                                                        map=s.map, Y=y, f=f, v=v).items()}
+        a = lambda *k: [d[x].ptr for x in k]  # noqa: E731
+        _fn(gpu, "SnapComputeFi", "pppppppp" "ddd" "ppppppp" "iiiiiii")(
+            *a("f", "v", "Y", "Y", "rp", "rij", "wj", "rad"), s.rmin0, s.rfac0, s.rcutfac, None,
+            *a("map", "aii", "ai", "aj", "ti", "tj"), 4, s.idxu_max, 20, 20, 300, 1, int("elements" in route))
+        message = mdp_amd.last_error()
+        f, v = d["f"].numpy(), d["v"].numpy()
+    assert ("centre index out of range" if array == "aii" else "negative pair atom index") in message
+    assert np.all(f == 0.75) and np.all(v == 0.75)
