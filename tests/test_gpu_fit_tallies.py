@@ -1,6 +1,6 @@
 """Tallies and normal equations of the batched fit where their kernels change form: configurations around the
 number of threads of a workgroup and above what it holds, atoms with long incoming lists, every number of 16-column
-tiles of the normal equations, several element types.
+tiles of the normal equations (1 to 5), several element types.
 
 Reference: numpy in float64 on the engine's own B, dB/dr and pair list.  Sums of m terms, m <= 200,000 here, differ by
 at most m 2^-53 of the sum of the magnitudes; the orders used keep it far below the 1e-11 allowed.
@@ -47,12 +47,14 @@ def _reference(fit, configs, types):
 
 
 @pytest.mark.parametrize("sizes,J,types", [([2, 511, 512, 513], 4, 1), ([2047, 1, 65], 2, 1), ([2100, 30], 4, 1),
-                                           ([64, 40], 8, 1), ([63, 100], 6, 1), ([128, 60], 6, 2)])
+                                           ([64, 40], 8, 1), ([63, 100], 6, 1), ([128, 60], 6, 2), ([70, 33], 4, 3),
+                                           ([60, 95], 4, 5)])
 def test_tallies_and_normal_equations(sizes, J, types):
     configs = [_config(n, 40 + k, types=types) for k, n in enumerate(sizes)]
     if sizes[0] == 64:   # tightly packed cells: more than 128 incoming pairs per atom
         configs.append(_config(54, 90, a=1.7))
-    fit = SnapFit(configs, J, elemradius=(0.5, 0.47)[:types], elemweight=(1.0, 0.8)[:types])
+    fit = SnapFit(configs, J, elemradius=(0.5, 0.47, 0.45, 0.52, 0.49)[:types],
+                  elemweight=(1.0, 0.8, 0.9, 1.1, 0.7)[:types])
     fit.compute()
     ref = _reference(fit, configs, types)
     print(f"tallies {sizes} J={J} types={types}", flush=True)
