@@ -40,9 +40,8 @@ struct mdp_fit {
     std::vector<int> a0_h;   // [C+1]
     std::vector<double> boxes_h, tilts_h;   // tilts_h empty: every cell orthogonal
     DevBuf x, type, cfg_of, cfg_a0, cfg_L, cfg_T, cfg_p0, rc2, pcnt, poff, scan_tmp, flags, counter;
-    std::vector<int> cfg_ord_h;
-    int n_large = 0;    // how many of them the tallies treat as large (lsq_large_configuration)
-    DevBuf cfg_ord;     // configurations, most atoms first
+    DevBuf cfg_ord;                // configurations, most atoms first
+    std::vector<int> cfg_size_h;   // their atom counts, in that order
     DevBuf chunk_ord;   // 64-atom chunks of the pair build, most candidate tests first
     DevBuf pi, pj, pti, ptj, rij, Ur, Ui, zt, blist, bpart, dblist, bzero, t_lo, t_b, t_z, t_w, zorder, t_wtab, t_hlo, t_hb, t_hz,
         t_hw, t_mz, t_mw, t_mcomb, pgeo;
@@ -181,15 +180,13 @@ struct mdp_fit {
             std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return cost[a] > cost[b]; });
             put(chunk_ord, ord.data(), sizeof(int) * std::max(nch, 1));
         }
-        cfg_ord_h.resize(C);
-        for (int c = 0; c < C; ++c) cfg_ord_h[c] = c;
-        std::stable_sort(cfg_ord_h.begin(), cfg_ord_h.end(),
+        std::vector<int> by_size(C);
+        for (int c = 0; c < C; ++c) by_size[c] = c;
+        std::stable_sort(by_size.begin(), by_size.end(),
                          [&](int a, int b) { return a0_h[a + 1] - a0_h[a] > a0_h[b + 1] - a0_h[b]; });
-        put(cfg_ord, cfg_ord_h.data(), sizeof(int) * C);
-        for (n_large = 0; n_large < C; ++n_large) {
-            const int c = cfg_ord_h[n_large];
-            if (a0_h[c + 1] - a0_h[c] <= lsq_large_configuration()) break;
-        }
+        put(cfg_ord, by_size.data(), sizeof(int) * C);
+        cfg_size_h.resize(C);
+        for (int k = 0; k < C; ++k) cfg_size_h[k] = a0_h[by_size[k] + 1] - a0_h[by_size[k]];
         put(bzero, bz.data(), sizeof(double) * bz.size());
         put(t_lo, lo.data(), sizeof(int) * lo.size());
         put(t_b, tb.data(), sizeof(int) * tb.size());
@@ -486,12 +483,6 @@ struct mdp_fit {
         MDP_HIP(hipGraphLaunch(gexec, st));
     }
 
-    int max_natoms() const {
-        int m = 0;
-        for (int c = 0; c < C; ++c) m = std::max(m, a0_h[c + 1] - a0_h[c]);
-        return m;
-    }
-
     // Tallies of the last compute for the linear fit (upstream cpuSnapTallyBispectrum{,Deriv,Virial}
     // layouts per configuration) and the stress rows of the fit.
     void lsq_tallies() {
@@ -509,8 +500,8 @@ struct mdp_fit {
                             scan_tmp.as<int>(), st);
         launch_lsq_tallies(blist.as<double>(), dblist.as<double>(), rij.as<double>(), poff.as<int>(), l_off.as<int>(),
                            l_idx.as<int>(), pti.as<int>(), type.as<int>(), cfg_of.as<int>(), cfg_a0.as<int>(),
-                           cfg_p0.as<int>(), cfg_ord.as<int>(), n_large, C, N, IB, ntypes, max_natoms(), l_bi.as<double>(), l_bd.as<double>(),
-                           l_bv.as<double>(), l_as.as<double>(), st);
+                           cfg_p0.as<int>(), cfg_ord.as<int>(), cfg_size_h.data(), C, N, IB, ntypes, l_bi.as<double>(),
+                           l_bd.as<double>(), l_bv.as<double>(), l_as.as<double>(), st);
         MDP_HIP(hipGetLastError());
     }
 

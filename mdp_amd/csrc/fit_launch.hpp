@@ -104,12 +104,11 @@ void launch_lsq_incoming(const int* pj, long P, int N, int* in_cnt, int* in_off,
                          int* scan_tmp, hipStream_t st);
 // per configuration c: bi[c*Kt + col], bd at 3*a0_c*Kt ([comp + 3 ii + 3 N_c col]), bv[c*6*Kt + 6 col + m]
 // (upstream tally layouts, Kt = ntypes*IB, col = (type-1)*IB + k) and the stress rows as[(6c + m')*Kt + col];
-// cfg_ord: the configurations, largest first, of which n_large have more than lsq_large_configuration() atoms
-int lsq_large_configuration();
+// cfg_ord: the configurations, largest first; sizes (on the host): their atom counts in that order
 void launch_lsq_tallies(const double* blist, const double* dblist, const double* rij, const int* poff,
                         const int* in_off, const int* in_idx, const int* pti, const int* type, const int* cfg_of,
-                        const int* cfg_a0, const int* cfg_p0, const int* cfg_ord, int n_large, int C, int N, int IB,
-                        int ntypes, int max_natoms, double* bi, double* bd, double* bv, double* as, hipStream_t st);
+                        const int* cfg_a0, const int* cfg_p0, const int* cfg_ord, const int* sizes, int C, int N,
+                        int IB, int ntypes, double* bi, double* bd, double* bv, double* as, hipStream_t st);
 // out[0 .. K(K+1)/2) = upper triangle of sum w^2 a a^T (row-major), out[K(K+1)/2 + k] = sum w^2 a_k b;
 // part: G * (K(K+1)/2 + K) doubles; K <= lsq_gram_max_columns()
 int lsq_gram_max_columns();

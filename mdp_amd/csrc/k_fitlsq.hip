@@ -9,6 +9,8 @@
 // Every sum runs in a fixed order, so the results do not depend on scheduling.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "fit_launch.hpp"
 #include "runtime.hpp"
 #include "snap_launch.hpp"
@@ -132,12 +134,13 @@ __global__ void k_lsq_bd(const double* __restrict__ dblist, const int* __restric
 // of k through LDS in tiles of BD_TILE pairs, adds each pair's virial on the way, and then every atom adds its own
 // pairs of the tile and subtracts its incoming ones (both ascending), in registers of the thread that owns it: up to
 // H atoms per thread.  The indices of an atom's next two incoming pairs are kept loaded: a tile without one costs no
-// memory access, and one load's latency passes behind the other's pair.  Configurations come largest first (cfg_ord),
-// those of more than BD_TH atoms in a launch of their own.  105,000 atoms, 2.1 M pairs, twojmax 8:
+// memory access, and one load's latency passes behind the other's pair.  Configurations come largest first (cfg_ord), those
+// of more than BD_TH and of more than 4 BD_TH atoms in launches of their own, so that small ones don't carry the registers of
+// large ones.  105,000 atoms, 2.1 M pairs, twojmax 8:
 // 1,312 us (2.1 TB/s); a pass per plane for bd and a second read of dB/dr for the virial took 1,841 + 813 us.
 // bv[c*6*Kt + 6*k + m], components m = (xx, yy, zz, xy, xz, yz); as[(6c + m')*Kt + k] are the same as the stress rows of
 // the fit, in the upstream row order m' -> m = (0, 1, 2, 5, 4, 3) (snapcpp.jl:660-662).
-constexpr int BD_TILE = 1280, BD_TH = 512, BD_MAXH = 4;
+constexpr int BD_TILE = 1280, BD_TH = 512, BD_MAXH = 6;
 
 template <int H>
 __global__ __launch_bounds__(BD_TH) void k_lsq_bd_bv(const double* __restrict__ dblist, const double* __restrict__ rij,
@@ -303,19 +306,27 @@ __global__ __launch_bounds__(256) void k_lsq_bv(const double* __restrict__ dblis
 
 void launch_lsq_tallies(const double* blist, const double* dblist, const double* rij, const int* poff,
                         const int* in_off, const int* in_idx, const int* pti, const int* type, const int* cfg_of,
-                        const int* cfg_a0, const int* cfg_p0, const int* cfg_ord, int n_large, int C, int N, int IB,
-                        int ntypes, int max_natoms, double* bi, double* bd, double* bv, double* as, hipStream_t st) {
+                        const int* cfg_a0, const int* cfg_p0, const int* cfg_ord, const int* sizes, int C, int N,
+                        int IB, int ntypes, double* bi, double* bd, double* bv, double* as, hipStream_t st) {
     const int kt = ntypes * IB;
-    // one element type and at most BD_MAXH atoms per thread: one read of dB/dr for both tallies
-    const int per_thread = (max_natoms + BD_TH - 1) / BD_TH;
-    const bool fused = ntypes == 1 && per_thread <= BD_MAXH;
+    // One element type and at most BD_MAXH atoms per thread (3,072 atoms) in any configuration: one read of dB/dr for both
+    // tallies.  24 configurations of 2,500 atoms, twojmax 8, tallies and the energy row: 970 us, against 6,990 with the thread
+    // per atom and descriptor and the second read that larger ones take; 200 of 250 atoms and one of 2,500: 900 against 6,240.
+    const bool fused = ntypes == 1 && (C == 0 || sizes[0] <= BD_MAXH * BD_TH);
     if (fused) {
-        if (n_large > 0)
-            hipLaunchKernelGGL(k_lsq_bd_bv<BD_MAXH>, dim3(static_cast<unsigned>(n_large) * IB), dim3(BD_TH), 0, st, dblist,
-                               rij, poff, in_off, in_idx, cfg_a0, cfg_p0, cfg_ord, IB, bd, bv, as);
-        if (n_large < C)
-            hipLaunchKernelGGL(k_lsq_bd_bv<1>, dim3(static_cast<unsigned>(C - n_large) * IB), dim3(BD_TH), 0, st, dblist,
-                               rij, poff, in_off, in_idx, cfg_a0, cfg_p0, cfg_ord + n_large, IB, bd, bv, as);
+        // configurations of more than `atoms` atoms: the first so many of cfg_ord
+        auto above = [&](int atoms) {
+            return static_cast<int>(std::partition_point(sizes, sizes + C, [&](int n) { return n > atoms; }) - sizes);
+        };
+        const int n4 = above(4 * BD_TH), n1 = above(BD_TH);
+        auto launch = [&](auto kernel, int first, int end) {
+            if (first < end)
+                hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(end - first) * IB), dim3(BD_TH), 0, st, dblist, rij, poff,
+                                   in_off, in_idx, cfg_a0, cfg_p0, cfg_ord + first, IB, bd, bv, as);
+        };
+        launch(k_lsq_bd_bv<BD_MAXH>, 0, n4);
+        launch(k_lsq_bd_bv<4>, n4, n1);
+        launch(k_lsq_bd_bv<1>, n1, C);
     } else {
         hipLaunchKernelGGL(k_lsq_bd, dim3(nblocks(static_cast<long>(N) * IB, 256)), dim3(256), 0, st, dblist, poff,
                            in_off, in_idx, pti, type, cfg_of, cfg_a0, cfg_p0, N, IB, ntypes, bd);
@@ -421,8 +432,6 @@ __global__ __launch_bounds__(1024) void k_lsq_gram_sum(const double* __restrict_
     for (int k = 1; k < 16; ++k) s += sum[k][lane];
     out[e] = s;
 }
-
-int lsq_large_configuration() { return BD_TH; }
 
 int lsq_gram_max_columns() { return 77; }
 

@@ -5,6 +5,8 @@ tiles of the normal equations (1 to 5), several element types.
 Reference: numpy in float64 on the engine's own B, dB/dr and pair list.  Sums of m terms, m <= 200,000 here, differ by
 at most m 2^-53 of the sum of the magnitudes; the orders used keep it far below the 1e-11 allowed.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -46,7 +48,8 @@ def _reference(fit, configs, types):
     return out
 
 
-@pytest.mark.parametrize("sizes,J,types", [([2, 511, 512, 513], 4, 1), ([2047, 1, 65], 2, 1), ([2100, 30], 4, 1),
+@pytest.mark.parametrize("sizes,J,types", [([2, 511, 512, 513], 4, 1), ([2047, 1, 65], 2, 1), ([2048, 2049, 30], 4, 1),
+                                           ([3072, 513, 2100], 2, 1), ([3073, 40], 2, 1),
                                            ([64, 40], 8, 1), ([63, 100], 6, 1), ([128, 60], 6, 2), ([70, 33], 4, 3),
                                            ([60, 95], 4, 5)])
 def test_tallies_and_normal_equations(sizes, J, types):
@@ -81,3 +84,28 @@ def test_tallies_and_normal_equations(sizes, J, types):
         at += n
     assert np.all(np.abs(L - Lr) <= 1e-11 * (Lm + 1e-300))
     assert np.all(np.abs(h - hr) <= 1e-11 * (hm + 1e-300))
+
+
+def _tally_time(sizes, J=8):
+    """median microseconds per thousand pairs of the tallies, the energy row's normal equations with them"""
+    fit = SnapFit([_config(n, 10 + k) for k, n in enumerate(sizes)], J)
+    fit.compute()
+    e = np.ones(len(sizes))
+    t = []
+    for _ in range(9):
+        t0 = time.perf_counter()
+        fit.normal_equations(e, None, None, e, e, e)
+        t.append(time.perf_counter() - t0)
+    pairs = len(fit.pairs()[0])
+    fit.close()
+    return 1e9 * float(np.median(t)) / pairs
+
+
+def test_a_larger_configuration_does_not_slow_the_batch():
+    """Configurations of 2,049 to 2,730 atoms, alone and as one of many, keep about the rate of smaller ones.  The form that
+    reads dB/dr pair by pair takes six to nine times as long; twice allows for the clock."""
+    small, many = _tally_time([2000] * 24), _tally_time([250] * 200)
+    for sizes, rate in (([2500] * 24, small), ([2730] * 24, small), ([250] * 200 + [2500], many)):
+        now = _tally_time(sizes)
+        print(f"{len(sizes)} configurations, largest {max(sizes)}: {now:.2f} us per 1,000 pairs, {rate:.2f} without", flush=True)
+        assert now < 2 * rate
