@@ -809,6 +809,32 @@ __global__ __launch_bounds__(AB * SUB / PARTS) void k_pair_list(const double* __
     }
 }
 
+// The pair potential's sums alone, SUB lanes per atom in the order of k_pair_list: where its time is asked for, which the pair
+// list's launch cannot show.
+template <int SUB>
+__global__ __launch_bounds__(256) void k_zbl(const double* __restrict__ x, const int* __restrict__ nb_cnt,
+                                             const int2* __restrict__ nbr, double Lx, double Ly, double Lz, int N,
+                                             ZblParams zp, double* __restrict__ zacc) {
+    const int al = threadIdx.x / SUB, sub = threadIdx.x % SUB, i = blockIdx.x * (256 / SUB) + al;
+    const bool live = i < N;
+    const int n = live ? nb_cnt[i] : 0;
+    const int2* __restrict__ list = nbr + static_cast<size_t>(i) * NBMAX;
+    double za[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    for (int k = sub; k < n; k += SUB) {
+        const int2 e = list[k];
+        double dx, dy, dz;
+        entry_disp(x, i, e.x, e.y, Lx, Ly, Lz, dx, dy, dz);
+        zbl_add(zp, dist2_nc(dx, dy, dz), dx, dy, dz, za);
+    }
+#pragma unroll
+    for (int w = SUB / 2; w >= 1; w /= 2)
+#pragma unroll
+        for (int k = 0; k < 10; ++k) za[k] += __shfl_xor(za[k], w);
+    if (live && sub == 0)
+#pragma unroll
+        for (int k = 0; k < 10; ++k) zacc[10 * static_cast<size_t>(i) + k] = za[k];
+}
+
 // f, per-atom virial and energy of atom i without atomics; optionally the second velocity half-step (integrate
 // 1), and with it the first half-step and drift of the next step (2).
 // 16 lanes per atom: lane s takes the atom's pairs s, s+16, ... and incoming entries s, s+16, ... (the
@@ -1253,25 +1279,40 @@ struct mdp_md {
     int pair_atoms() const { return N <= PAIR_SMALL ? 16 : 64; }   // atoms per block of the pair list
     int pair_blocks() const { return (N + pair_atoms() - 1) / pair_atoms(); }
 
-    // pair list (and the reference pair potential of every atom into zacc, added by the tally that follows)
+    // pair list (and the reference pair potential of every atom into zacc, added by the tally that follows; in a launch of its
+    // own where that is timed)
     void pairs() {
-        auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(pair_blocks()), dim3(512), 0, st, x.as<double>(), type.as<int>(),
-                               nb_cnt.as<int>(), nbr.as<int2>(), rc2.as<double>(), ntypes, pair_base.as<int>(),
-                               block_np.as<int>(), poff.as<int>(), pend.as<int>(), pi.as<int>(), pti.as<int>(),
-                               ptj.as<int>(), prij.as<double>(), entry_pair.as<int>(), L[0], L[1], L[2], N, tab.view,
-                               pgeo.as<double>(), zp, zacc.as<double>());
-        };
-        if (N <= PAIR_SMALL) {
-            if (zbl)
-                launch(k_pair_list<true, 16, 32, 1>);
+        const bool apart = zbl && timing && (timing_mask & (1u << T_PAIRPOT)), with = zbl && !apart;
+        timed(T_PAIRS, [&] {
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(pair_blocks()), dim3(512), 0, st, x.as<double>(), type.as<int>(),
+                                   nb_cnt.as<int>(), nbr.as<int2>(), rc2.as<double>(), ntypes, pair_base.as<int>(),
+                                   block_np.as<int>(), poff.as<int>(), pend.as<int>(), pi.as<int>(), pti.as<int>(),
+                                   ptj.as<int>(), prij.as<double>(), entry_pair.as<int>(), L[0], L[1], L[2], N, tab.view,
+                                   pgeo.as<double>(), zp, zacc.as<double>());
+            };
+            if (N <= PAIR_SMALL) {
+                if (with)
+                    launch(k_pair_list<true, 16, 32, 1>);
+                else
+                    launch(k_pair_list<false, 16, 32, 1>);
+            } else if (with) {
+                launch(k_pair_list<true, 64, 16, 2>);
+            } else {
+                launch(k_pair_list<false, 64, 16, 2>);
+            }
+        });
+        if (!apart) return;
+        timed(T_PAIRPOT, [&] {
+            auto launch = [&](auto kernel, int sub) {
+                hipLaunchKernelGGL(kernel, dim3(nb(static_cast<long>(N) * sub, 256)), dim3(256), 0, st, x.as<double>(),
+                                   nb_cnt.as<int>(), nbr.as<int2>(), L[0], L[1], L[2], N, zp, zacc.as<double>());
+            };
+            if (N <= PAIR_SMALL)
+                launch(k_zbl<32>, 32);
             else
-                launch(k_pair_list<false, 16, 32, 1>);
-        } else if (zbl) {
-            launch(k_pair_list<true, 64, 16, 2>);
-        } else {
-            launch(k_pair_list<false, 64, 16, 2>);
-        }
+                launch(k_zbl<16>, 16);
+        });
     }
 
     void dedr_launch(int variant) {
@@ -1592,7 +1633,7 @@ struct mdp_md {
 
     void compute() {
         timed(T_REBUILD, [&] { rebuild(false); });
-        timed(T_PAIRS, [&] { pairs(); });
+        pairs();
         snap_and_tally(0);
         if (!tuned) {
             autotune();
@@ -1731,7 +1772,7 @@ struct mdp_md {
             begun = false;
             stats[4] += 1;
             if (stats[4] % rebuild_every == 0) timed(T_REBUILD, [&] { rebuild(true); });
-            timed(T_PAIRS, [&] { pairs(); });
+            pairs();
             const bool aud = sur && audit_every > 0 && stats[4] % audit_every == 0;
             const int integrate = aud ? 0 : (next && !nvt ? 2 : 1);
             if (sur)

@@ -176,3 +176,23 @@ def test_md_snap_plus_zbl_energy_error_scales_with_dt2(oracle):
         md.close()
     ratio = dev[0] / dev[1]
     assert 3.0 < ratio < 5.0, (dev, ratio)
+
+
+@pytest.mark.parametrize("ncell", [4, 21])
+def test_pair_potential_timer(oracle, ncell):
+    """With every stage timed the pair potential is a launch of its own (128 atoms, and 18,522, above the pair list's small
+    blocks): recorded in every step, and the same forces, to rounding, as in the pair list's launch."""
+    J = 2
+    x, box = lattice.crystal("bcc", ncell, 3.0, 0.1, 5)
+    out = []
+    for timed in (0, 1):
+        md = _snap_zbl_engine(oracle, J, x, box, _coeff(oracle, J, 7))
+        md.compute()
+        md.set_timing(timed)
+        md.run(3)
+        out.append(md.state())
+        ms, launches = md.timers()["pair_potential"]
+        assert launches == 3 * timed and (ms > 0.0) == bool(timed)
+        md.close()
+    for k in ("f", "eatom", "vatom"):
+        assert relerr(out[0][k], out[1][k]) < 1e-12, k
