@@ -1201,12 +1201,13 @@ struct mdp_md {
     void ensure_pairs(size_t cap) {
         if (pi.cap >= sizeof(int) * std::max<size_t>(cap, 1)) return;
         const size_t c = cap + cap / 4 + 64;
-        pi.ensure(sizeof(int) * c);
+        pi.release();   // its capacity stands for all of them: it comes last
         pti.ensure(sizeof(int) * c);
         ptj.ensure(sizeof(int) * c);
         prij.ensure(sizeof(double) * 3 * c);
         pgeo.ensure(sizeof(double) * 5 * c);
         dedr.ensure(sizeof(double) * 3 * c);
+        pi.ensure(sizeof(int) * c);
     }
 
     // the cell-list neighbour kernel: 0 = eight lanes per atom through L1, 1 = the LDS tile on 128 lanes per cell,
@@ -1771,7 +1772,11 @@ struct mdp_md {
             }
             begun = false;
             stats[4] += 1;
-            if (stats[4] % rebuild_every == 0) timed(T_REBUILD, [&] { rebuild(true); });
+            if (stats[4] % rebuild_every == 0) {
+                forces_current = false;   // a rebuild that fails leaves a list that the pair arrays may have no room for
+                timed(T_REBUILD, [&] { rebuild(true); });
+                forces_current = true;
+            }
             pairs();
             const bool aud = sur && audit_every > 0 && stats[4] % audit_every == 0;
             const int integrate = aud ? 0 : (next && !nvt ? 2 : 1);

@@ -5,7 +5,7 @@
   cell-list builder truncates silently, cpuNeighborList3D.cpp:399-409.)
 * Non-finite positions or velocities: rejected when the engine is created and when the host sets a new
   state, leaving the engine usable; a coordinate that runs away during a run (a velocity of 1e300 A/ps,
-  finite but unphysical) is reported by the next neighbour rebuild.
+  finite but unphysical) is reported by the next neighbour rebuild.  A run after a failed rebuild reports it again.
 * Coincident atoms: the drop-in pair filter drops pairs with r^2 <= 1e-20 (cpuSnap.cpp:278) exactly as the
   oracle does, and the MD engine's pair list does the same, so forces stay finite.
 """
@@ -67,6 +67,24 @@ def test_runaway_position_reported_by_rebuild():
     md.compute()
     with pytest.raises(RuntimeError, match="runaway"):
         md.run(3)
+
+
+def test_a_failed_rebuild_is_not_run_on(oracle):
+    """Atoms that fall together in one step: the rebuild reports them, and so does a further run, which must not go on with a
+    list that its arrays have no room for; with a sound state the engine works as a new one."""
+    x, box = lattice.crystal("bcc", 10, 3.316, 0.05, 3)
+    dt = 0.0005
+    v = (0.5 * box - x) * (0.6 / dt)                     # to 0.4 of the distances in one step
+    md = _engine(x, box, v=v, every=1, dt=dt)
+    md.compute()
+    f0 = md.state()["f"]
+    for k in range(3):
+        print(f"run {k} of a collapsing crystal, {len(x)} atoms", flush=True)
+        with pytest.raises(RuntimeError, match="96 neighbours"):
+            md.run(1)
+    md.set_state(x, np.zeros_like(x))
+    md.run(0)
+    assert relerr(md.state()["f"], f0) < 1e-12
 
 
 def test_coincident_atoms_dropped(oracle):
