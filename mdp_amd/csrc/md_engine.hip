@@ -25,6 +25,7 @@
 #include <string>
 #include <cstring>
 #include <memory>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/mdpsnap.h"
@@ -576,15 +577,18 @@ constexpr int PSUB = 16;   // lanes that share an atom in the per-atom kernels
 
 // The pair list's blocks of `ab` atoms (16 or 64) divide the workgroup's 64: a block's room there is its entry count
 // rounded up to 64.
+// E is the type of an entry's number: int, or long above 22,369,621 atoms, where NBMAX N does not fit an int.
+template <class E>
 __global__ __launch_bounds__(1024) void k_incoming(const int* __restrict__ nb_cnt, const int2* __restrict__ nbr,
-                                                   int* __restrict__ in_cnt, int* __restrict__ in_e, int N,
+                                                   int* __restrict__ in_cnt, E* __restrict__ in_e, int N,
                                                    int* __restrict__ overflow, unsigned long long* __restrict__ total,
                                                    int* __restrict__ room, int ab) {
     __shared__ int part[64];
     const int al = threadIdx.x / PSUB, sub = threadIdx.x % PSUB, i = blockIdx.x * 64 + al;
     const int n = i < N ? nb_cnt[i] : 0;
     for (int k = sub; k < n; k += PSUB) {
-        const int e = i * NBMAX + k, j = nbr[e].x;
+        const E e = static_cast<E>(i) * NBMAX + k;
+        const int j = nbr[e].x;
         const int slot = atomicAdd(&in_cnt[j], 1);
         if (slot < NBMAX)
             in_e[static_cast<size_t>(j) * NBMAX + slot] = e;
@@ -608,17 +612,18 @@ __global__ __launch_bounds__(1024) void k_incoming(const int* __restrict__ nb_cn
 
 // ascending order of each atom's incoming list: 16 lanes per atom rank its entries from an LDS copy.  (One lane per
 // atom sorting by insertion took 20 us at 250 atoms and 63 us at 128,000.)
-__global__ __launch_bounds__(256) void k_incoming_sort(int* __restrict__ in_cnt, int* __restrict__ in_e, int N) {
+template <class E>
+__global__ __launch_bounds__(256) void k_incoming_sort(int* __restrict__ in_cnt, E* __restrict__ in_e, int N) {
     constexpr int APB = 256 / PSUB;
-    __shared__ int list[APB][NBMAX];
+    __shared__ E list[APB][NBMAX];
     const int t = blockIdx.x * 256 + threadIdx.x, i = t / PSUB, sub = t % PSUB;
-    int* __restrict__ a = in_e + static_cast<size_t>(i) * NBMAX;
-    int* l = list[threadIdx.x / PSUB];
+    E* __restrict__ a = in_e + static_cast<size_t>(i) * NBMAX;
+    E* l = list[threadIdx.x / PSUB];
     const int n = i < N ? min(in_cnt[i], NBMAX) : 0;
     for (int k = sub; k < n; k += PSUB) l[k] = a[k];
     __syncthreads();
     for (int k = sub; k < n; k += PSUB) {
-        const int v = l[k];
+        const E v = l[k];
         int rank = 0;
         for (int m = 0; m < n; ++m) rank += l[m] < v;
         a[rank] = v;
@@ -839,10 +844,11 @@ __global__ __launch_bounds__(256) void k_zbl(const double* __restrict__ x, const
 // 1), and with it the first half-step and drift of the next step (2).
 // 16 lanes per atom: lane s takes the atom's pairs s, s+16, ... and incoming entries s, s+16, ... (the
 // pair reads of a wave are then contiguous), and the 16 partial sums are combined by a butterfly.
+template <class E>
 __global__ __launch_bounds__(256) void k_tally(const double* __restrict__ dedr, const double* __restrict__ prij,
                                                const int* __restrict__ poff, const int* __restrict__ pend,
                                                const int* __restrict__ in_cnt,
-                                               const int* __restrict__ in_e, const int* __restrict__ entry_pair,
+                                               const E* __restrict__ in_e, const int* __restrict__ entry_pair,
                                                const double* __restrict__ epart, int nrows, double e0,
                                                const double* __restrict__ eext, double* __restrict__ f,
                                                double* __restrict__ vir, double* __restrict__ eatom,
@@ -1177,7 +1183,7 @@ struct mdp_md {
         scan_tmp.ensure(sizeof(int) * (scan_tmp_ints(static_cast<int>(std::max(n, ncells))) + 8));
         nb_cnt.ensure(sizeof(int) * n);
         nbr.ensure(sizeof(int2) * n * NBMAX);
-        in_e.ensure(sizeof(int) * n * NBMAX);
+        in_e.ensure((wide_entries() ? sizeof(long) : sizeof(int)) * n * NBMAX);
         poff.ensure(sizeof(int) * n);
         pend.ensure(sizeof(int) * n);
         pair_room.ensure(sizeof(int) * pair_blocks());
@@ -1248,12 +1254,14 @@ struct mdp_md {
             hipLaunchKernelGGL(k_neighbors_brute, dim3(nb(N, 4)), dim3(256), 0, st, x.as<double>(), nb_cnt.as<int>(),
                                nbr.as<int2>(), L[0], L[1], L[2], rcs, rcs * rcs, N, report()->flags);
         }
-        hipLaunchKernelGGL(k_incoming, dim3(nb(N, 64)), dim3(1024), 0, st, nb_cnt.as<int>(), nbr.as<int2>(),
-                           in_cnt(), in_e.as<int>(), N, report()->flags, &report()->entries, pair_room.as<int>(),
-                           pair_atoms());
-        exclusive_scan(pair_room.as<int>(), pair_base.as<int>(), pair_blocks(), scan_tmp.as<int>(), st);
-        hipLaunchKernelGGL(k_incoming_sort, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, in_cnt(),
-                           in_e.as<int>(), N);
+        with_entries([&](auto* e) {
+            using E = std::remove_pointer_t<decltype(e)>;
+            hipLaunchKernelGGL(k_incoming<E>, dim3(nb(N, 64)), dim3(1024), 0, st, nb_cnt.as<int>(), nbr.as<int2>(),
+                               in_cnt(), e, N, report()->flags, &report()->entries, pair_room.as<int>(), pair_atoms());
+            exclusive_scan(pair_room.as<int>(), pair_base.as<int>(), pair_blocks(), scan_tmp.as<int>(), st);
+            hipLaunchKernelGGL(k_incoming_sort<E>, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, in_cnt(),
+                               e, N);
+        });
         // a single small readback per rebuild: overflow flags, displacement and entry count
         MDP_HIP(hipMemcpyAsync(report_h, report(), sizeof(Report), hipMemcpyDeviceToHost, st));
         MDP_HIP(hipStreamSynchronize(st));
@@ -1275,6 +1283,15 @@ struct mdp_md {
         if (slots > 0x7fffffffL) throw Error("neighbour build failed: too many entries");
         pair_slots = static_cast<int>(slots);
         ensure_pairs(static_cast<size_t>(slots));
+    }
+
+    bool wide_entries() const { return static_cast<long>(N) * NBMAX > 0x7fffffffL; }
+    template <class F>
+    void with_entries(F&& f) {
+        if (wide_entries())
+            f(in_e.as<long>());
+        else
+            f(in_e.as<int>());
     }
 
     int pair_atoms() const { return N <= PAIR_SMALL ? 16 : 64; }   // atoms per block of the pair list
@@ -1381,13 +1398,21 @@ struct mdp_md {
         timed(T_DEDR, [&] {
             dedr_launch(dedr_variant);
         });
+        tally(epart.as<double>(), nrows, e0, nullptr, fo, vo, eo, integrate, count);
+    }
+
+    // forces, virials and energies of every atom from dE/dr: the energies from nrows partials each and e0, or from eext
+    void tally(const double* part, int rows, double first, const double* eext, double* fo, double* vo, double* eo,
+               int integrate, bool count) {
         timed(T_TALLY, [&] {
-            hipLaunchKernelGGL(k_tally, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, dedr.as<double>(), prij.as<double>(),
-                               poff.as<int>(), pend.as<int>(), in_cnt(), in_e.as<int>(), entry_pair.as<int>(),
-                               epart.as<double>(), nrows, e0, nullptr, fo, vo, eo, v.as<double>(),
-                               x.as<double>(), type.as<int>(), massinv.as<double>(), dtf, dt, integrate, N, block_np.as<int>(),
-                               pair_blocks(), count ? pair_sum.as<unsigned long long>() : nullptr,
-                               zbl ? zacc.as<double>() : nullptr);
+            with_entries([&](auto* e) {
+                using E = std::remove_pointer_t<decltype(e)>;
+                hipLaunchKernelGGL(k_tally<E>, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st,
+                                   dedr.as<double>(), prij.as<double>(), poff.as<int>(), pend.as<int>(), in_cnt(), e,
+                                   entry_pair.as<int>(), part, rows, first, eext, fo, vo, eo, v.as<double>(), x.as<double>(), type.as<int>(),
+                                   massinv.as<double>(), dtf, dt, integrate, N, block_np.as<int>(), pair_blocks(),
+                                   count ? pair_sum.as<unsigned long long>() : nullptr, zbl ? zacc.as<double>() : nullptr);
+            });
         });
     }
 
@@ -1465,14 +1490,7 @@ struct mdp_md {
                         ptj.as<int>(), nullptr, dedr.as<double>(), N, pair_slots, pair_base.as<int>() + pair_blocks(), st,
                         true, 10);
         });
-        timed(T_TALLY, [&] {
-            hipLaunchKernelGGL(k_tally, dim3(nb(static_cast<long>(N) * PSUB, 256)), dim3(256), 0, st, dedr.as<double>(), prij.as<double>(),
-                               poff.as<int>(), pend.as<int>(), in_cnt(), in_e.as<int>(), entry_pair.as<int>(),
-                               epart.as<double>(), 0, 0.0, sE.as<double>(), f.as<double>(), vir.as<double>(),
-                               eatom.as<double>(), v.as<double>(), x.as<double>(), type.as<int>(),
-                               massinv.as<double>(), dtf, dt, integrate, N, block_np.as<int>(), pair_blocks(),
-                               pair_sum.as<unsigned long long>(), zbl ? zacc.as<double>() : nullptr);
-        });
+        tally(epart.as<double>(), 0, 0.0, sE.as<double>(), f.as<double>(), vir.as<double>(), eatom.as<double>(), integrate, true);
     }
 
     // plain SNAP on the same state; RMS force difference; plain forces replace the surrogate's when the

@@ -1,0 +1,44 @@
+"""The MD engine beyond what 32 bits count: 22,478,848 atoms have 2.16e9 slots in their neighbour lists.
+
+A displaced crystal repeated 8 times along each axis: every copy of an atom has to have the energy, force and virial that
+the engine finds for the crystal alone, within 1e-10 of the largest (positions up to 743 A round at 1e-13 A).
+"""
+import numpy as np
+import pytest
+
+from conftest import relerr
+from mdp_amd import lattice
+from mdp_amd.md import SnapMD
+
+pytestmark = pytest.mark.gpu
+
+REP = 8
+
+
+def _compute(x, box, rcut):
+    md = SnapMD(x, box, np.ones(len(x), np.int32), 2, lattice.snap_coefficients(5, seed=2), [0.5], [1.0], [180.95],
+                rcutfac=rcut)
+    try:
+        print(f"{len(x)} atoms, cutoff {rcut}", flush=True)
+        md.compute()
+        return md.state(), md.stats()["pairs"]
+    except RuntimeError as e:
+        if "out of memory" in str(e):
+            pytest.skip("not enough free device memory")
+        raise
+    finally:
+        md.close()
+
+
+@pytest.mark.parametrize("cells,rcut", [(28, 3.6)])
+def test_repeated_crystal(cells, rcut):
+    x, box = lattice.crystal("bcc", cells, 3.316, 0.05, 1)
+    tile, pairs = _compute(x, box, rcut)
+    r = np.arange(REP)
+    shift = np.stack(np.meshgrid(r, r, r, indexing="ij"), -1).reshape(-1, 1, 3) * box
+    big, n = _compute((x + shift).reshape(-1, 3), REP * box, rcut)
+    assert n == pairs * REP ** 3
+    for k in ("eatom", "f", "vatom"):
+        got = big[k].reshape(REP ** 3, -1)
+        for c in range(REP ** 3):
+            assert relerr(got[c], tile[k].ravel()) < 1e-10, (k, c)
