@@ -26,7 +26,8 @@ __global__ __launch_bounds__(64) void k_dedr(SnapDev s, const double* __restrict
     const int tjp = tj[p];
     const double rc = (s.radelem[ti[p]] + s.radelem[tjp]) * s.rcutfac;
     PairGeom g;
-    pair_geometry<true>(rij[3 * p], rij[3 * p + 1], rij[3 * p + 2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
+    const double* __restrict__ r = rij + 3 * static_cast<size_t>(p);
+    pair_geometry<true>(r[0], r[1], r[2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
     const size_t n = static_cast<size_t>(N);
     const size_t yb = static_cast<size_t>(ya) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
     double d0 = 0.0, d1 = 0.0, d2 = 0.0;
@@ -79,7 +80,8 @@ __global__ __launch_bounds__(64 * NW, WPE) void k_dedr_split(SnapDev s, const do
     const int tjp = tj[p];
     const double rc = (s.radelem[ti[p]] + s.radelem[tjp]) * s.rcutfac;
     PairGeom g;
-    pair_geometry<true>(rij[3 * p], rij[3 * p + 1], rij[3 * p + 2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
+    const double* __restrict__ r = rij + 3 * static_cast<size_t>(p);
+    pair_geometry<true>(r[0], r[1], r[2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
     // move this lane's component into slot 0
     const double uk = comp == 0 ? g.u[0] : (comp == 1 ? g.u[1] : g.u[2]);
     g.dar[0] = comp == 0 ? g.dar[0] : (comp == 1 ? g.dar[1] : g.dar[2]);
@@ -147,7 +149,8 @@ __global__ __launch_bounds__(64 * NW) void k_dedr_gen(SnapDev s, const double* _
     const int tjp = tj[p];
     const double rc = (s.radelem[ti[p]] + s.radelem[tjp]) * s.rcutfac;
     PairGeom g;
-    pair_geometry<true>(rij[3 * p], rij[3 * p + 1], rij[3 * p + 2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
+    const double* __restrict__ r = rij + 3 * static_cast<size_t>(p);
+    pair_geometry<true>(r[0], r[1], r[2], rc, s.rmin0, s.rfac0, s.switchflag, s.wjelem[tjp], g);
     const size_t n = static_cast<size_t>(N);
     const size_t yb = static_cast<size_t>(ya) + (ybase ? static_cast<size_t>(ybase[p]) : 0);
     double f = 0.5 * Yr[yb], t0 = 0.0, t1 = 0.0, t2 = 0.0;
@@ -243,7 +246,8 @@ __global__ __launch_bounds__(64, 2) void k_dedr_atom(const double* __restrict__ 
         const int tjp = tj[p];
         const double rc = (radelem[ti[p]] + radelem[tjp]) * rcutfac;
         PairGeom g;
-        pair_geometry<true>(rij[3 * p], rij[3 * p + 1], rij[3 * p + 2], rc, rmin0, rfac0, switchflag, wjelem[tjp], g);
+        const double* __restrict__ r = rij + 3 * static_cast<size_t>(p);
+        pair_geometry<true>(r[0], r[1], r[2], rc, rmin0, rfac0, switchflag, wjelem[tjp], g);
         const double uk = comp == 0 ? g.u[0] : (comp == 1 ? g.u[1] : g.u[2]);
         g.dar[0] = comp == 0 ? g.dar[0] : (comp == 1 ? g.dar[1] : g.dar[2]);
         g.dai[0] = comp == 0 ? g.dai[0] : (comp == 1 ? g.dai[1] : g.dai[2]);
