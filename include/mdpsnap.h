@@ -409,8 +409,10 @@ int mdp_sumsq(const double *v, long n, double *partials, int nblocks, void *stre
  * every pointer a device pointer.  Semantics of the upstream C++ core (src/C++/Core/cpuSnap4.cpp):
  * Ui and AddWself2Ui, Ei and Fi accumulate into their outputs, Yi zeroes and writes; the element of
  * atom i is map[type[i]] in Ei and Yi; Fi writes forces AoS and the virial SoA vatom[k*anum + atom]
- * with -r(x)dE/2 added to both atoms of each pair.  Small index and table arrays are read back to the
- * host once per call; the large arrays are used in place.  Errors: mdp_snap_last_error(). */
+ * with -r(x)dE/2 added to both atoms of each pair.  Every call of parts 5 and 6 but Cell2AtomListNoAlloc waits first for the
+ * work that the caller has queued on the device, on whatever stream, and returns when its own is done.  The large arrays are
+ * used in place; of the small ones a call reads back to the host what it needs there: with chemflag 0 Ui and Fi read the ranges
+ * of their index arrays and AddWself2Ui nothing.  Errors: mdp_snap_last_error(). */
 /* replaces hipSnapComputeUi in SnapComputeUi (mdpcore.h:3093-3116) */
 void mdp_hipSnapComputeUi(double *Stotr, double *Stoti, double *rootpqarray, double *rij, double *wjelem,
                           double *radelem, double rmin0, double rfac0, double rcutfac, int *idxu_block, int *map,

@@ -1099,7 +1099,7 @@ void mdp_hipNeighPairList(int* pairnum, int* pairlist, double* x, double* rcutsq
     guarded([&] {
         if (inum <= 0) return;
         if (jnum <= 0 || dim != 3 || ntypes < 1) throw Error("NeighPairList: needs jnum > 0, dim = 3, ntypes >= 1");
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_pair_list_strided(pairnum, pairlist, x, rcutsq, ilist, neighlist, neighnum, atomtype, alist, inum, jnum,
                                  dim, ntypes, st);
         finish(st);
@@ -1112,7 +1112,7 @@ void mdp_hipNeighPairListCut(int* pairnum, int* pairlist, double* x, double rcut
     guarded([&] {
         if (inum <= 0) return;
         if (jnum <= 0 || dim != 3) throw Error("NeighPairList: needs jnum > 0 and dim = 3");
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_pair_list_strided_cut(pairnum, pairlist, x, rcutsq, ilist, neighlist, neighnum, inum, jnum, dim, st);
         finish(st);
     });
@@ -1123,7 +1123,7 @@ void mdp_hipCumsum(int* d_out, int* d_in, int* d_sums, int* d_incr, int length) 
     (void)d_sums; (void)d_incr;
     guarded([&] {
         if (length <= 0) return;
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         const int n = length - 1;
         int* d_tmp = dev<int>(0, scan_tmp_ints(std::max(n, 1)));
         exclusive_scan(d_in, d_out, n, d_tmp, st);   // out[0..n], out[n] = total
@@ -1246,7 +1246,7 @@ void mdp_hipNeighPairs(double* xij, double* x, int* aii, int* ai, int* aj, int* 
     guarded([&] {
         if (inum <= 0) return;
         if (jnum <= 0 || dim < 1) throw Error("NeighPairs: needs jnum > 0 and dim >= 1");
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_pair_arrays_strided(xij, x, aii, ai, aj, ti, tj, pairnum, pairlist, pairnumsum, ilist, atomtype, alist,
                                    inum, jnum, dim, st);
         finish(st);
@@ -1318,7 +1318,7 @@ void mdp_hipAddUarraytotPairs(double* ulisttot_r, double* ulisttot_i, double* ul
     (void)nelements;
     guarded([&] {
         if (inum <= 0 || idxu_max <= 0) return;
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_add_utot_pairs(ulisttot_r, ulisttot_i, ulist_r, ulist_i, pairnum, pairnumsum, map, tj, idxu_max, inum,
                               ijnum, chemflag, st);
         finish(st);
@@ -1466,7 +1466,7 @@ void mdp_hipSnapTallyBispectrumVirial(double* bv, double* bispectrum, double* db
 void mdp_hipSnapTallyEnergyFull(double* eatom, double* bispectrum, double* coeffelem, int* ilist, int* map, int* type,
                                 int inum, int ncoeff, int ncoeffall, int quadraticflag) {
     guarded([&] {
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_tally_energy_full(eatom, bispectrum, coeffelem, ilist, map, type, inum, ncoeff, ncoeffall,
                                  quadraticflag, 0, st);
         finish(st);
@@ -1477,7 +1477,7 @@ void mdp_hipSnapTallyEnergyFull(double* eatom, double* bispectrum, double* coeff
 void mdp_hipSnapTallyEnergyFull2(double* eatom, double* bispectrum, double* coeffelem, int* ilist, int* map,
                                  int* type, int inum, int ncoeff, int ncoeffall, int quadraticflag) {
     guarded([&] {
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_tally_energy_full(eatom, bispectrum, coeffelem, ilist, map, type, inum, ncoeff, ncoeffall,
                                  quadraticflag, 1, st);
         finish(st);
@@ -1488,7 +1488,7 @@ void mdp_hipSnapTallyEnergyFull2(double* eatom, double* bispectrum, double* coef
 void mdp_hipSnapTallyForceFull(double* fatom, double* fij, int* ai, int* aj, int* alist, int ijnum) {
     (void)alist;
     guarded([&] {
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_tally_force_full(fatom, fij, ai, aj, ijnum, st);
         finish(st);
     });
@@ -1497,7 +1497,7 @@ void mdp_hipSnapTallyForceFull(double* fatom, double* fij, int* ai, int* aj, int
 // SnapTallyVirialFull backend 3 (mdpcore.h:3712-3730; SoA vatom[c*inum + atom], half to each atom)
 void mdp_hipSnapTallyVirialFull(double* vatom, double* fij, double* rij, int* ai, int* aj, int inum, int ijnum) {
     guarded([&] {
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         launch_tally_virial_full(vatom, fij, rij, ai, aj, inum, ijnum, st);
         finish(st);
     });

@@ -95,7 +95,7 @@ void mdp_hipPairaGradient(double* u, double* u_xij, double* xij, double* qi, dou
         if (nmu < 3 || !mu) throw Error("mdp_hipPairaGradient: mu must hold [cut_inner, cut_outer, z]");
         if (ng < 0) throw Error("mdp_hipPairaGradient: negative pair count");
         if (ng == 0) return;
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         double m[3];
         MDP_HIP(hipMemcpyAsync(m, mu, sizeof(m), hipMemcpyDeviceToHost, st));
         MDP_HIP(hipStreamSynchronize(st));
@@ -110,7 +110,7 @@ void mdp_hipFullNeighPairDecomposition(double* e, double* f, double* eij, double
     guarded_call([&] {
         if (dim != 2 && dim != 3) throw Error("mdp_hipFullNeighPairDecomposition: dim must be 2 or 3");
         if (ijnum <= 0) return;
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         hipLaunchKernelGGL(k_full_pair_decomp, dim3(blocks(ijnum, 256)), dim3(256), 0, st, e, f, eij, fij, ai, ijnum,
                            dim);
         sync(st);
@@ -122,7 +122,7 @@ void mdp_hipVirialPairTally(double* v, double* fij, double* rij, double factor, 
     guarded_call([&] {
         if (dim != 2 && dim != 3) throw Error("mdp_hipVirialPairTally: dim must be 2 or 3");
         if (ijnum <= 0) return;
-        hipStream_t st = library_stream();
+        hipStream_t st = stream_after_callers();
         hipLaunchKernelGGL(k_virial_pair_tally, dim3(blocks(ijnum, 256)), dim3(256), 0, st, v, fij, rij, factor, ai,
                            dim, inum, ijnum);
         sync(st);

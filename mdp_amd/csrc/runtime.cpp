@@ -24,6 +24,11 @@ hipStream_t library_stream() {
     return s;
 }
 
+hipStream_t stream_after_callers() {
+    MDP_HIP(hipDeviceSynchronize());
+    return library_stream();
+}
+
 std::mutex& library_mutex() {
     static std::mutex m;
     return m;

@@ -68,6 +68,9 @@ struct DevTables {
 };
 
 hipStream_t library_stream();
+// The same for calls on a caller's device arrays, after what the caller's streams still do to them: the library stream waits
+// for no other, the default stream included.
+hipStream_t stream_after_callers();
 std::mutex& library_mutex();
 
 // Effective weight of each coupling triple in Y for element combination (e1,e2,e3) of an atom of

@@ -151,3 +151,44 @@ def test_negative_and_centre_indices_of_forces_are_refused(gpu, route, array, va
         f, v = d["f"].numpy(), d["v"].numpy()
     assert ("centre index out of range" if array == "aii" else "negative pair atom index") in message
     assert np.all(f == 0.75) and np.all(v == 0.75)
+
+
+@pytest.mark.parametrize("call", ["AddWself2Ui", "Cumsum", "SnapTallyForceFull", "VirialPairTally"])
+def test_waits_for_the_callers_default_stream(gpu, call):
+    """Outputs cleared, and for Cumsum inputs, by memsets that still wait on the default stream behind 48 GB of others when the
+    call is made: it sees what they leave.  (Were it to run before them, sums would be lost or start from the old values.)"""
+    import mdp_amd
+    from mdp_amd.devarray import DevArray
+    c = gpu.cdll
+    c.hipMemsetAsync.argtypes, c.hipMemsetAsync.restype = [ctypes.c_void_p, I, ctypes.c_size_t, ctypes.c_void_p], I
+    clear = lambda d: c.hipMemsetAsync(d.ptr, 0, d.nbytes, None)  # noqa: E731
+    n, J = 1000, 4
+    s = _sna(gpu, J)
+    ones = lambda m, t=np.float64: DevArray.from_numpy(np.ones(m, t))  # noqa: E731
+    big = DevArray(1 << 30)
+    i, force = np.arange(n, dtype=np.int32), np.arange(3.0 * n)
+    ai, aj, fij, ty, mp = (DevArray.from_numpy(a) for a in (i, (i + 1) % n, force, np.ones(n, np.int32), s.map))
+    U, V, f, v, count, total = (ones(m, t) for m, t in ((n * s.idxu_max, float), (n * s.idxu_max, float), (3 * n, float),
+                                                        (6 * n, float), (n, np.int32), (n + 1, np.int32)))
+    work = {"AddWself2Ui": ("ppd" "pppp" "iiiiii", (U.ptr, V.ptr, 3.0, None, ty.ptr, mp.ptr, ai.ptr, 0, 0, s.idxu_max, 1, J, n)),
+            "Cumsum": ("ppppi", (total.ptr, count.ptr, None, None, n + 1)),
+            "SnapTallyForceFull": ("pppppi", (f.ptr, fij.ptr, ai.ptr, aj.ptr, None, n)),
+            "VirialPairTally": ("pppdpiii", (v.ptr, fij.ptr, fij.ptr, 2.0, ai.ptr, 3, n, n))}
+    shape, args = work[call]
+    fn = _fn(gpu, call, shape)
+    print(call, flush=True)
+    for _ in range(6):
+        assert c.hipMemsetAsync(big.ptr, 1, big.nbytes, None) == 0
+    for d in (U, V, f, v, count):
+        assert clear(d) == 0
+    fn(*args)
+    mdp_amd.check(call)
+    if call == "AddWself2Ui":
+        assert U.numpy().sum() == 3.0 * n * sum(j + 1 for j in range(J + 1)) and not V.numpy().any()
+    elif call == "Cumsum":
+        assert not total.numpy().any()
+    elif call == "SnapTallyForceFull":
+        assert np.array_equal(f.numpy(), force - np.roll(force, 3))
+    else:
+        x, y, z = force.reshape(n, 3).T
+        assert np.array_equal(v.numpy().reshape(6, n), 2.0 * np.array([x * x, y * y, z * z, x * y, x * z, y * z]))
