@@ -184,8 +184,10 @@ __global__ void k_nh_chain(const double* __restrict__ part, int nparts, double* 
 // The thermostat between two steps in one workgroup, for systems of at most NVT_ONE atoms: the closing half-step of
 // one step (CLOSE: sum of m v^2, chain, v *= factor), the opening half-step of the next (OPEN: the same, then
 // v += dtf/m f and x += dt v), or both.  The chain runs on thread 0 from an LDS copy of its state.  Each of these
-// was three launches; at 128 atoms six launches a step took 18 us, a quarter of the step.
-constexpr int NVT_ONE = 8192;
+// was three launches.  us a step of a twojmax 2 run under the thermostat, one workgroup / six launches: 128 atoms
+// 29.8 / 39.8, 1,024 32.8 / 40.6, 2,000 36.4 / 41.8, 3,456 41.8 / 45.1, 4,394 47.5 / 47.6, 5,488 51.3 / 48.3, 8,192
+// 61.9 / 52.6: at some 4,400 atoms one workgroup's passes over all of them cost what the launches do.
+constexpr int NVT_ONE = 4096;
 
 template <bool CLOSE, bool OPEN>
 __global__ __launch_bounds__(1024) void k_nvt_one(double* __restrict__ x, double* __restrict__ v,
