@@ -53,8 +53,7 @@ struct mdp_fit {
     FitTerms terms;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    DevBuf l_cnt, l_off, l_cur, l_idx, l_bi, l_bd, l_bv, l_as, l_chunks, l_ekl, l_part, l_out, l_T, l_W;
-    int l_ekl_k = 0;         // column count the (k, l) table was built for
+    DevBuf l_cnt, l_off, l_cur, l_idx, l_bi, l_bd, l_bv, l_as, l_chunks, l_part, l_out, l_T, l_W;
     int dbdr_groups = 1024;
     bool tuned = false;
     std::string tuning_json = "{}";
