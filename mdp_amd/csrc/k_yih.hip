@@ -33,9 +33,6 @@ void launch_yi_class_8(const SnapDev&, const double*, const double*, const doubl
 void launch_yi_class_small(const SnapDev&, const double*, const double*, const double*, double*, double*, double*, int,
                            hipStream_t);
 
-constexpr int YI_ROWS = 208;    // variant id of k_yi_rows
-constexpr int YI_CLASS = 308;   // variant id of k_yi_class
-
 void yi_row_order(int J, int* out) {
     auto cgn = [](int m, int j1, int j2, int j) {
         const int lo = std::max(0, (2 * m - j - j2 + j1) / 2);

@@ -6,13 +6,13 @@ namespace mdp {
 void launch_yi_full_8(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
                       const int* order, int N, bool rows, hipStream_t st);
 
-// A workgroup per output row where a workgroup per 64 atoms would leave most CUs idle (yi_default_variant's lines), then
-// the classes.  15,972 atoms at twojmax 8: 167 us, against 203 with the rows of 64 atoms in one workgroup and 699 for the row
+// A workgroup per output row where yi_default_variant says so (a workgroup per 64 atoms would leave most CUs idle), else the
+// classes.  15,972 atoms at twojmax 8: 167 us, against 203 with the rows of 64 atoms in one workgroup and 699 for the row
 // per wave from global memory that any U and any coupling table still take.
 void launch_yi_full(const SnapDev& s, const double* Ur, const double* Ui, const double* beta_t, double* Yr, double* Yi,
                     const int* order, int N, hipStream_t st) {
     if (N <= 0) return;
-    const bool rows = N <= 64 * (s.J == 8 ? 60 : (s.J == 6 ? 112 : 50));
+    const bool rows = yi_default_variant(s.J, N) == YI_ROWS;
     switch (s.J) {
 #define YF_CASE(JV, WV)                                                                                              \
     case JV:                                                                                                         \

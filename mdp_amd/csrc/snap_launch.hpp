@@ -80,6 +80,8 @@ void launch_yi_half(const SnapDev& s, const double* Uhr, const double* Uhi, cons
                     double* Yhi, double* epart, const int* row_order, int natoms, hipStream_t st, int waves = 8);
 // waves-per-workgroup variants available for twojmax J (ids = waves); returns their number
 int yi_half_variants(int J, int* ids);
+constexpr int YI_ROWS = 208;    // the variant with a workgroup per output row (k_yi_rows)
+constexpr int YI_CLASS = 308;   // with a wave per class of output rows (k_yi_class)
 int yi_default_variant(int J, int N);   // by the number of atoms
 // row ids of the half domain sorted by decreasing compute_yi work
 void yi_row_order(int J, int* out);
