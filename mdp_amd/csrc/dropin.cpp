@@ -778,8 +778,9 @@ void cpuSnapTallyBispectrumVirial(double* bv, double* bispectrum, double* dbdr, 
 
 // ---- backend-3 entry points of the C++ core dispatch (src/C++/Common/mdpcore.h) -----------------
 // Device arrays in and out, same argument lists as the dispatch's backend branches (without backend).
-// The large arrays are used in place; the small index and table arrays are read back once to drive the
-// same host-side set-up as the cpuSnap.h entry points above.
+// The large arrays are used in place.  Where the set-up on the host needs them, the small index and table arrays are read
+// back for the same bodies as the cpuSnap.h entry points above; with one element Ui, AddWself2Ui and Fi, and always Ei, use
+// them where they are.
 
 namespace {
 // device -> host copy of a small argument array (after the caller's device work has finished)

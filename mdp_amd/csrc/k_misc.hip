@@ -1,7 +1,7 @@
 // Device kernels of the descriptor path (cpuComputeSij/Uij, Zero/AddUarraytot, Bi2, Dbidrj), the
-// tallies, the pair-list builders, AddWself2Ui and a device-wide exclusive scan.  These follow the
-// upstream functions one output element (or one pair) per thread with runtime loops; the
-// performance-critical force path lives in k_ui/k_yi/k_dedr and the MD engine.
+// tallies, the pair-list builders, AddWself2Ui, checks of index arrays and a device-wide exclusive scan.  Most follow
+// the upstream functions one output element (or one pair) per thread with runtime loops; where another split is taken
+// the kernel says so.  The force path lives in k_ui/k_yi/k_dedr and the MD engine.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -180,8 +180,8 @@ void launch_csr_of_sorted(const int* a, int n, int* off, int m, hipStream_t st) 
 // of one derivative in registers, every finished row (j, mb) written as it comes, with its mirror image where upstream
 // writes one.  Component 0 also writes U.  What upstream leaves unwritten (the derivative rows 2 mb > j of even
 // layers, and those behind (j + 1)/2 of odd ones) is left alone; the derivative row mb = (j + 1)/2 of an odd layer holds
-// the bare dU, as upstream leaves it.  `packed`: the derivative rows that are written lie one after another (du_block).  (One lane per pair with all rows, its recursion through global memory: 737 us
-// for 1,080 pairs at twojmax 8; 13 so.)
+// the bare dU, as upstream leaves it.  `packed`: the derivative rows that are written lie one after another (du_block).
+// (One lane per pair with all rows, its recursion through global memory: 737 us for 1,080 pairs at twojmax 8; 13 so.)
 template <int J>
 __global__ __launch_bounds__(64) void k_uij(SnapDev s, double* __restrict__ Sr, double* __restrict__ Si,
                                             double* __restrict__ dr0, double* __restrict__ dr1, double* __restrict__ dr2,

@@ -12,9 +12,9 @@
 // Options (template flags of k_yi_half): SA orders a row's couplings (j1, mb1, j2) so that each U row of
 // the larger layer is read from LDS once per output row; CX stores (re, im) of an element next to each
 // other in LDS, one 16-byte read per element; SYM takes each unordered pair of U rows of a (j1, j1)
-// coupling once (its sum is symmetric under the swap of the two factors).  All three together (the MD
-// default at every twojmax) read 13,446 LDS elements and execute 84% of the upstream flops per atom at
-// twojmax 8.
+// coupling once (its sum is symmetric under the swap of the two factors).  All three together read 13,446
+// LDS elements and execute 84% of the upstream flops per atom at twojmax 8; k_yi_rows has them all, and so has the
+// variant that the MD engine takes at twojmax 6 between k_yi_rows and the classes of k_yic.hpp.
 #pragma once
 #include <hip/hip_runtime.h>
 

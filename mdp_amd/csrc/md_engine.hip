@@ -7,14 +7,14 @@
 //      neighbour list at rcut+skin (a workgroup per cell stages the 27 surrounding cells in LDS)
 //      and its transpose (incoming entries per atom, sorted)
 //   3. pair list: neighbour entries with d^2 < rc(ti,tj)^2 and d^2 > 1e-20 (cpuSnap.cpp:258-286),
-//      compacted by centre atom within blocks of 64 atoms in one pass (and the reference pair potential of the same
-//      entries)
+//      compacted by centre atom within blocks of 16 atoms (up to 16,384) or 64 in one pass (and the reference pair
+//      potential of the same entries)
 //   4. SNAP: Utot (k_ui), Y + energy partials (k_yi), dE/dr per pair (k_dedr)
 //   5. tally per atom without atomics: f_i = sum over own pairs - sum over incoming pairs,
 //      W_i = -sum_j r_ij (x) dE/dr_ij, E_i from the energy partials; then v += dt/2 f/m, and inside a run the
 //      first half-step and drift of the next step with it.
 // Neighbour entries are (owner j, image shift) pairs stored atom-major (slot k of atom i at i*NBMAX + k): the
-// 16 lanes that share an atom in the per-step kernels read one contiguous run.  Positions stay unwrapped
+// lanes that share an atom in the per-step kernels read one contiguous run.  Positions stay unwrapped
 // between rebuilds and the displacement of a neighbour is always (x_j + shift*L) - x_i, evaluated without
 // contraction.
 #include <hip/hip_runtime.h>
@@ -40,7 +40,7 @@ using namespace mdp;
 namespace {
 
 constexpr int NBMAX = 96;      // neighbour slots per atom at rcut+skin
-constexpr int CELLCAP = 48;    // atoms per cell accepted (bounds the per-cell insertion sort)
+constexpr int CELLCAP = 48;    // atoms per cell accepted (a wave ranks a cell's atoms)
 constexpr int SHK = 8;         // image shifts are coded in [-SHK, SHK] per axis
 constexpr double FTM2V = 1.0 / 1.0364269e-4;   // metal units, eV/A/amu -> A/ps^2
 constexpr double MVV2E = 1.0364269e-4;
@@ -662,7 +662,7 @@ static_assert(NBMAX / PSUB <= 32, "one bit per pass");
 // full-list conventions (cpuFullNeighPairList's d^2 <= rc^2 test, src/C++/Core/cpuNeighCount.cpp:60-81;
 // cpuFullNeighPairDecomposition and cpuVirialPairTally with factor -1/2, cpuPotentials.cpp:1587-1649 and
 // the sign flip of :1837): e_i = sum_j u(r_ij)/2, F_i = sum_j du/dxij, W_i = -1/2 sum_j xij (x) du/dxij,
-// xij = x_j - x_i.  Each atom owns its sums (16 lanes combine by a butterfly), so there are no atomics.
+// xij = x_j - x_i.  Each atom owns its sums (its 16 or 32 lanes combine by a butterfly), so there are no atomics.
 // zacc[10 i + c]: force x, y, z, virial xx, yy, zz, xy, xz, yz, energy.
 __device__ __forceinline__ void zbl_add(const ZblParams& zp, double d2, double dx, double dy, double dz, double (&a)[10]) {
     if (d2 > zp.rout2) return;
@@ -985,11 +985,11 @@ struct mdp_md {
     DevTables tab;
     std::vector<double> massinv_h, rc2_h;
     // device state
-    // cleared: what a rebuild starts from zero (ClearedPart), cleared by one fill
+    // cleared: what a rebuild starts from zero (its layout is below), cleared by one fill
     DevBuf x, v, f, type, massinv, xref, cell_of, cleared, cell_start, cell_atoms, scan_tmp, nb_cnt, nbr, in_e, poff,
         pi, pti, ptj, prij, entry_pair, Ur, Ui, Yr, Yi, epart, dedr, eatom, vir, beta_t, rc2, row_order, yt, pair_sum,
         pgeo, zacc;
-    // pair list (k_pair_list): room, place and pair count of each block of 64 atoms, end of each atom's pairs
+    // pair list (k_pair_list): room, place and pair count of each block of pair_atoms() atoms, end of each atom's pairs
     DevBuf pair_room, pair_base, block_np, pend;
     int pair_slots = 0;   // total room
     // Layout of `cleared`: the rebuild's report to the host (max displacement^2 bits, neighbour entries, flags),
@@ -1523,8 +1523,8 @@ struct mdp_md {
                            massinv.as<double>(), dtf, N);
     }
 
-    // Time every compiled variant of the two heaviest kernels on the live data (both are pure
-    // functions of their inputs, so re-running them is harmless) and keep the fastest.
+    // Time the candidate variants of the heaviest kernels and of the neighbour build on the live data (all are pure functions
+    // of their inputs, so re-running them is harmless) and keep the fastest.
     template <class F>
     double time_launch(F&& f, int reps) {
         hipEvent_t a = ev(), b = ev();
