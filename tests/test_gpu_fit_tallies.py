@@ -48,7 +48,8 @@ def _reference(fit, configs, types):
     return out
 
 
-@pytest.mark.parametrize("sizes,J,types", [([2, 511, 512, 513], 4, 1), ([2047, 1, 65], 2, 1), ([2048, 2049, 30], 4, 1),
+@pytest.mark.parametrize("sizes,J,types", [([2, 511, 512, 513], 4, 1), ([2047, 1, 65], 2, 1), ([2100, 30], 4, 1),
+                                           ([2048, 2049, 30], 4, 1),
                                            ([3072, 513, 2100], 2, 1), ([3073, 40], 2, 1),
                                            ([64, 40], 8, 1), ([63, 100], 6, 1), ([128, 60], 6, 2), ([70, 33], 4, 3),
                                            ([60, 95], 4, 5)])
